@@ -1,8 +1,10 @@
 // GEMM dispatch: alignment checks, tile choice, and the element-wise kernel
-// used for operands the MFMA fast path cannot take (leading dimensions not a
-// multiple of 8, misaligned pointers).  Ragged N and K (not multiples of 8)
-// run on the MFMA path: ragged columns are stored element by element, and K
-// not a multiple of 8 runs the instantiations that mask the last K-step.
+// used for what no MFMA instantiation takes (fewer than 8 columns in an
+// operand row, activations on an NN operand).  Ragged N and K (not multiples
+// of 8) run on the MFMA path: ragged columns are stored element by element,
+// K not a multiple of 8 runs the instantiations that mask the last K-step,
+// and rows off the 16-byte grid (leading dimensions not a multiple of 8,
+// misaligned pointers) those that load their tiles through registers.
 #include "gemm_impl.h"
 
 namespace hxmi {
@@ -11,6 +13,8 @@ hipError_t launch_fast_f16(int tile, bool nn, int epi, bool out_f32, bool rms, c
 hipError_t launch_fast_bf16(int tile, bool nn, int epi, bool out_f32, bool rms, const KArgs& k, hipStream_t s);
 hipError_t launch_fast_w8(int tile, int epi, bool out_f32, const KArgs& k, hipStream_t s);
 hipError_t launch_fast_ragged(int tile, bool bf16, bool nn, int epi, bool out_f32, const KArgs& k, hipStream_t s);
+hipError_t launch_fast_unaligned(int tile, bool bf16, bool nn, int epi, bool out_f32, bool rms, const KArgs& k,
+                                 hipStream_t s);
 
 namespace {
 
@@ -97,20 +101,45 @@ bool aligned(const void* p, uintptr_t n) { return ((uintptr_t)p % n) == 0; }
 }  // namespace
 }  // namespace gemm
 
-bool gemm_fast_path_ok(const GemmProblem& p) {
+namespace gemm {
+namespace {
+
+// Whether the operands suit the direct-to-LDS loads: 16-byte aligned rows
+// within 32-bit buffer offsets.  C may lie anywhere (its 16-byte stores take
+// any element address at the same cost).
+bool operands_aligned(const GemmProblem& p) {
   const bool i8 = p.dtype == DT_W8A16;
   if (i8 && (p.K % 16 || p.N % 8)) return false;
   if (p.epilogue == EPI_SILU_MUL && p.N % 32) return false;
   if (p.K % 8 && p.rms) return false;  // the RMS prologue sums whole fragments
-  if (p.lda % 8 || p.ldb % (i8 ? 16 : 8) || p.ldc % 8) return false;
-  if (p.batch > 1 && (p.sA % 8 || p.sB % (i8 ? 16 : 8) || p.sC % 8)) return false;
-  if (!gemm::aligned(p.A, 16) || !gemm::aligned(p.B, 16) || !gemm::aligned(p.C, 16)) return false;
-  if (p.bias && !gemm::aligned(p.bias, 8)) return false;
+  if (p.lda % 8 || p.ldb % (i8 ? 16 : 8)) return false;
+  if (p.batch > 1 && (p.sA % 8 || p.sB % (i8 ? 16 : 8))) return false;
+  if (!aligned(p.A, 16) || !aligned(p.B, 16)) return false;
+  if (p.bias && !aligned(p.bias, 8)) return false;
   // 32-bit buffer offsets inside one tile row-panel
   if ((int64_t)256 * p.lda * 2 >= (1ll << 31) || (int64_t)256 * p.ldb * 2 >= (1ll << 31)) return false;
   if (p.M >= (1ll << 31) || p.N >= (1ll << 31) || p.K >= (1ll << 31)) return false;
   if (p.b_nt == 0 && i8) return false;
   return true;
+}
+
+// Whether some MFMA instantiation computes p with operands and C at any
+// element address: rows of at least 8 elements (the unaligned tiles load a
+// row's last chunk as its last 8 elements) and the epilogues it is built for.
+bool any_alignment_ok(const GemmProblem& p) {
+  if (p.dtype == DT_W8A16 || p.K < 8 || (!p.b_nt && p.N < 8)) return false;
+  if (p.epilogue == EPI_SILU_MUL && p.N % 32) return false;
+  if (!p.b_nt && p.epilogue != EPI_NONE && p.epilogue != EPI_BIAS) return false;
+  if (p.out_f32 && (p.epilogue != EPI_NONE || p.rms || p.dtype != DT_F16)) return false;
+  if (p.rms && (!p.b_nt || p.epilogue == EPI_GELU_TANH || p.epilogue == EPI_BIAS_GELU_TANH)) return false;
+  return p.M < (1ll << 31) && p.N < (1ll << 31) && p.K < (1ll << 31);
+}
+
+}  // namespace
+}  // namespace gemm
+
+bool gemm_fast_path_ok(const GemmProblem& p) {
+  return gemm::operands_aligned(p) && p.ldc % 8 == 0 && (p.batch <= 1 || p.sC % 8 == 0) && gemm::aligned(p.C, 16);
 }
 
 // Pick the tile that minimises an estimate of makespan: rounds of tiles over
@@ -188,11 +217,14 @@ int gemm_pick_tile(const GemmProblem& p) {
 namespace gemm {
 namespace {
 
+// The ragged-K and unaligned instantiations: 128x128 once its tiles cover the CUs.
+int tile_of_two(const GemmProblem& p) {
+  const int64_t t128 = ((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch;
+  return t128 >= 256 ? TILE_128x128 : TILE_64x64;
+}
+
 int tile_for(const GemmProblem& p) {
-  if (p.K % 8) {  // the ragged-K instantiations: 128x128 once its tiles cover the CUs
-    const int64_t t128 = ((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch;
-    return t128 >= 256 ? TILE_128x128 : TILE_64x64;
-  }
+  if (p.K % 8) return tile_of_two(p);
   int tile = p.tile >= 0 ? p.tile : knob_or(KNOB_GEMM_TILE, -1);
   // (an override of 128x192 for a layout it does not take: the picker's tile)
   if (tile < 0 || tile >= TILE_COUNT || (tile == TILE_128x192_W8 && (!p.b_nt || p.dtype == DT_W8A16)))
@@ -320,6 +352,17 @@ hipError_t launch_gemm(const GemmProblem& p, hipStream_t stream) {
   const bool i8 = p.dtype == DT_W8A16;
   if (!gemm_fast_path_ok(p)) {
     if (i8) return hipErrorNotSupported;
+    if (gemm::any_alignment_ok(p)) {
+      if (gemm::operands_aligned(p)) {  // only C is off the 16-byte grid
+        const int tile = gemm::tile_for(p);
+        return gemm::launch_fast(p, tile, gemm::make_kargs(p, tile), stream);
+      }
+      const int tile = gemm::tile_of_two(p);
+      const gemm::KArgs k = gemm::make_kargs(p, tile);
+      if ((int64_t)k.tiles_m * k.tiles_n * k.batch >= (1ll << 31)) return hipErrorInvalidValue;
+      return gemm::launch_fast_unaligned(tile, p.dtype == DT_BF16, !p.b_nt, p.epilogue, p.out_f32, p.rms != 0, k,
+                                         stream);
+    }
     gemm::GArgs g;
     g.A = (const char*)p.A;
     g.B = (const char*)p.B;

@@ -139,13 +139,38 @@ __device__ __forceinline__ void store4(char* p, float v0, float v1, float v2, fl
   *(short4v*)p = __builtin_bit_cast(short4v, t);
 }
 
+// 16- and 8-byte accesses to global memory at any element address: gfx950
+// runs with unaligned access enabled, so these compile to the same single
+// global instructions as the aligned types.
+typedef int int4u __attribute__((ext_vector_type(4), aligned(2)));
+typedef short short4u __attribute__((ext_vector_type(4), aligned(2)));
+typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// The 8 packed 16-bit values from element s on, zeros behind (s >= 0).
+__device__ __forceinline__ int4v drop_first(int4v v, int s) {
+  typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
+  const u64x2 q = __builtin_bit_cast(u64x2, v);
+  const int sh = (s & 3) * 16;
+  uint64_t lo = q[0], hi = q[1];
+  if (s >= 4) {
+    lo = hi;
+    hi = 0;
+  }
+  if (s >= 8) lo = 0;
+  if (sh) {
+    lo = (lo >> sh) | (hi << (64 - sh));
+    hi >>= sh;
+  }
+  return __builtin_bit_cast(int4v, u64x2{lo, hi});
+}
+
 template <typename T>
 __device__ __forceinline__ void load_bias4(const char* bias, int n, int N, float* out) {
   if (n + 4 > N) {  // ragged last columns
 #pragma unroll
     for (int i = 0; i < 4; ++i) out[i] = n + i < N ? (float)((const T*)bias)[n + i] : 0.f;
   } else if (n < N) {
-    short4v raw = *(const short4v*)(bias + (int64_t)n * 2);
+    short4v raw = *(const short4u*)(bias + (int64_t)n * 2);
     T t[4];
     __builtin_memcpy(t, &raw, 8);
 #pragma unroll
@@ -253,8 +278,18 @@ __device__ __forceinline__ void pp_barrier() {
 // barriers: while one group issues its MFMAs from registers, the other
 // loads its next step's fragments from LDS and issues the global->LDS loads,
 // so every SIMD's MFMA pipe alternates between its two waves.
+//
+// UNAL = true: operand rows at any element address and any leading dimension
+// (a contiguous matrix with an odd number of columns).  A direct-to-LDS load
+// needs 4-byte aligned sources, so these tiles are loaded with unaligned
+// 16-byte loads into registers, one K-step ahead, and written to one of two
+// LDS stages in the same layout.  Nothing outside a matrix is read: rows
+// past the end repeat the last one (their results are not stored), and the
+// chunk that would cross the end of a row is loaded from the row's last 8
+// elements and shifted, which leaves zeros past K.
 template <int BM, int BN, int WM, int WN, int BK, int STAGES, bool NN, typename T, int EPI, bool OUTF32,
-          bool BI8 = false, bool PP = false, bool RMS = false, bool RAGGED = false, int SB = 0, int FD = 1>
+          bool BI8 = false, bool PP = false, bool RMS = false, bool RAGGED = false, int SB = 0, int FD = 1,
+          bool UNAL = false>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a) {
   constexpr int NWM = BM / WM, NWN = BN / WN, NW = NWM * NWN, NT = NW * 64;
   constexpr int TM = WM / 32, TN = WN / 32;
@@ -289,6 +324,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
   static_assert(!PP || (NW == 8 && NWM == 2 && STAGES >= 3 && !BI8), "ping-pong: 2 x 4 waves, >= 3 stages");
   static_assert(!RMS || (!NN && !BI8 && !PP && !OUTF32), "RMSNorm prologue: NT, standard schedule");
   static_assert(!RAGGED || (!BI8 && !PP && !RMS), "ragged K: plain fp16 / bf16 operands, standard schedule");
+  static_assert(!UNAL || (!BI8 && !PP && !RAGGED && STAGES == 2 && SBS == 2), "unaligned rows: two LDS stages");
   __shared__ __attribute__((aligned(1024))) char smem[SMEM];
   auto sa = [&](int i) { return smem + i * A_BYTES; };              // A stage i
   auto sb = [&](int i) { return smem + A_REGION + i * B_BYTES; };   // B stage i
@@ -312,7 +348,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
   // they are issued before every operand load.  Other N read them from
   // global memory in the epilogue.
   static_assert(BN * 2 <= 1024, "column vector chunk");
-  const bool cv_lds = NCV > 0 && (a.N % 8) == 0;
+  const bool cv_lds = NCV > 0 && !UNAL && (a.N % 8) == 0;
   char* const cv_bias = smem + SMEM_OPS;
   char* const cv_scale = smem + SMEM_OPS + (HAS_BIAS ? 1024 : 0);
   if (cv_lds && w == 0) {
@@ -547,6 +583,82 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
       stw = (stw + 1 == STAGES) ? 0 : stw + 1;
     }
     if (grp == 0) pp_barrier();
+  } else if constexpr (UNAL) {
+    // Step kt + 1 is written to the other stage after step kt's MFMAs, and
+    // its registers then take step kt + 2, so a load has one K-step of MFMAs
+    // to return.  The barrier at the end of a step publishes the stage just
+    // written; the stage it overwrote was last read in the step before.
+    const int kl = K - 8;  // last full chunk of a k-contiguous row (the host checks K >= 8, and N >= 8 for NN)
+    const char* pA[IA];
+    const char* pB[IB];
+#pragma unroll
+    for (int i = 0; i < IA; ++i)
+      pA[i] = a.A + (b * a.sA + (int64_t)min(m0 + (i * NW + w) * RPIK + lane / CH, a.M - 1) * a.lda) * 2;
+    const int cN = NN ? ((lane % CPR) ^ nn_swz<BN>(w * RPI + lane / CPR)) * 8 : 0;  // this lane's column in an NN tile
+    const int nB = NN ? min(n0 + cN, a.N - 8) : 0;
+    const int dropN = NN ? n0 + cN - nB : 0;
+#pragma unroll
+    for (int i = 0; i < IB; ++i)
+      pB[i] = NN ? a.B + (b * a.sB + nB) * 2
+                 : a.B + (b * a.sB + (int64_t)min(n0 + (i * NW + w) * RPIK + lane / CH, a.N - 1) * a.ldb) * 2;
+    int4v va[IA], vb[IB];
+    auto fetch = [&](int kt) {
+      const int k = min(kt * BK + cA * 8, kl);
+#pragma unroll
+      for (int i = 0; i < IA; ++i) va[i] = *(const int4u*)(pA[i] + (int64_t)k * 2);
+#pragma unroll
+      for (int i = 0; i < IB; ++i)
+        vb[i] = NN ? *(const int4u*)(pB[i] + (int64_t)min(kt * BK + (i * NW + w) * RPI + lane / CPR, K - 1) * a.ldb * 2)
+                   : *(const int4u*)(pB[i] + (int64_t)k * 2);
+    };
+    auto commit = [&](int kt, int stage) {
+      if (kt == nk - 1) {  // past K: zeros in both operands
+        const int drop = max(kt * BK + cA * 8 - kl, 0);
+#pragma unroll
+        for (int i = 0; i < IA; ++i) va[i] = drop_first(va[i], drop);
+#pragma unroll
+        for (int i = 0; i < IB; ++i) {
+          if constexpr (NN) {
+            if (kt * BK + (i * NW + w) * RPI + lane / CPR >= K) vb[i] = int4v{};
+          } else {
+            vb[i] = drop_first(vb[i], drop);
+          }
+        }
+      }
+      if (NN && n0 + BN > a.N) {
+#pragma unroll
+        for (int i = 0; i < IB; ++i) vb[i] = drop_first(vb[i], dropN);
+      }
+#pragma unroll
+      for (int i = 0; i < IA; ++i) *(int4v*)(sa(stage) + (i * NW + w) * 1024 + lane * 16) = va[i];
+#pragma unroll
+      for (int i = 0; i < IB; ++i) *(int4v*)(sb(stage) + (i * NW + w) * 1024 + lane * 16) = vb[i];
+    };
+    fetch(0);
+    commit(0, 0);
+    if (nk > 1) fetch(1);
+    __syncthreads();
+    for (int kt = 0; kt < nk; ++kt) {
+      const char* sA_ = sa(kt & 1);
+      const char* sB_ = sb(kt & 1);
+      static_for<SUBS>([&](auto S) {
+        short8v fa[TM], fb[TN];
+        read_frags(fa, fb, sA_, sB_, decltype(S)::value, kt);
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+#pragma unroll
+          for (int j = 0; j < TM; ++j) acc[i][j] = Mfma<T>::run(fb[i], fa[j], acc[i][j]);
+        if constexpr (RMS) {
+#pragma unroll
+          for (int j = 0; j < TM; ++j) ss[j] = sumsq8<T>(fa[j], ss[j]);
+        }
+      });
+      if (kt + 1 < nk) {
+        commit(kt + 1, (kt + 1) & 1);
+        if (kt + 2 < nk) fetch(kt + 2);
+      }
+      __syncthreads();
+    }
   } else {
   // Issue order, step by step: step t issues A(t + STAGES), then
   // B(t + SBS); the prologue runs the virtual steps t = -SBS .. -1 (A only
@@ -767,7 +879,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
             for (int q = 0; q < 4; ++q) v[q] = gelu_tanh(v[q]);
           }
           if (m < a.M && n + 4 <= a.N) {
-            *(float4v*)(Cb + ((int64_t)m * a.ldc + n) * 4) = float4v{v[0], v[1], v[2], v[3]};
+            *(float4u*)(Cb + ((int64_t)m * a.ldc + n) * 4) = float4v{v[0], v[1], v[2], v[3]};
           } else if (m < a.M && n < a.N) {  // ragged last columns
 #pragma unroll
             for (int q = 0; q < 4; ++q)
@@ -836,7 +948,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
       const int m = m0 + row, n = n0o + cc * 8;
       if (m < a.M && n + 8 <= Nout) {
         int4v v = *(const int4v*)(smem + row * SROW + cc * 16);
-        *(int4v*)(Cb + ((int64_t)m * a.ldc + n) * 2) = v;
+        *(int4u*)(Cb + ((int64_t)m * a.ldc + n) * 2) = v;
       } else if (m < a.M && n < Nout) {  // ragged last columns
         const short* src = (const short*)(smem + row * SROW + cc * 16);
         short* dst = (short*)(Cb + ((int64_t)m * a.ldc + n) * 2);
@@ -897,7 +1009,8 @@ constexpr TileShape kTiles[TILE_COUNT] = {
     {64, 64, 32, 32, 64, 4, false, 0, 3},      // TILE_64x64_S4
 };
 
-template <int TILE, bool NN, typename T, int EPI, bool OUTF32, bool BI8, bool RMS = false, bool RAGGED = false>
+template <int TILE, bool NN, typename T, int EPI, bool OUTF32, bool BI8, bool RMS = false, bool RAGGED = false,
+          bool UNAL = false>
 hipError_t launch_one(const KArgs& k, hipStream_t stream) {
   constexpr TileShape s = kTiles[TILE];
   constexpr int threads = (s.BM / s.WM) * (s.BN / s.WN) * 64;
@@ -907,8 +1020,9 @@ hipError_t launch_one(const KArgs& k, hipStream_t stream) {
   // weights stream from HBM, so B is prefetched several K-steps ahead
   constexpr int W8_A = s.BM * 128, W8_B = s.BN * 64;
   constexpr int W8_SB = W8_A / W8_B + 3 > 6 ? 6 : W8_A / W8_B + 3;
-  hipLaunchKernelGGL((gemm_mfma<s.BM, s.BN, s.WM, s.WN, (BI8 ? 64 : s.BK), (BI8 ? 2 : s.STAGES), NN, T, EPI, OUTF32, BI8,
-                                (s.PP && !BI8 && !RMS), RMS, RAGGED, (BI8 ? W8_SB : s.SB), (BI8 || s.PP ? 1 : s.FD)>),
+  hipLaunchKernelGGL((gemm_mfma<s.BM, s.BN, s.WM, s.WN, (BI8 ? 64 : s.BK), (BI8 || UNAL ? 2 : s.STAGES), NN, T, EPI,
+                                OUTF32, BI8, (s.PP && !BI8 && !RMS), RMS, RAGGED, (BI8 ? W8_SB : s.SB),
+                                (BI8 || s.PP || UNAL ? 1 : s.FD), UNAL>),
                      dim3((unsigned)blocks), dim3(threads), 0, stream, k);
   return hipGetLastError();
 }

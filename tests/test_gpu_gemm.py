@@ -124,6 +124,45 @@ def test_gemm_ragged_k_exact_integer(pkg, dev, layout, K):
     assert np.array_equal(c.cpu().numpy(), f16_round(exact.numpy()))
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("layout", ["nn", "nt"])
+@pytest.mark.parametrize("batch,M,N,K", [(1, 1, 9, 8), (1, 65, 63, 15), (3, 64, 64, 65), (2, 129, 197, 71),
+                                         (70, 197, 197, 64), (66, 131, 197, 197)])
+def test_gemm_unaligned_rows_exact(pkg, dev, layout, dtype, batch, M, N, K):
+    """Operands and C at odd element offsets with odd row strides (the tiles
+    loaded through registers; 64x64, and 128x128 from 256 tiles on): small
+    integers give exact sums, NaN around and between the rows must not reach
+    one, and the elements around and between C's rows stay untouched."""
+    g = torch.Generator().manual_seed(41)
+
+    def padded(rows, cols, fill):
+        ld = cols + 1 + cols % 2  # odd
+        buf = torch.full((1 + batch * rows * ld + 8,), fill, dtype=dtype)
+        return buf, lambda t: t[1:1 + batch * rows * ld].view(batch, rows, ld)[:, :, :cols]
+
+    abuf, a = padded(M, K, float("nan"))
+    bbuf, b = padded(*((K, N) if layout == "nn" else (N, K)), float("nan"))
+    cbuf, c = padded(M, N, 7.0)
+    a(abuf).copy_(torch.randint(-1, 2, (batch, M, K), generator=g))
+    b(bbuf).copy_(torch.randint(-1, 2, b(bbuf).shape, generator=g))  # |sums| <= 197: exact in bf16 too
+    cdev = cbuf.to(dev)
+    pkg.bgemm(a(abuf.to(dev)), b(bbuf.to(dev)), b_layout=layout, out=c(cdev))
+    torch.cuda.synchronize()
+    bt = b(bbuf).float() if layout == "nn" else b(bbuf).float().transpose(1, 2)
+    c(cbuf).copy_(torch.matmul(a(abuf).float(), bt))
+    assert torch.equal(cdev.cpu(), cbuf)
+
+
+@pytest.mark.parametrize("epi", ["bias", "gelu_tanh", "bias_gelu_tanh", "silu_mul"])
+def test_gemm_unaligned_rows_epilogues(pkg, dev, epi):
+    M, N, K = 77, 96 if epi == "silu_mul" else 93, 301
+    x, w, bias = normal((M, K), 42), normal((N, K), 43, std=0.05), normal((N + 1,), 44, std=0.1)
+    b = bias.to(dev)[1:] if "bias" in epi else None  # 2-byte aligned
+    y = pkg.gemm(x.to(dev), w.to(dev), b_layout="nt", epilogue=epi, bias=b)
+    exp = ref.gemm_epilogue(x.numpy(), w.numpy(), "nt", epi, bias[1:].numpy())
+    assert ref.max_rel_err(np32(y.cpu()), exp) <= TOL
+
+
 @pytest.mark.parametrize("epi", ["bias", "gelu_tanh", "bias_gelu_tanh", "silu_mul"])
 def test_gemm_ragged_k_epilogues(pkg, dev, epi):
     M, N, K = 200, 96 if epi == "silu_mul" else 93, 301
