@@ -33,11 +33,11 @@ HIPFLAGS = [
 ]
 
 
-# Per-source extra flags.  attention.hip rescales its MFMA accumulators with
-# vector ALU ops between MFMAs; with accumulators in AGPRs (the compiler's
-# default) every key block copies them to VGPRs and back, so that file asks
-# for the VGPR form of the MFMA operands.
-EXTRA = {"attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+# Per-source extra flags.  The attention kernel rescales its MFMA accumulators
+# with vector ALU ops between MFMAs; with accumulators in AGPRs (the
+# compiler's default) every key block copies them to VGPRs and back, so its
+# files ask for the VGPR form of the MFMA operands.
+EXTRA = {f"attention_{t}.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"] for t in ("f16", "bf16")}
 
 
 def hipcc() -> str:

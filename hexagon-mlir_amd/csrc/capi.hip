@@ -408,7 +408,9 @@ int hxmi_softmax_masked_bf16(const void* x, void* y, int64_t slices, int64_t s_q
 }
 
 namespace {
-int attention_common(const char* name, const void* q, const void* k, const void* v, void* o, int64_t bh,
+constexpr char kHeadDims[] = "%s: head dim %lld unsupported (64 or 128)";  // the fp16-only entries
+
+int attention_common(const char* name, int dtype, const void* q, const void* k, const void* v, void* o, int64_t bh,
                      int64_t s_q, int64_t s_kv, int64_t d, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldo,
                      int64_t stride_q, int64_t stride_k, int64_t stride_v, int64_t stride_o, int64_t kv_group,
                      const void* mask, int64_t ldm, int64_t stride_m, int64_t mask_group, int causal, float scale,
@@ -416,7 +418,6 @@ int attention_common(const char* name, const void* q, const void* k, const void*
   REQUIRE(bh >= 0 && s_q >= 0 && s_kv >= 0 && d >= 0, "%s: negative size", name);
   if (bh == 0 || s_q == 0) return ok();
   REQUIRE(s_kv > 0, "%s: softmax over zero keys", name);
-  REQUIRE(d == 64 || d == 128, "%s: head dim %lld unsupported (64 or 128)", name, (long long)d);
   REQUIRE(q && k && v && o, "%s: null pointer", name);
   REQUIRE(scale > 0.f && scale < INFINITY, "%s: scale must be positive and finite", name);
   REQUIRE(kv_group >= 1 && bh % kv_group == 0, "%s: kv_group %lld must divide bh %lld", name, (long long)kv_group,
@@ -460,16 +461,31 @@ int attention_common(const char* name, const void* q, const void* k, const void*
   p.mask_group = mask ? mask_group : 1;
   p.causal = causal;
   p.scale = scale;
+  p.dtype = dtype;
   return from_hip(hxmi::launch_attention(p, (hipStream_t)stream), name);
 }
 }  // namespace
+
+int hxmi_attention_ex(int is_bf16, const void* q, const void* k, const void* v, void* o, int64_t bh, int64_t s_q,
+                      int64_t s_kv, int64_t d, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldo, int64_t stride_q,
+                      int64_t stride_k, int64_t stride_v, int64_t stride_o, int64_t kv_group, const void* mask,
+                      int64_t ldm, int64_t stride_m, int64_t mask_group, int causal, float scale, void* stream) {
+  const char* name = "hxmi_attention_ex";
+  REQUIRE(is_bf16 == 0 || is_bf16 == 1, "%s: is_bf16 must be 0 or 1", name);
+  REQUIRE(bh <= 0 || s_q <= 0 || (d % 8 == 0 && d >= 8 && d <= 128),
+          "%s: head dim %lld unsupported (multiples of 8 up to 128)", name, (long long)d);
+  return attention_common(name, is_bf16 ? hxmi::DT_BF16 : hxmi::DT_F16, q, k, v, o, bh, s_q, s_kv, d, ldq, ldk, ldv,
+                          ldo, stride_q, stride_k, stride_v, stride_o, kv_group, mask, ldm, stride_m, mask_group,
+                          causal, scale, stream);
+}
 
 int hxmi_attention_ex_f16(const void* q, const void* k, const void* v, void* o, int64_t bh, int64_t s_q,
                           int64_t s_kv, int64_t d, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldo,
                           int64_t stride_q, int64_t stride_k, int64_t stride_v, int64_t stride_o, int64_t kv_group,
                           const void* mask, int64_t ldm, int64_t stride_m, int64_t mask_group, int causal,
                           float scale, void* stream) {
-  return attention_common("hxmi_attention_ex_f16", q, k, v, o, bh, s_q, s_kv, d, ldq, ldk, ldv, ldo, stride_q,
+  REQUIRE(bh <= 0 || s_q <= 0 || s_kv <= 0 || d == 64 || d == 128, kHeadDims, "hxmi_attention_ex_f16", (long long)d);
+  return attention_common("hxmi_attention_ex_f16", hxmi::DT_F16, q, k, v, o, bh, s_q, s_kv, d, ldq, ldk, ldv, ldo, stride_q,
                           stride_k, stride_v, stride_o, kv_group, mask, ldm, stride_m, mask_group, causal, scale,
                           stream);
 }
@@ -477,7 +493,8 @@ int hxmi_attention_ex_f16(const void* q, const void* k, const void* v, void* o, 
 int hxmi_attention_f16(const void* q, const void* k, const void* v, void* o, int64_t bh, int64_t s_q, int64_t s_kv,
                        int64_t d, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldo, int64_t stride_q,
                        int64_t stride_k, int64_t stride_v, int64_t stride_o, float scale, void* stream) {
-  return attention_common("hxmi_attention_f16", q, k, v, o, bh, s_q, s_kv, d, ldq, ldk, ldv, ldo, stride_q, stride_k,
+  REQUIRE(bh <= 0 || s_q <= 0 || s_kv <= 0 || d == 64 || d == 128, kHeadDims, "hxmi_attention_f16", (long long)d);
+  return attention_common("hxmi_attention_f16", hxmi::DT_F16, q, k, v, o, bh, s_q, s_kv, d, ldq, ldk, ldv, ldo, stride_q, stride_k,
                           stride_v, stride_o, 1, nullptr, 0, 0, 1, 0, scale, stream);
 }
 

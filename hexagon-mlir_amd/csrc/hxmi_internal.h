@@ -189,6 +189,7 @@ struct AttnProblem {
   int64_t mask_group;  // (batch, head) slices sharing one mask slice
   int causal;          // 0 none, 1 key <= query, 2 key <= query + skv - s
   float scale;
+  int dtype;  // DT_F16 or DT_BF16 (the mask is fp16 either way)
 };
 
 hipError_t launch_attention(const AttnProblem& p, hipStream_t stream);

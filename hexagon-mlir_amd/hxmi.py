@@ -54,6 +54,7 @@ SIGNATURES = {
     "hxmi_softmax_masked_f16": ([_P, _P] + [_I64] * 7 + [_P, _I64, _I64, _I64, _I, _F, _P], _I),
     "hxmi_softmax_masked_bf16": ([_P, _P] + [_I64] * 7 + [_P, _I64, _I64, _I64, _I, _F, _P], _I),
     "hxmi_attention_f16": ([_P, _P, _P, _P] + [_I64] * 12 + [_F, _P], _I),
+    "hxmi_attention_ex": ([_I, _P, _P, _P, _P] + [_I64] * 13 + [_P, _I64, _I64, _I64, _I, _F, _P], _I),
     "hxmi_attention_ex_f16": ([_P, _P, _P, _P] + [_I64] * 13 + [_P, _I64, _I64, _I64, _I, _F, _P], _I),
     "hxmi_rmsnorm_linear_f16": ([_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I, _F, _P, _P, _P], _I),
     "hxmi_rmsnorm_linear_bf16": ([_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I, _F, _P, _P, _P], _I),
@@ -562,6 +563,28 @@ def _mask_slices(mask: torch.Tensor, lead: tuple, S: int, Skv: int) -> tuple[tor
     return m, Skv, S * Skv, 1
 
 
+def _fused_attention_ok(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float,
+                        out: Optional[torch.Tensor]) -> bool:
+    """Whether attention() runs the fused kernel.  fp16 at head dims 64 and
+    128 always does; the others where the three steps take nothing more: at
+    least one key, K / V slices of at most 2 GiB, a finite scale, operands on
+    the 16-byte grid and an out whose rows take the kernel's 8-byte stores."""
+    D = q.shape[-1]
+    if q.dtype not in (torch.float16, torch.bfloat16) or k.dtype != q.dtype or v.dtype != q.dtype \
+            or v.shape[-1] != D or D % 8 or not 8 <= D <= 128 or not scale > 0:
+        return False
+    if q.dtype == torch.float16 and D in (64, 128):
+        return True
+    S, Skv = q.shape[-2], k.shape[-2]
+    if not 0 < Skv < 1 << 30 or S >= 1 << 30 or scale == float("inf"):
+        return False
+    if any(Skv * max(t.stride(-2), D) * 2 > 1 << 31 for t in (k, v)):
+        return False
+    if any(t.data_ptr() % 16 or (t.is_contiguous() and any(st % 8 for st in t.stride()[:-1])) for t in (q, k, v)):
+        return False  # (other tensors off the 16-byte grid are copied)
+    return out is None or (out.is_contiguous() and out.data_ptr() % 8 == 0)
+
+
 def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional[float] = None,
               out: Optional[torch.Tensor] = None, *, mask: Optional[torch.Tensor] = None,
               causal: int = 0) -> torch.Tensor:
@@ -569,9 +592,9 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional
     q [..., S, D], k and v [..., S_kv, D].  K/V may have fewer slices than q in their last leading dim
     (grouped-query attention: that many q heads per kv head).  mask: additive (or boolean keep) mask
     broadcastable to [..., S, S_kv]; causal: 1 masks keys after the query (torch's is_causal), 2 after
-    query + S_kv - S.  fp16 with D in {64, 128} and scale > 0 runs the fused kernel (hxmi_attention_ex_f16);
-    every other case (bf16, other head dims) runs the reference's three steps as bmm(Q, K^T) -> softmax
-    (with the mask and causal rule: hxmi_softmax_masked_*) -> bmm(P, V)."""
+    query + S_kv - S.  fp16 and bf16 with D a multiple of 8 up to 128 and scale > 0 run the fused kernel
+    (hxmi_attention_ex); every other case (other head dims, v of another width) runs the reference's three
+    steps as bmm(Q, K^T) -> softmax (with the mask and causal rule: hxmi_softmax_masked_*) -> bmm(P, V)."""
     if scale is None:
         scale = q.shape[-1] ** -0.5
     S, D = q.shape[-2:]
@@ -586,8 +609,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional
     q3 = q.reshape(-1, S, D)
     k3 = k.reshape(-1, Skv, D)
     v3 = v.reshape(-1, Skv, v.shape[-1])
-    if q.dtype == torch.float16 and D in (64, 128) and v.shape[-1] == D and k.dtype == v.dtype == q.dtype \
-            and scale > 0:
+    if _fused_attention_ok(q, k, v, scale, out):
         _require_gpu(q3, k3, v3)
         q3, k3, v3 = (t if t.stride(-1) == 1 and t.stride(1) % 8 == 0 and t.stride(0) % 8 == 0
                       and t.data_ptr() % 16 == 0 else t.contiguous() for t in (q3, k3, v3))
@@ -610,9 +632,10 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional
             _require_gpu(mask)
             m, ldm, sm, mg = _mask_slices(mask, lead, S, Skv)
             mp = m.data_ptr()
-        _check(load_library().hxmi_attention_ex_f16(q3.data_ptr(), k3.data_ptr(), v3.data_ptr(), o.data_ptr(),
-                                                    q3.shape[0], S, Skv, D, ldq, ldk, ldv, ldo, bq, bk, bv, bo,
-                                                    group, mp, ldm, sm, mg, int(causal), float(scale), _stream(q)))
+        _check(load_library().hxmi_attention_ex(int(q.dtype == torch.bfloat16), q3.data_ptr(), k3.data_ptr(),
+                                                v3.data_ptr(), o.data_ptr(), q3.shape[0], S, Skv, D, ldq, ldk, ldv,
+                                                ldo, bq, bk, bv, bo, group, mp, ldm, sm, mg, int(causal),
+                                                float(scale), _stream(q)))
         return out if out is not None else o.reshape(*lead, S, D)
     # The reference's three steps: bmm(Q, K^T) * scale -> (+ mask, causal)
     # softmax -> bmm(P, V).  The query heads of one K/V head form one batch

@@ -348,6 +348,18 @@ int hxmi_attention_ex_f16(const void* q, const void* k, const void* v, void* o, 
                           float scale, void* stream);
 
 /*
+ * The same for both 16-bit types (is_bf16: 0 fp16, 1 bf16; the mask is fp16
+ * either way) and every head dimension d that is a multiple of 8 up to 128.
+ * Other arguments as hxmi_attention_ex_f16.
+ * Replaces: tm_tensor.attention with its mask operand
+ * (LowerTmTensor.cpp:52-250).
+ */
+int hxmi_attention_ex(int is_bf16, const void* q, const void* k, const void* v, void* o, int64_t bh, int64_t s_q,
+                      int64_t s_kv, int64_t d, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldo, int64_t stride_q,
+                      int64_t stride_k, int64_t stride_v, int64_t stride_o, int64_t kv_group, const void* mask,
+                      int64_t ldm, int64_t stride_m, int64_t mask_group, int causal, float scale, void* stream);
+
+/*
  * One-token decoder step of a Llama / Qwen2 stack of `layers` layers at
  * position 0 (empty KV cache), fp16 in and out, fp32 accumulation, as ONE
  * persistent launch (plus the lm_head GEMV when w_lm is given):

@@ -328,6 +328,53 @@ def test_attention_three_step_negative_scale(pkg, dev):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("d", [8, 40, 64, 72, 96, 104, 128])
+@pytest.mark.parametrize("masked", [False, True])
+def test_attention_fused_head_dims(pkg, dev, dtype, d, masked):
+    """The fused kernel at head dims that fill its LDS rows only partly, in
+    both types: rows of NaN-padded buffers, 2 grouped heads per K/V head, more
+    keys than one LDS chunk, bottom-right causal, with and without a mask."""
+    b, hq, hkv, s, skv = 1, 4, 2, 70, 333
+
+    def padded(h, n, seed):
+        t = torch.full((b, h, n, d + 8), float("nan"), dtype=dtype)
+        t[..., :d] = uniform((b, h, n, d), seed, dtype=dtype)
+        return t
+
+    q, k, v = padded(hq, s, 211), padded(hkv, skv, 212), padded(hkv, skv, 213)
+    m = normal((s, skv), 214) if masked else None
+    dq, dk, dv = (t.to(dev)[..., :d] for t in (q, k, v))
+    assert pkg.hxmi._fused_attention_ok(dq, dk, dv, d**-0.5, None)
+    out = pkg.attention(dq, dk, dv, mask=m.to(dev) if masked else None, causal=2).cpu()
+    exp = ref.sdpa(*(np32(t[..., :d]) for t in (q, k, v)), d**-0.5, mask=np32(m) if masked else None, causal=2,
+                   kv_group=hq // hkv)
+    _check_nan_tol(out, exp, RMS[dtype])
+
+
+@pytest.mark.parametrize("bh,s", [(3, 200), (12, 700), (50, 512), (72, 512), (75, 512), (130, 512), (136, 512)])
+def test_attention_causal_block_orders(pkg, dev, bh, s):
+    """Every query block is computed once whatever order the causal rule gives
+    the workgroups: resident pairs (up to 512 of them, below and above 256)
+    and heaviest first, slices dividing over the 8 XCDs or not."""
+    q, k, v = (uniform((bh, s, 64), 221 + i) for i in range(3))
+    out = pkg.attention(q.to(dev), k.to(dev), v.to(dev), causal=1).cpu()
+    _check_nan_tol(out, ref.sdpa(np32(q), np32(k), np32(v), 0.125, causal=1), RMS[torch.float16])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_attention_three_step_value_width(pkg, dev, dtype):
+    """A value width other than the head dim stays on the three steps: mask,
+    grouped heads and the causal rule."""
+    b, hq, hkv, s, d, dv = 2, 4, 2, 77, 64, 40
+    q, k, v = uniform((b, hq, s, d), 231, dtype=dtype), uniform((b, hkv, s, d), 232, dtype=dtype), \
+        uniform((b, hkv, s, dv), 233, dtype=dtype)
+    m = normal((b, 1, s, s), 234)
+    out = pkg.attention(q.to(dev), k.to(dev), v.to(dev), mask=m.to(dev), causal=1).cpu()
+    exp = ref.sdpa(np32(q), np32(k), np32(v), d**-0.5, mask=np32(m), causal=1, kv_group=hq // hkv)
+    _check_nan_tol(out, exp, RMS[dtype])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_softmax_masked_through_abi(pkg, dev, dtype):
     """hxmi_softmax_masked_*: scores [slices, s_q, s_kv] in padded rows, scale,
     a mask shared by groups of two slices, causal = 2, in place and out of
