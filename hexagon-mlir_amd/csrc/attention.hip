@@ -13,14 +13,24 @@ namespace {
 int pick_cfg(const AttnProblem& p) {
   const int64_t forced = knob(KNOB_ATTN_CFG);
   if (forced != KNOB_UNSET) return (int)forced;
-  // Enough 128-query workgroups to cover most CUs: 4 query waves (x2 key
-  // splits at D = 64, where the merge fits in LDS); otherwise one query group
-  // per workgroup with the keys split over 4 waves (ViT-B/16 batch 8: 7.3 us
-  // against 7.6 / 10.8; a 32-head 512-token causal prefill: 8.3 us against
-  // 10.9 / 11.3, measured on MI355X)
-  const int64_t wg4 = p.bh * ((p.s + 127) / 128);
-  if (wg4 >= 192) return p.d <= 64 ? 42 : 41;
-  return 14;
+  // Queries per workgroup: the most that still spread over the chip, since
+  // each workgroup reads its K and V through LDS once; 128 queries are split
+  // over two halves of the keys to have eight waves (four with few keys, and
+  // at head dims over 64, whose merge and registers allow no more).  us, graph replays on MI355X, 128 / 64 / 32
+  // queries a workgroup:
+  //   head dim 64, full:    96 x 197 keys (192 / 384 / 672 workgroups) 7.0 (8 waves: 7.3) / 7.5 / 9.9; 48 x 257
+  //                         (144 / 240 / 432) 8.3 / 6.5 / 7.2; 32 x 577 (160 / 320 / 608) 10.7 / 11.5 /
+  //                         13.6; 32 x 300 (96 / 160 / 320) 8.1 / 6.5 / 7.2; 8 x 2048 (128 / 256 / 512)
+  //                         20.4 / 16.0 / 17.7; 4 x 2048 (64 / 128 / 256) 20.3 / 15.9 / 13.4
+  //   head dim 64, causal:  32 x 2048 (512 / 1024 / 2048) 25.1 / 28.8 / 38.7; 32 x 1024 (256 / 512 /
+  //                         1024) 13.8 / 11.3 / 15.4; 32 x 512 (128 / 256 / 512) 9.5 / 7.3 / 6.9
+  // With few keys a key split over four waves costs more than it spreads;
+  // and a causal workgroup count of two per CU lets heavy and light blocks
+  // pair up, so the causal lines lie at about twice the others.
+  const bool few_keys = p.skv <= 384;
+  const int64_t wg128 = p.bh * ((p.s + 127) / 128), wg64 = p.bh * ((p.s + 63) / 64);
+  if (wg128 >= (p.causal ? 320 : few_keys ? 192 : 144)) return p.d <= 64 && !few_keys ? 42 : 41;
+  return wg64 >= (few_keys ? 144 : p.causal ? 288 : 192) ? 22 : 14;
 }
 
 }  // namespace
@@ -41,8 +51,6 @@ hipError_t launch_attention(const AttnProblem& p, hipStream_t stream) {
   a.mask_group = (int)(p.mask_group > 0 ? p.mask_group : 1);
   a.causal_off = p.causal == 1 ? 0 : p.causal == 2 ? (int)(p.skv - p.s) : (int)p.skv;
   a.mask_vec = p.mask && p.ldm % 4 == 0 && p.sm % 4 == 0 && ((uintptr_t)p.mask & 7) == 0;
-  a.kbytes = (uint32_t)(((p.skv - 1) * p.ldk + p.d) * 2);
-  a.vbytes = (uint32_t)(((p.skv - 1) * p.ldv + p.d) * 2);
   a.ldq = p.ldq;
   a.ldk = p.ldk;
   a.ldv = p.ldv;

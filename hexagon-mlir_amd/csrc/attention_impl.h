@@ -12,10 +12,10 @@
 //     QG x KS waves: wave (qg, kh) takes the 32 queries of group qg against
 //     every KS-th block of 32 keys, and the KS partial (max, sum, O) of a
 //     query group are merged through LDS at the end;
-//   * K and V pass through LDS in chunks of 256 keys (D = 64; 128 for
-//     D = 128: 64 KB either way) with direct global->LDS buffer loads, whose
-//     out-of-range rows read as zeros; a head dim below 64 / 128 fills its
-//     rows up with zeros there (and for 72-96 leaves out the MFMAs of the
+//   * K and V pass through two LDS stages of 128 keys (D = 64; 64 keys for
+//     D = 128) with direct global->LDS buffer loads, one stage ahead of the
+//     one computed; rows out of range read as zeros, and a head dim below
+//     64 / 128 fills its rows up with zeros (72-96 leave out the MFMAs of the
 //     last quarter);
 //   * S is computed as D[key][query] = K . Q^T with v_mfma_f32_32x32x16_f16,
 //     so every lane owns one query's scores: the row max / sum are in-lane
@@ -27,6 +27,14 @@
 //     the P.V MFMA for two 16-key steps (the k order inside an MFMA is free as
 //     long as both operands use the same one); the matching V^T operand comes
 //     from LDS with ds_read_b64_tr_b16, so P never leaves registers;
+//   * the vector ALUs bound it (a 32 x 32 tile's softmax is ~62 of their
+//     instructions, 16 of them v_exp_f32 at half rate, against 8-16 MFMAs of 32
+//     clocks).  Two blocks at a time share one maximum, one rescale test and
+//     two independent MFMA chains, and leave four waves a SIMD at head dim
+//     64 (122 registers); with the stage loads out of the way, 32 heads x
+//     2048 x 2048 at head dim 64 went 53.0 -> 42.9 us (800 TFLOP/s), causal
+//     33.2 -> 26.3, head dim 128 x 4096 312 -> 277 us (994 TFLOP/s) against one
+//     stage of twice the keys, waited for whole, and one block at a time;
 //   * O = D[d][query] accumulates in registers and is divided by the sum of
 //     the same 16-bit weights once at the end.  A query whose every key is
 //     masked divides 0 by 0 (NaN), as the reference's decomposition does.
@@ -57,7 +65,6 @@ struct AArgs {
   int causal_off;  // key > query + causal_off is masked (skv: no causal rule)
   int mask_vec;    // mask rows allow aligned 8-byte loads
   int order;       // OrderId: workgroup -> (slice, query block)
-  uint32_t kbytes, vbytes;  // extent of one K / V slice
   int64_t ldq, ldk, ldv, ldo, ldm;  // row strides, elements
   int64_t bq, bk, bv, bo, bm;       // slice strides, elements
   float c;                          // scale * log2(e)
@@ -154,35 +161,37 @@ __device__ __forceinline__ int v_off(int r, int c) {
   return r * (2 * D) + ((c ^ v_swz<D>(r)) << 4);
 }
 
-// Head dims up to 64 run in LDS rows of D = 64, others in rows of 128.
-// DT: 32-wide output tiles computed (fewer than D / 32 for head dims 72-96).
-template <int D, int QG, int KS>
+// Head dims up to 64 run in LDS rows of D = 64, others in rows of 128.  K and
+// V pass through ST LDS stages of KC keys, 64 KB in all (two workgroups a
+// CU); a wave takes NB 32-key blocks at a time (a group), GPC groups a stage.
+template <int D, int QG, int KS, bool MASK>
 struct AttnShape {
   static constexpr int NT = 64 * QG * KS;
-  static constexpr int KC = D == 64 ? 256 : 128;  // keys per LDS chunk
-  static constexpr int CHUNK = KC * 2 * D;        // bytes of K (and of V) per chunk: 32 KB
-  static constexpr int NV = D / 32 * 16 + 2;      // floats per lane in the key-split merge
-  static constexpr bool ok = NT <= 1024 && (KS - 1) * QG * NV * 64 * 4 <= 2 * CHUNK;
+  static constexpr int KC = D == 64 || KS == 4 ? 128 : 64;
+  static constexpr int ST = KC * D > 8192 ? 1 : 2;
+  static constexpr int NB = KC / 32 / KS >= 2 && !MASK ? 2 : 1;  // (two blocks' mask entries would not fit)
+  static constexpr int GPC = KC / 32 / KS / NB;
+  static constexpr int CHUNK = KC * 2 * D;    // bytes of K (and of V) per stage: 16 or 32 KB
+  static constexpr int NV = D / 32 * 16 + 2;  // floats per lane in the key-split merge
+  static constexpr int WPE = QG * KS / 2;     // waves per SIMD that two workgroups a CU make
+  static constexpr bool ok = NT <= 1024 && (KS - 1) * QG * NV * 64 * 4 <= 2 * ST * CHUNK;
 };
 
-// PIPE: the key blocks of a chunk start load index by load index (below);
-// chosen at launch for sequences of at least one chunk.
+// DT: 32-wide output tiles computed (fewer than D / 32 for head dims 72-96).
 // PART: the head dim a.d is below D; rows fill up with zeros.
-template <typename T, int D, int DT, bool PART, int QG, int KS, bool MASK, bool PIPE>
-__global__ __launch_bounds__(64 * QG * KS) void attention_fwd(AArgs a) {
-  using Sh = AttnShape<D, QG, KS>;
+template <typename T, int D, int DT, bool PART, int QG, int KS, bool MASK>
+__global__ __launch_bounds__(64 * QG * KS, (AttnShape<D, QG, KS, MASK>::WPE)) void attention_fwd(AArgs a) {
+  using Sh = AttnShape<D, QG, KS, MASK>;
   static_assert(Sh::ok, "attention shape");
   constexpr int NW = QG * KS;
-  constexpr int KC = Sh::KC;
+  constexpr int KC = Sh::KC, NB = Sh::NB, GPC = Sh::GPC, ST = Sh::ST;
   constexpr int CHUNK = Sh::CHUNK;
   constexpr int RB = 2 * D;     // bytes per K / V row
   constexpr int DS = DT * 2;    // 16-deep MFMA steps over the head dim
   static_assert(PART || DT == D / 32, "whole rows");
-  constexpr int LPW = CHUNK / 1024 / NW;  // 1 KB direct loads of K (and of V) per wave per chunk
-  static_assert(LPW * NW * 1024 == CHUNK, "chunk split");
-  __shared__ __attribute__((aligned(1024))) char lds[2 * CHUNK];
-  char* const ks = lds;
-  char* const vs = lds + CHUNK;
+  constexpr int LPW = CHUNK / 1024 / NW;  // 1 KB direct loads of K (and of V) per wave per stage
+  static_assert(LPW * NW * 1024 == CHUNK, "stage split");
+  __shared__ __attribute__((aligned(1024))) char lds[2 * ST * CHUNK];  // K, V of stage 0, then of stage 1
 
   const int lane = threadIdx.x & 63;
   // wave-uniform values live in scalar registers, so branches on them are
@@ -205,51 +214,14 @@ __global__ __launch_bounds__(64 * QG * KS) void attention_fwd(AArgs a) {
   const int wg_qlast = min(qb0 + 32 * QG, a.sq) - 1;
   const int kend = min(a.skv, wg_qlast + a.causal_off + 1);
   const int wkend = q0 < a.sq ? max(0, min(a.skv, min(q0 + 31, a.sq - 1) + a.causal_off + 1)) : 0;
+  const int nchunk = kend > 0 ? (kend + KC - 1) / KC : 0;
 
   const _Float16* mrow = nullptr;
   if (MASK && qme < a.sq)
     mrow = (const _Float16*)a.mask + ((int64_t)(bh / a.mask_group) * a.bm + (int64_t)qme * a.ldm);
 
-  // direct loads: wave w's load i fills LDS bytes [(i*NW + w) KB, +1 KB) of
-  // the chunk; lane l's 16 bytes there are row (i*NW + w) * (1024/RB) + lr,
-  // stored chunk cs, which holds the row's chunk cs ^ swizzle(row)
-  const int lr = lane / (RB / 16), cs = lane % (RB / 16);
-  const __amdgpu_buffer_rsrc_t rK = make_rsrc(Kp, a.kbytes);
-  const __amdgpu_buffer_rsrc_t rV = make_rsrc(Vp, a.vbytes);
-
-  float16v oacc[DT];
-#pragma unroll
-  for (int t = 0; t < DT; ++t) oacc[t] = float16v{};
-  float m_run = -INFINITY, l_run = 0.f;
-  // This lane's V^T fragment reads for output tile dt sit at vbase[dt] plus
-  // a multiple of 4 rows: the chunk's V swizzle depends on (row & 3) only,
-  // so rows 4h + L/4 + 32b + 16t (+ 8) share one column offset.
-  int vbase[DT];
-#pragma unroll
-  for (int dt = 0; dt < DT; ++dt) {
-    const int g = lane >> 4, L = lane & 15;
-    const int d = dt * 32 + ((g & 1) << 4) + ((L & 3) << 2);
-    vbase[dt] = v_off<D>(4 * h + (L >> 2), d >> 3) + (d & 7) * 2;
-  }
-
-  auto issue_chunk = [&](int c0) {
-#pragma unroll
-    for (int i = 0; i < LPW; ++i) {
-      const int row = (i * NW + w) * (1024 / RB) + lr;
-      const int key = c0 + row;
-      const bool live = key < kend;
-      const int kc = cs ^ k_swz<D>(row), vc = cs ^ v_swz<D>(row);
-      const uint32_t ko = live && !(PART && kc * 8 >= a.d) ? (uint32_t)(key * a.ldk * 2 + (kc << 4)) : kOOB;
-      const uint32_t vo = live && !(PART && vc * 8 >= a.d) ? (uint32_t)(key * a.ldv * 2 + (vc << 4)) : kOOB;
-      load_lds16(rK, (HXMI_LDS void*)to_lds(ks + (i * NW + w) * 1024), ko);
-      load_lds16(rV, (HXMI_LDS void*)to_lds(vs + (i * NW + w) * 1024), vo);
-    }
-  };
-  // Q fragments of this wave's 32 queries (zero past the sequence), then
-  // the first chunk's K / V: the chunk's loads are waited for load index by
-  // load index (below), which leaves the later ones in flight only when Q
-  // was issued before them.  The Q loads take no branch (an offset past the
-  // buffer reads zeros), so the compiler does not wait for them early.
+  // Q fragments of this wave's 32 queries (zero past the sequence).  The
+  // loads take no branch (an offset past the buffer reads zeros).
   short8v qf[DS];
   {
     const __amdgpu_buffer_rsrc_t rQ = make_rsrc(Q, 0x7fffffffu);
@@ -260,160 +232,222 @@ __global__ __launch_bounds__(64 * QG * KS) void attention_fwd(AArgs a) {
                                   ? (uint32_t)(((int64_t)qme * a.ldq + s * 16 + h * 8) * 2)
                                   : kOOB));
   }
-  if (kend > 0) issue_chunk(0);
 
-  // Keys [c0, c0 + KC) of one chunk, its loads issued: load index i of every
-  // wave brings keys [i KPL, (i + 1) KPL) of K and V.  PIPE: before the key
-  // blocks of round j (block kh + j KS of wave kh) every wave waits for its
-  // loads up to the last index the round reads (the next round's K for the
-  // scores computed ahead), then one barrier, so the first blocks start when
-  // their keys have landed rather than the whole chunk.  That pays on full
-  // chunks (2 x 12 x 1024: 17.2 -> 16.85 us; head dim 128, 16 x 512 causal:
-  // 10.47 -> 10.15 us) but not on a short one, where the extra barriers
-  // cost more than the overlap gives (ViT-B/16, 197 keys: 7.47 -> 7.56 us),
-  // so the launch takes PIPE only for sequences of at least KC keys; the
-  // other instance waits for the first half of the chunk, then for the
-  // rest (ViT-B/16 7.35-7.41 -> 7.31-7.32 us against one wait for all).  (One kernel with both
-  // paths, chosen per chunk, took 30-60 more VGPRs, and the head-dim-128
-  // instances then held one wave per SIMD instead of two.)
-  constexpr int KPL = NW * (1024 / RB);
-  constexpr int JMAX = KC / 32 / KS;
-  constexpr auto li_end = [](int b) constexpr {
-    const int i = ((b + 1) * 32 - 1) / KPL;  // the load index of block b's last key, within the chunk
-    return i < LPW - 1 ? i : LPW - 1;
+  // Direct loads: wave w's load i fills LDS bytes [(i*NW + w) KB, +1 KB) of
+  // the stage's K (V); lane l's 16 bytes there are row (i*NW + w) *
+  // (1024/RB) + lr, stored chunk cs, which holds the row's chunk cs ^
+  // swizzle(row).  The offsets are those of the first stage; a later one
+  // moves the buffer's base, and keys from kend on lie past its end.
+  const int lr = lane / (RB / 16), cs = lane % (RB / 16);
+  uint32_t ko[LPW], vo[LPW];
+#pragma unroll
+  for (int i = 0; i < LPW; ++i) {
+    const int row = (i * NW + w) * (1024 / RB) + lr;
+    const int kc = cs ^ k_swz<D>(row), vc = cs ^ v_swz<D>(row);
+    const int64_t kr = row * a.ldk * 2, vr = row * a.ldv * 2;  // (a slice spans at most 2 GiB)
+    ko[i] = (PART && kc * 8 >= a.d) || kr >= kOOB ? kOOB : (uint32_t)kr + (kc << 4);
+    vo[i] = (PART && vc * 8 >= a.d) || vr >= kOOB ? kOOB : (uint32_t)vr + (vc << 4);
+  }
+  auto issue = [&](int c, int stage) {
+    const int left = kend - c * KC;  // > 0
+    char* const base = lds + stage * 2 * CHUNK;
+    const __amdgpu_buffer_rsrc_t rK =
+        make_rsrc(Kp + (int64_t)c * KC * a.ldk * 2, (uint32_t)(((left - 1) * a.ldk + a.d) * 2));
+    const __amdgpu_buffer_rsrc_t rV =
+        make_rsrc(Vp + (int64_t)c * KC * a.ldv * 2, (uint32_t)(((left - 1) * a.ldv + a.d) * 2));
+#pragma unroll
+    for (int i = 0; i < LPW; ++i) {
+      load_lds16(rK, (HXMI_LDS void*)to_lds(base + (i * NW + w) * 1024), ko[i]);
+      load_lds16(rV, (HXMI_LDS void*)to_lds(base + CHUNK + (i * NW + w) * 1024), vo[i]);
+    }
   };
-  auto run_chunk = [&](int c0) {
-    const int cn = min(KC, wkend - c0);
-    const int nblk = cn > 0 ? (cn + 31) >> 5 : 0;
-    // S block b: D[key][query], lane holds query lane%32, keys 8g + 4h + j
-    auto scores = [&](int b) {
-      float16v sb = {};
+
+  float16v oacc[DT];
 #pragma unroll
-      for (int st = 0; st < DS; ++st) {
-        const short8v kf = *(const short8v*)(ks + k_off<D>(b * 32 + (lane & 31), st * 2 + h));
-        sb = Num<T>::mfma(kf, qf[st], sb);
-      }
-      return sb;
-    };
-    // mask entries of block b's 16 scores of this lane: keys kb + 8g + 4h + j
-    auto mask_vals = [&](int b, _Float16 (&mk)[16]) {
-      const int kb = c0 + b * 32;
+  for (int t = 0; t < DT; ++t) oacc[t] = float16v{};
+  float m_run = -INFINITY, l_run = 0.f;
+  // This lane's K fragment of step st and V^T fragment of output tile dt in
+  // a stage sit at kbase[st] / vbase[dt] plus a multiple of 32 / 4 rows:
+  // neither swizzle changes over those.
+  int kbase[DS], vbase[DT];
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int kk = kb + 8 * g + 4 * h;
-        if (mrow && a.mask_vec && kk + 4 <= a.skv) {
-          const half4v m4 = *(const half4v*)(mrow + kk);
+  for (int st = 0; st < DS; ++st) kbase[st] = k_off<D>(lane & 31, st * 2 + h);
 #pragma unroll
-          for (int j = 0; j < 4; ++j) mk[4 * g + j] = m4[j];
-        } else {
+  for (int dt = 0; dt < DT; ++dt) {
+    const int g = lane >> 4, L = lane & 15;
+    const int d = dt * 32 + ((g & 1) << 4) + ((L & 3) << 2);
+    vbase[dt] = CHUNK + v_off<D>(4 * h + (L >> 2), d >> 3) + (d & 7) * 2;
+  }
+
+  // mask entries of the 32-key block at kb for this lane's 16 scores: keys kb + 8g + 4h + j
+  auto mask_vals = [&](int kb, half4v (&mk)[4]) {
 #pragma unroll
-          for (int j = 0; j < 4; ++j) mk[4 * g + j] = (mrow && kk + j < a.skv) ? mrow[kk + j] : (_Float16)0.f;
-        }
-      }
-    };
-    // Block b: its scores s (and mask entries mk) are in registers; the MFMAs
-    // of the next block's scores (and its mask loads) go out into s_nx / mk_nx
-    // first, so they run while this block's softmax occupies the vector
-    // ALUs.
-    auto block = [&](int b, float16v& s, float16v& s_nx, _Float16 (&mk)[16], _Float16 (&mk_nx)[16]) {
-      const int kb = c0 + b * 32;
-      if (MASK && b + KS < nblk) mask_vals(b + KS, mk_nx);
-      if (b + KS < nblk) s_nx = scores(b + KS);
-      // ragged keys and the causal rule only reach the blocks at their edges
-      const bool edge = kb + 32 > a.skv || kb + 31 > q0 + a.causal_off;
-      const bool scaled = MASK || edge;
-      float mx = -INFINITY;
-      if (scaled) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          float t = s[i] * a.c;
-          if constexpr (MASK) t = fmaf((float)mk[i], kLog2e, t);
-          if (edge) {
-            const int key = kb + 8 * (i >> 2) + 4 * h + (i & 3);
-            if (key >= a.skv || key > qme + a.causal_off) t = -INFINITY;
-          }
-          s[i] = t;
-          mx = fmaxf(mx, t);
-        }
+    for (int g = 0; g < 4; ++g) {
+      const int kk = kb + 8 * g + 4 * h;
+      if (mrow && a.mask_vec && kk + 4 <= a.skv) {
+        mk[g] = *(const half4v*)(mrow + kk);
       } else {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
-        mx *= a.c;  // scale > 0
+        for (int j = 0; j < 4; ++j) mk[g][j] = (mrow && kk + j < a.skv) ? mrow[kk + j] : (_Float16)0.f;
       }
-      mx = xor32_max(mx);
-      const bool upd = mx > m_run + 8.0f;
-      if (__any(upd)) {
-        const float alpha = upd ? __builtin_amdgcn_exp2f(m_run - mx) : 1.0f;  // 0 on a first block
-        if (upd) m_run = mx;
-        l_run *= alpha;
+    }
+  };
+
+  // The group of keys from kb on, its K rows at `rows` in LDS.  EDGE: some
+  // of the keys may be past the sequence or the causal limit.
+  auto group = [&](auto EDGE_, int kb, const char* rows, half4v (&mk)[MASK ? NB : 1][4]) {
+    constexpr int N = NB;
+    constexpr bool SCALED = decltype(EDGE_)::value;  // scores multiplied by a.c before the maximum
+    // S: D[key][query], lane holds query lane%32, keys 8g + 4h + j of each
+    // block.  Fragments are read one step ahead of their MFMAs; the
+    // scheduling barriers keep the compiler from reading them all first,
+    // which costs the registers of a wave per SIMD.
+    float16v s[N];
+    short8v kf[2][N], vf[2][DT];
+    auto read_k = [&](int st) {
 #pragma unroll
-        for (int t = 0; t < DT; ++t) oacc[t] *= alpha;
-      }
-      const float m_use = m_run == -INFINITY ? 0.f : m_run;  // every key so far masked: weights 0
-      const float cs = scaled ? 1.0f : a.c;                    // s already scaled on the edge path
-      typename Num<T>::pair p2[8];
+      for (int n = 0; n < N; ++n) kf[st & 1][n] = *(const short8v*)(rows + kbase[st] + n * 32 * RB);
+    };
+    // V^T of the 16-key step u: keys {16u + 4h + j, 16u + 8 + 4h + j}, at
+    // rows 16 u (+ 8) past this lane's V base
+    auto read_v = [&](int u) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
-        p2[i] = typename Num<T>::pair{(T)__builtin_amdgcn_exp2f(fmaf(s[2 * i], cs, -m_use)),
-                                      (T)__builtin_amdgcn_exp2f(fmaf(s[2 * i + 1], cs, -m_use))};
-      // the row sum uses the 16-bit weights P.V sees, so O is their exact
-      // weighted average (a constant V comes back unchanged)
-      float psum = 0.f;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) psum = Num<T>::add_pair(p2[i], psum);
-      l_run += psum;
-      // two 16-key MFMA steps: step t uses keys {16t + 4h + j, 16t + 8 + 4h + j},
-      // at rows 32 b + 16 t (+ 8) past this lane's V base
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        short8v pf;
-        __builtin_memcpy(&pf, &p2[4 * t], 16);
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-          const char* vb = vs + vbase[dt] + (b * 32 + 16 * t) * RB;
-          const short4v lo = lds_read_tr16(vb);
-          const short4v hi = lds_read_tr16(vb + 8 * RB);
-          const short8v vf = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-          oacc[dt] = Num<T>::mfma(vf, pf, oacc[dt]);
-        }
+      for (int dt = 0; dt < DT; ++dt) {
+        const char* vb = rows + vbase[dt] + 16 * u * RB;
+        const short4v lo = lds_read_tr16(vb);
+        const short4v hi = lds_read_tr16(vb + 8 * RB);
+        vf[u & 1][dt] = short8v{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
       }
     };
-    constexpr bool pipe = PIPE;
-    // (the other instance: the first half of the chunk, then the rest)
-    constexpr int L0 = pipe ? li_end(KS - 1) : (li_end(KS - 1) > LPW / 2 - 1 ? li_end(KS - 1) : LPW / 2 - 1);
-    wait_vmcnt<2 * (LPW - 1 - L0)>();
-    barrier_after_lds_loads();
-    float16v s_next = kh < nblk ? scores(kh) : float16v{};
-    _Float16 mk_next[16];
-    if (MASK && kh < nblk) mask_vals(kh, mk_next);
-    static_for<JMAX>([&](auto J) {
-      constexpr int j = decltype(J)::value;
-      constexpr int need = li_end(KS - 1 + (j + 1) * KS), prev = li_end(KS - 1 + j * KS);
-      constexpr int wn = pipe ? need : (need <= L0 ? L0 : LPW - 1);
-      constexpr int wp = pipe ? prev : (prev <= L0 ? L0 : LPW - 1);
-      if constexpr (wn > wp) {
-        wait_vmcnt<2 * (LPW - 1 - wn)>();
-        barrier_after_lds_loads();
-      }
-      const int b = kh + j * KS;
-      if (b < nblk) {
-        float16v s = s_next;
-        _Float16 mk[16];
-        if constexpr (MASK) {
+    read_k(0);
 #pragma unroll
-          for (int i = 0; i < 16; ++i) mk[i] = mk_next[i];
+    for (int st = 0; st < DS; ++st) {
+      if (st + 1 < DS) read_k(st + 1);
+      else read_v(0);
+#pragma unroll
+      for (int n = 0; n < N; ++n) s[n] = Num<T>::mfma(kf[st & 1][n], qf[st], st == 0 ? float16v{} : s[n]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (SCALED) {
+#pragma unroll
+      for (int n = 0; n < N; ++n)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          s[n][i] *= a.c;
+          if constexpr (MASK) s[n][i] = fmaf((float)mk[n][i >> 2][i & 3], kLog2e, s[n][i]);
         }
-        block(b, s, s_next, mk, mk_next);
+      if (kb + N * 32 > min(a.skv, q0 + a.causal_off + 1)) {  // (wave-uniform)
+        const int last = min(a.skv - 1, qme + a.causal_off) - kb - 4 * h;
+#pragma unroll
+        for (int n = 0; n < N; ++n)
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            if (n * 32 + 8 * (i >> 2) + (i & 3) > last) s[n][i] = -INFINITY;
       }
-    });
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[n][i]);
+    if constexpr (!SCALED) mx *= a.c;  // scale > 0
+    mx = xor32_max(mx);
+    const bool upd = mx > m_run + 8.0f;
+    if (__any(upd)) {
+      const float alpha = upd ? __builtin_amdgcn_exp2f(m_run - mx) : 1.0f;  // 0 on a first block
+      if (upd) m_run = mx;
+      l_run *= alpha;
+#pragma unroll
+      for (int t = 0; t < DT; ++t) oacc[t] *= alpha;
+    }
+    const float m_use = m_run == -INFINITY ? 0.f : m_run;  // every key so far masked: weights 0
+    const float sc = SCALED ? 1.0f : a.c;
+    // The weights of a step are taken while the MFMAs of the step before it
+    // run.  The row sum uses the 16-bit weights P.V sees, so O is their
+    // exact weighted average (a constant V comes back unchanged).
+    float psum = 0.f;
+    auto weights = [&](int u) {
+      typename Num<T>::pair p2[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int e = (u & 1) * 8 + 2 * i;
+        p2[i] = typename Num<T>::pair{(T)__builtin_amdgcn_exp2f(fmaf(s[u >> 1][e], sc, -m_use)),
+                                      (T)__builtin_amdgcn_exp2f(fmaf(s[u >> 1][e + 1], sc, -m_use))};
+        psum = Num<T>::add_pair(p2[i], psum);
+      }
+      short8v pf;
+      __builtin_memcpy(&pf, p2, 16);
+      return pf;
+    };
+    short8v pf = weights(0);
+#pragma unroll
+    for (int u = 0; u < 2 * N; ++u) {
+      short8v pn = pf;
+      if (u + 1 < 2 * N) {
+        read_v(u + 1);
+        pn = weights(u + 1);
+      }
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) oacc[dt] = Num<T>::mfma(vf[u & 1][dt], pf, oacc[dt]);
+      pf = pn;
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    l_run += psum;
   };
-  // the first chunk outside the loop: the compiler waits for every
-  // outstanding load before a loop that reads registers loaded before it (Q)
-  if (kend > 0) run_chunk(0);
-  for (int c0 = KC; c0 < kend; c0 += KC) {
-    __syncthreads();  // previous chunk fully consumed
-    issue_chunk(c0);
-    run_chunk(c0);
+
+  // Two stages, one barrier a stage: past the barrier every wave's loads of
+  // stage c have landed and every wave is done with stage c - 1, which
+  // takes the loads of stage c + 1 while stage c is computed.  The first two
+  // stages are issued together.  (One stage: its loads wait until every wave
+  // is done with it, and only the other workgroup of the CU covers them.)
+  if (nchunk > 0) issue(0, 0);
+  if (ST == 2 && nchunk > 1) issue(1, 1);
+  auto stage_in = [&](int c) {
+    if (ST == 1 && c > 0) {
+      barrier_before_refill();
+      issue(c, 0);
+    }
+    if (ST == 2 && c == 0 && nchunk > 1) wait_vmcnt<2 * LPW>();
+    else wait_vmcnt0();
+    barrier_before_refill();
+  };
+  auto stage_out = [&](int c) {
+    if (ST == 2 && c > 0 && c + 1 < nchunk) issue(c + 1, (c + 1) & 1);
+  };
+  auto stage_at = [&](int c) { return lds + (c & (ST - 1)) * 2 * CHUNK; };
+  // Leading stages that no wave needs the edge form for (a uniform count:
+  // the waves meet at the barriers), then the rest.
+  int nfull = 0;
+  if constexpr (!MASK) nfull = max(0, min(a.skv, qb0 + a.causal_off + 1) / KC);
+  half4v mk[MASK ? GPC : 1][MASK ? NB : 1][4];
+  int c = 0;
+  for (; c < min(nfull, nchunk); ++c) {
+    stage_in(c);
+    stage_out(c);
+#pragma unroll
+    for (int g = 0; g < GPC; ++g) {
+      const int row = (g * KS + kh) * NB * 32;
+      group(std::false_type{}, c * KC + row, stage_at(c) + row * RB, mk[0]);
+    }
+  }
+  for (; c < nchunk; ++c) {
+    stage_in(c);
+    if constexpr (MASK) {  // before the next stage's loads: loads return in order
+#pragma unroll
+      for (int g = 0; g < GPC; ++g)
+#pragma unroll
+        for (int n = 0; n < NB; ++n) {
+          const int kb = c * KC + ((g * KS + kh) * NB + n) * 32;
+          if (kb < wkend) mask_vals(kb, mk[g][n]);
+        }
+    }
+    stage_out(c);
+#pragma unroll
+    for (int g = 0; g < GPC; ++g) {
+      const int row = (g * KS + kh) * NB * 32;
+      if (c * KC + row < wkend)
+        group(std::true_type{}, c * KC + row, stage_at(c) + row * RB, mk[MASK ? g : 0]);
+    }
   }
 
   // merge the key-split partials of each query group into wave kh = 0
@@ -468,7 +502,7 @@ __global__ __launch_bounds__(64 * QG * KS) void attention_fwd(AArgs a) {
 
 template <typename T, int D, int DT, bool PART, int QG, int KS>
 hipError_t launch_cfg(AArgs a, const AttnProblem& p, bool mask, hipStream_t stream) {
-  if constexpr (!AttnShape<D, QG, KS>::ok) {
+  if constexpr (!AttnShape<D, QG, KS, false>::ok) {
     return hipErrorNotSupported;
   } else {
     a.nqb = (int)((p.s + 32 * QG - 1) / (32 * QG));
@@ -476,15 +510,10 @@ hipError_t launch_cfg(AArgs a, const AttnProblem& p, bool mask, hipStream_t stre
     if (blocks >= (1ll << 31)) return hipErrorInvalidValue;
     a.order = !p.causal ? ORDER_SLICES : (blocks <= 512 ? ORDER_PAIRED : ORDER_HEAVY);
     const dim3 grid((unsigned)blocks), block(64 * QG * KS);
-    const bool pipe = p.skv >= AttnShape<D, QG, KS>::KC;
-    if (mask && pipe)
-      hipLaunchKernelGGL((attention_fwd<T, D, DT, PART, QG, KS, true, true>), grid, block, 0, stream, a);
-    else if (mask)
-      hipLaunchKernelGGL((attention_fwd<T, D, DT, PART, QG, KS, true, false>), grid, block, 0, stream, a);
-    else if (pipe)
-      hipLaunchKernelGGL((attention_fwd<T, D, DT, PART, QG, KS, false, true>), grid, block, 0, stream, a);
+    if (mask)
+      hipLaunchKernelGGL((attention_fwd<T, D, DT, PART, QG, KS, true>), grid, block, 0, stream, a);
     else
-      hipLaunchKernelGGL((attention_fwd<T, D, DT, PART, QG, KS, false, false>), grid, block, 0, stream, a);
+      hipLaunchKernelGGL((attention_fwd<T, D, DT, PART, QG, KS, false>), grid, block, 0, stream, a);
     return hipGetLastError();
   }
 }
@@ -498,11 +527,11 @@ hipError_t launch_d(const AArgs& a, const AttnProblem& p, int cfg, hipStream_t s
     case 41: return launch_cfg<T, D, DT, PART, 4, 1>(a, p, m, stream);
     case 14: return launch_cfg<T, D, DT, PART, 1, 4>(a, p, m, stream);
     case 42: return launch_cfg<T, D, DT, PART, 4, 2>(a, p, m, stream);
+    case 22: return launch_cfg<T, D, DT, PART, 2, 2>(a, p, m, stream);
     default: break;
   }
   if constexpr (std::is_same_v<T, _Float16> && !PART) {
     switch (cfg) {
-      case 22: return launch_cfg<T, D, DT, PART, 2, 2>(a, p, m, stream);
       case 21: return launch_cfg<T, D, DT, PART, 2, 1>(a, p, m, stream);
       case 12: return launch_cfg<T, D, DT, PART, 1, 2>(a, p, m, stream);
       case 24: return launch_cfg<T, D, DT, PART, 2, 4>(a, p, m, stream);
