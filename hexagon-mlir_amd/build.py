@@ -1,4 +1,5 @@
-"""Build libhxmi.so (the C-ABI kernel library) in-tree with hipcc for gfx950.
+"""Build libhxmi.so (the C-ABI kernel library) in-tree with hipcc for gfx950,
+and hxmi_torch.so (the native entry of the torch-facing ops) on top of it.
 
     python hexagon-mlir_amd/build.py [--jobs N]
 
@@ -20,6 +21,7 @@ PKG = pathlib.Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 BUILD = CSRC / "_build"
 LIB = PKG / "lib" / "libhxmi.so"
+OPS = PKG / "lib" / "hxmi_torch.so"
 ARCH = "gfx950"
 
 # -packed-fp32-ops: keep hipcc from emitting packed fp32 VALU ops.
@@ -56,6 +58,27 @@ def _compile(src: pathlib.Path) -> pathlib.Path:
     return obj
 
 
+def _build_ops() -> None:
+    """torch_ops.cpp is host code only: g++ against torch's headers, linked to
+    the libhxmi.so beside it."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    root = pathlib.Path(torch.__file__).parent
+    inc = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"], "/opt/rocm/include"]
+    tmp = OPS.with_suffix(".so.tmp")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-DUSE_ROCM=1", "-D__HIP_PLATFORM_AMD__=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(f"-I{p}" for p in inc),
+           str(CSRC / "torch_ops.cpp"), "-o", str(tmp), f"-L{root / 'lib'}", "-lc10", "-lc10_hip", "-ltorch_cpu",
+           "-ltorch_python", f"-L{LIB.parent}", "-lhxmi", "-Wl,-rpath,$ORIGIN"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"compile failed: {' '.join(cmd)}\n{proc.stdout}\n{proc.stderr}")
+    os.replace(tmp, OPS)
+
+
 def build(jobs: int | None = None, verbose: bool = True) -> pathlib.Path:
     BUILD.mkdir(parents=True, exist_ok=True)
     LIB.parent.mkdir(parents=True, exist_ok=True)
@@ -71,8 +94,9 @@ def build(jobs: int | None = None, verbose: bool = True) -> pathlib.Path:
     if proc.returncode != 0:
         raise RuntimeError(f"link failed: {' '.join(cmd)}\n{proc.stdout}\n{proc.stderr}")
     os.replace(tmp, LIB)
+    _build_ops()
     if verbose:
-        print(f"[hxmi] built {LIB}", flush=True)
+        print(f"[hxmi] built {LIB} and {OPS.name}", flush=True)
     return LIB
 
 

@@ -11,12 +11,15 @@ import collections
 import dataclasses
 import contextlib
 import ctypes
+import importlib.machinery
+import importlib.util
 import pathlib
 from typing import Optional
 
 import torch
 
 LIB_PATH = pathlib.Path(__file__).resolve().parent / "lib" / "libhxmi.so"
+OPS_PATH = LIB_PATH.with_name("hxmi_torch.so")  # native entry of the ops below (csrc/torch_ops.cpp)
 
 EPILOGUES = {
     None: 0,
@@ -95,6 +98,27 @@ def load_library() -> ctypes.CDLL:
             fn.restype = res
         _lib = lib
     return _lib
+
+
+class _NativeOps:
+    """Stands for the extension module until its first use loads it.  Each of
+    its functions returns the op's result for plain operands and None for
+    anything else, which the Python form below it then takes."""
+
+    def __getattr__(self, name):
+        global _ops
+        load_library()
+        if not OPS_PATH.exists():
+            raise HxmiNotBuiltError(f"{OPS_PATH} is missing; build it with hexagon-mlir_amd/build.py")
+        loader = importlib.machinery.ExtensionFileLoader("hxmi_torch", str(OPS_PATH))
+        mod = importlib.util.module_from_spec(importlib.util.spec_from_file_location("hxmi_torch", OPS_PATH,
+                                                                                     loader=loader))
+        loader.exec_module(mod)
+        _ops = mod
+        return getattr(mod, name)
+
+
+_ops = _NativeOps()
 
 
 def _check(rc: int) -> None:
@@ -274,6 +298,10 @@ def gemm(
     For epilogue "silu_mul", b holds packed gate/up columns (see pack_gate_up)
     and the result has N/2 columns.
     """
+    if epilogue in EPILOGUES and b_layout in ("nn", "nt"):
+        y = _ops.gemm(a, b, b_layout == "nt", EPILOGUES[epilogue], bias, alpha, out)
+        if y is not None:
+            return y
     _require_gpu(a, b, bias, out)
     if a.dtype not in (torch.float16, torch.bfloat16) or b.dtype != a.dtype:
         raise HxmiError(f"gemm takes fp16 or bf16 operands of one dtype, got {a.dtype} and {b.dtype}")
@@ -326,6 +354,10 @@ def bgemm(
     out: Optional[torch.Tensor] = None,
 ) -> torch.Tensor:
     """Batched C[i] = epilogue(alpha * a[i] @ op(b[i])) over 3-D strided tensors."""
+    if epilogue in EPILOGUES:
+        y = _ops.bgemm(a, b, b_layout == "nt", EPILOGUES[epilogue], bias, alpha, out)
+        if y is not None:
+            return y
     _require_gpu(a, b, bias, out)
     if a.dtype not in (torch.float16, torch.bfloat16) or b.dtype != a.dtype:
         raise HxmiError("bgemm takes fp16 or bf16 operands of one dtype")
@@ -371,6 +403,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
         epi = "silu_mul"
     else:
         raise HxmiError(f"unknown activation {epilogue!r}")
+    y = _ops.linear(x, w, bias, EPILOGUES[epi], out)
+    if y is not None:
+        return y
     lead = x.shape[:-1]
     x2 = x.reshape(-1, x.shape[-1])
     y = gemm(x2, w, b_layout="nt", epilogue=epi, bias=bias, out=out)
@@ -421,6 +456,10 @@ def rms_norm_linear(x: torch.Tensor, w_folded: torch.Tensor, eps: float = 1e-5, 
     rscale_out (fp32, one per row of x) also receives the row scales
     rsqrt(mean(x^2) + eps); a later call on the same x can pass them as
     rscale_in and skip the statistics (eps is then ignored)."""
+    if out is None and epilogue in (None, "silu_mul"):
+        y = _ops.rms_norm_linear(x, w_folded, eps, EPILOGUES[epilogue], rscale_out, rscale_in, bias)
+        if y is not None:
+            return y
     _require_gpu(x, w_folded, out, rscale_out, rscale_in, bias)
     if rscale_out is not None and rscale_in is not None:
         raise HxmiError("rscale_out and rscale_in are exclusive")
@@ -457,6 +496,9 @@ def rms_norm_linear(x: torch.Tensor, w_folded: torch.Tensor, eps: float = 1e-5, 
 def gemv(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
          out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Decode linear y[M,N] = x[M,K] @ w[N,K].T (+ bias); HBM-streaming for M <= 16.  fp16 or bf16."""
+    y = _ops.gemv(x, w, bias, out)
+    if y is not None:
+        return y
     _require_gpu(x, w, bias, out)
     if x.dtype not in (torch.float16, torch.bfloat16) or w.dtype != x.dtype:
         raise HxmiError("gemv takes fp16 or bf16 x and w of one dtype")
@@ -480,6 +522,9 @@ def gemv(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
 def w8a16_linear(x: torch.Tensor, wq: torch.Tensor, scale: torch.Tensor, bias: Optional[torch.Tensor] = None,
                  out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Weight-only int8 linear: y = (x @ wq.T) * scale (+ bias); wq int8 [N,K], scale fp16 [N]."""
+    y = _ops.w8a16_linear(x, wq, scale, bias, out)
+    if y is not None:
+        return y
     _require_gpu(x, wq, scale, bias, out)
     if x.dtype != torch.float16 or wq.dtype != torch.int8:
         raise HxmiError("w8a16_linear takes fp16 x and int8 wq")
@@ -503,6 +548,9 @@ def w8a16_linear(x: torch.Tensor, wq: torch.Tensor, scale: torch.Tensor, bias: O
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5,
              out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """RMSNorm over the last dim: weight * T(x * rsqrt(mean(x^2) + eps))."""
+    y = _ops.rms_norm(x, weight, eps, out)
+    if y is not None:
+        return y
     _require_gpu(x, weight, out)
     if x.dtype not in (torch.float16, torch.bfloat16) or weight.dtype != x.dtype:
         raise HxmiError("rms_norm takes fp16 or bf16 x and weight of the same dtype")
@@ -522,6 +570,9 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5,
 
 def softmax(x: torch.Tensor, scale: float = 1.0, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """softmax(scale * x) over the last dim, fp32 math."""
+    y = _ops.softmax(x, scale, out)
+    if y is not None:
+        return y
     _require_gpu(x, out)
     if x.dtype not in (torch.float16, torch.bfloat16):
         raise HxmiError("softmax takes fp16 or bf16 input")
@@ -595,6 +646,10 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional
     query + S_kv - S.  fp16 and bf16 with D a multiple of 8 up to 128 and scale > 0 run the fused kernel
     (hxmi_attention_ex); every other case (other head dims, v of another width) runs the reference's three
     steps as bmm(Q, K^T) -> softmax (with the mask and causal rule: hxmi_softmax_masked_*) -> bmm(P, V)."""
+    if out is None and mask is None:
+        y = _ops.attention(q, k, v, scale, causal)
+        if y is not None:
+            return y
     if scale is None:
         scale = q.shape[-1] ** -0.5
     S, D = q.shape[-2:]
