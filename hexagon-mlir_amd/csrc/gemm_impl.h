@@ -56,6 +56,7 @@ struct KArgs {
 };
 
 
+// 32x32x16 (16 accumulators a lane) and 16x16x32 (4) MFMAs.
 template <typename T>
 struct Mfma;
 template <>
@@ -64,11 +65,19 @@ struct Mfma<_Float16> {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8v, a),
                                                   __builtin_bit_cast(half8v, b), c, 0, 0, 0);
   }
+  static __device__ __forceinline__ float4v run(short8v a, short8v b, float4v c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8v, a),
+                                                  __builtin_bit_cast(half8v, b), c, 0, 0, 0);
+  }
 };
 template <>
 struct Mfma<__bf16> {
   static __device__ __forceinline__ float16v run(short8v a, short8v b, float16v c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8v, a),
+                                                   __builtin_bit_cast(bf16x8v, b), c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ float4v run(short8v a, short8v b, float4v c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8v, a),
                                                    __builtin_bit_cast(bf16x8v, b), c, 0, 0, 0);
   }
 };
@@ -114,19 +123,22 @@ __device__ __forceinline__ short8v read_kc(const char* tile, int r_off, int s, i
   return *(const short8v*)(tile + r * RB + ((c ^ kc_swz<RB>(r)) << 4));
 }
 
-template <int BN>
+template <int BN, int MI = 32>
 __device__ __forceinline__ int nn_swz(int k) {
+  // 16-wide fragments: two lane groups of a read phase share their columns
+  // and lie 8 rows apart, so bit 3 of the row moves them 32 bytes apart
+  if (MI == 16) return ((k & 3) << 2) | ((k >> 2) & 2);
   return (BN / 8 >= 16) ? ((k & 3) << 2) : ((k & 3) << 1);
 }
 
 // Fragment of an n-contiguous [64][BN] tile (B in NN form) for the same MFMA
 // operand layout, built from two transposing LDS reads.
-template <int BN>
+template <int BN, int MI = 32>
 __device__ __forceinline__ short8v read_nn(const char* tile, int n_off, int s, int lane) {
   const int g = lane >> 4, li = lane & 15;
-  const int n = n_off + ((g & 1) << 4) + ((li & 3) << 2);
-  const int k = (s << 4) + ((g >> 1) << 3) + (li >> 2);
-  const int sw = nn_swz<BN>(k);  // same for k and k+4
+  const int n = n_off + (MI == 32 ? ((g & 1) << 4) : 0) + ((li & 3) << 2);
+  const int k = (MI == 32 ? (s << 4) + ((g >> 1) << 3) : (s << 5) + (g << 3)) + (li >> 2);
+  const int sw = nn_swz<BN, MI>(k);  // same for k and k+4
   const int col = ((((n >> 3) ^ sw)) << 4) + ((n & 7) << 1);
   short4v lo = lds_read_tr16(tile + k * (BN * 2) + col);
   short4v hi = lds_read_tr16(tile + (k + 4) * (BN * 2) + col);
@@ -257,6 +269,30 @@ __device__ __forceinline__ void schedule_substep() {
   });
 }
 
+// The same for 16x16x32 MFMAs, of which a substep has many: its NB + NA
+// fragments (NBR reads per B fragment) and, in turn with them, NVM global->LDS
+// loads over the first SPAN MFMAs.  (4096^3 NT on the 8-wave 256x256 tile:
+// loads behind the reads at the substep's end 108.3 us, in turn 100.8.)
+template <int NMF, int NB, int NA, int NBR, int NVM, int NVA>
+__device__ __forceinline__ void schedule_pieces() {
+  constexpr int kVALU = 0x002, kMFMA = 0x008, kVMEMR = 0x020, kDSR = 0x100;
+  constexpr int NP = NB + NA, SPAN = NMF - NMF / 8, HALF = NMF - NMF / 2;
+  static_for<NMF>([&](auto M) {
+    constexpr int m = decltype(M)::value;
+    __builtin_amdgcn_sched_group_barrier(kMFMA, 1, 0);
+    constexpr int p0 = m < SPAN ? m * NP / SPAN : NP, p1 = m < SPAN ? (m + 1) * NP / SPAN : NP;
+    static_for<p1 - p0>([&](auto Q) {
+      constexpr int p = p0 + decltype(Q)::value;
+      constexpr int nr = p < NB ? NBR : 1, nv = (p + 1) * NVM / NP - p * NVM / NP;
+      if constexpr (nr > 0) __builtin_amdgcn_sched_group_barrier(kDSR, nr, 0);
+      if constexpr (nv > 0) __builtin_amdgcn_sched_group_barrier(kVMEMR, nv, 0);
+    });
+    constexpr int ma = m - (NMF - HALF);
+    constexpr int na = (NVA > 0 && ma >= 0) ? (ma + 1) * NVA / HALF - ma * NVA / HALF : 0;
+    if constexpr (na > 0) __builtin_amdgcn_sched_group_barrier(kVALU, na, 0);
+  });
+}
+
 // Barrier of the ping-pong schedule: nothing is moved across it, and every
 // LDS read of the wave has returned (so no stage is refilled under a reader).
 __device__ __forceinline__ void pp_barrier() {
@@ -289,10 +325,13 @@ __device__ __forceinline__ void pp_barrier() {
 // elements and shifted, which leaves zeros past K.
 template <int BM, int BN, int WM, int WN, int BK, int STAGES, bool NN, typename T, int EPI, bool OUTF32,
           bool BI8 = false, bool PP = false, bool RMS = false, bool RAGGED = false, int SB = 0, int FD = 1,
-          bool UNAL = false>
+          bool UNAL = false, int MI = 32>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a) {
   constexpr int NWM = BM / WM, NWN = BN / WN, NW = NWM * NWN, NT = NW * 64;
-  constexpr int TM = WM / 32, TN = WN / 32;
+  constexpr int TM = WM / MI, TN = WN / MI;
+  constexpr int KS = 512 / MI;          // k per MFMA: one substep
+  constexpr int G = MI / 8 == 4 ? 4 : 1;  // groups of four consecutive columns a lane holds of a fragment
+  using Acc = std::conditional_t<MI == 32, float16v, float4v>;
   constexpr int RB = BK * 2;            // bytes per k-contiguous tile row
   constexpr int CH = RB / 16;           // 16-byte chunks per row
   constexpr int RPIK = 1024 / RB;       // k-contiguous rows per 1 KB wave instruction
@@ -324,6 +363,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
   static_assert(!PP || (NW == 8 && NWM == 2 && STAGES >= 3 && !BI8), "ping-pong: 2 x 4 waves, >= 3 stages");
   static_assert(!RMS || (!NN && !BI8 && !PP && !OUTF32), "RMSNorm prologue: NT, standard schedule");
   static_assert(!RAGGED || (!BI8 && !PP && !RMS), "ragged K: plain fp16 / bf16 operands, standard schedule");
+  static_assert(MI == 32 || (MI == 16 && BK == 64 && !PP && !RAGGED && !UNAL && BN >= 128), "16x16x32 MFMAs");
   static_assert(!UNAL || (!BI8 && !PP && !RAGGED && STAGES == 2 && SBS == 2), "unaligned rows: two LDS stages");
   __shared__ __attribute__((aligned(1024))) char smem[SMEM];
   auto sa = [&](int i) { return smem + i * A_BYTES; };              // A stage i
@@ -396,12 +436,12 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
   // instruction start on multiples of 16).
   constexpr int IB = BI8 ? BN / 16 / NW : (NN ? (BK / RPI / NW) : (BN / RPIK / NW));
   static_assert(IB >= 1, "B load plan");
-  static_assert(!NN || (NW * RPI) % 4 == 0, "NN swizzle period");
+  static_assert(!NN || (NW * RPI) % (MI == 16 ? 16 : 4) == 0, "NN swizzle period");
   uint32_t voffB, stepB, bytesB;
   int cB8 = 0;
   if constexpr (NN) {
-    const int rowl = w * RPI + lane / CPR;  // (row & 3) is the same for every instruction
-    const int c = (lane % CPR) ^ nn_swz<BN>(rowl);
+    const int rowl = w * RPI + lane / CPR;  // (row & 3, and & 15, are the same for every instruction)
+    const int c = (lane % CPR) ^ nn_swz<BN, MI>(rowl);
     voffB = (n0 + c * 8) < a.N ? (uint32_t)(rowl * a.ldb * 2 + c * 16) : kOOB;
     stepB = (uint32_t)(NW * RPI * a.ldb * 2);
     bytesB = (uint32_t)(a.ldb * 2);  // per valid k-row
@@ -419,48 +459,52 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
 
   // Loads of K-step kt into A / B stage `stage`; a step past the end issues
   // loads against an empty buffer (all zeros, nothing touched).
-  auto issueA = [&](int kt, int stage) {
+  // (LO .. HI of the wave's loads of one operand, all of them by default)
+  auto issueA = [&](int kt, int stage, auto LO, auto HI) {
     const int k0 = kt * BK;
     const bool live = kt < nk;
     char* sA_ = sa(stage);
     const __amdgpu_buffer_rsrc_t rA = make_rsrc(Ab + (int64_t)k0 * 2, live ? bytesA - 2u * k0 : 0u);
     const uint32_t vA = (k0 + cA * 8) < K ? voffA : kOOB;
 #pragma unroll
-    for (int i = 0; i < IA; ++i)
+    for (int i = decltype(LO)::value; i < decltype(HI)::value; ++i)
       load_lds16(rA, (HXMI_LDS void*)to_lds(sA_ + (i * NW + w) * 1024), vA + i * stepA);
   };
-  auto issueB = [&](int kt, int stage) {
+  auto issueB = [&](int kt, int stage, auto LO, auto HI) {
     const int k0 = kt * BK;
     const bool live = kt < nk;
     char* sB_ = sb(stage);
+    const char* base;
+    uint32_t bytes, vB;
     if constexpr (NN) {
-      const uint32_t rows = (uint32_t)min(BK, K - k0);
-      const __amdgpu_buffer_rsrc_t rB = make_rsrc(Bb + (int64_t)k0 * a.ldb * 2, live ? rows * bytesB : 0u);
-#pragma unroll
-      for (int i = 0; i < IB; ++i)
-        load_lds16(rB, (HXMI_LDS void*)to_lds(sB_ + (i * NW + w) * 1024), voffB + i * stepB);
+      base = Bb + (int64_t)k0 * a.ldb * 2;
+      bytes = (uint32_t)min(BK, K - k0) * bytesB;
+      vB = voffB;
     } else if constexpr (BI8) {
-      const __amdgpu_buffer_rsrc_t rB = make_rsrc(Bb + k0, live ? bytesB - (uint32_t)k0 : 0u);
-      const uint32_t vB = (k0 + cB8 * 16) < K ? voffB : kOOB;
-#pragma unroll
-      for (int i = 0; i < IB; ++i)
-        load_lds16(rB, (HXMI_LDS void*)to_lds(sB_ + (i * NW + w) * 1024), vB + i * stepB);
+      base = Bb + k0;
+      bytes = bytesB - (uint32_t)k0;
+      vB = (k0 + cB8 * 16) < K ? voffB : kOOB;
     } else {
-      const __amdgpu_buffer_rsrc_t rB = make_rsrc(Bb + (int64_t)k0 * 2, live ? bytesB - 2u * k0 : 0u);
-      const uint32_t vB = (k0 + cA * 8) < K ? voffB : kOOB;
-#pragma unroll
-      for (int i = 0; i < IB; ++i)
-        load_lds16(rB, (HXMI_LDS void*)to_lds(sB_ + (i * NW + w) * 1024), vB + i * stepB);
+      base = Bb + (int64_t)k0 * 2;
+      bytes = bytesB - 2u * k0;
+      vB = (k0 + cA * 8) < K ? voffB : kOOB;
     }
+    const __amdgpu_buffer_rsrc_t rB = make_rsrc(base, live ? bytes : 0u);
+#pragma unroll
+    for (int i = decltype(LO)::value; i < decltype(HI)::value; ++i)
+      load_lds16(rB, (HXMI_LDS void*)to_lds(sB_ + (i * NW + w) * 1024), vB + i * stepB);
   };
+  constexpr std::integral_constant<int, 0> kFirst{};
+  constexpr std::integral_constant<int, IA> kAllA{};
+  constexpr std::integral_constant<int, IB> kAllB{};
   auto issue = [&](int kt, int stage) {
-    issueA(kt, stage);
-    issueB(kt, stage);
+    issueA(kt, stage, kFirst, kAllA);
+    issueB(kt, stage, kFirst, kAllB);
   };
 
   // Byte offset of this lane's 16-byte chunk in a k-contiguous fragment of
   // substep s: the swizzle repeats every 16 rows and fragments start on
-  // multiples of 32 rows, so it depends on the lane alone; the wave's first
+  // multiples of MI rows, so it depends on the lane alone; the wave's first
   // row is folded in, leaving a constant per fragment (an immediate offset).
   //
   // Int8 B (BI8) is read 16 bytes (16 k) at a time, one chunk per pair of
@@ -471,35 +515,39 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
   // substeps still cover k = 0..63 once.  The 16-byte read matters: after an
   // 8-byte LDS read (the plain int8 fragment) the compiler waited for every
   // outstanding direct-to-LDS load (vmcnt(0)), which drained the prefetch in
-  // every K-step.
-  constexpr int SUBS_ = BK / 16;
+  // every K-step.  (16x16x32: lane group g = l / 16 takes k = 16g + 8s .. +7
+  // in substep s, chunk 2g + s of its A row.)
+  constexpr int SUBS_ = BK / KS;
   uint32_t lofA[SUBS_], lofB[SUBS_], lofB8[SUBS_];
 #pragma unroll
   for (int s = 0; s < SUBS_; ++s) {
-    const int l = lane & 31, h = lane >> 5;
-    const int ca = BI8 ? ((s >> 1) << 2) + (h << 1) + (s & 1) : (s << 1) + h;
+    const int l = lane & (MI - 1), h = lane / MI;
+    const int cb = MI == 32 ? (s << 1) + h : (s << 2) + h;
+    const int ca = !BI8 ? cb : MI == 32 ? ((s >> 1) << 2) + (h << 1) + (s & 1) : (h << 1) + s;
     lofA[s] = (uint32_t)(wm * WM * RB + l * RB + ((ca ^ kc_swz<RB>(l)) << 4));
-    lofB[s] = (uint32_t)(wn * WN * RB + l * RB + ((((s << 1) + h) ^ kc_swz<RB>(l)) << 4));
+    lofB[s] = (uint32_t)(wn * WN * RB + l * RB + ((cb ^ kc_swz<RB>(l)) << 4));
     // int8 B rows (BK bytes) keep chunk c of row r at c ^ ((r >> 2) & 3)
-    lofB8[s] = (uint32_t)((wn * WN + l) * BK + (((2 * (s >> 1) + h) ^ ((l >> 2) & 3)) << 4));
+    lofB8[s] = (uint32_t)((wn * WN + l) * BK + (((MI == 32 ? 2 * (s >> 1) + h : h) ^ ((l >> 2) & 3)) << 4));
   }
   short8v fbo[BI8 ? TN : 1];  // BI8: the odd substep's B fragments, dequantised with the even one's
   // RAGGED (K % 8 != 0): the 16-byte chunk that straddles K brings in
   // elements past K (row padding, or the next row).  In the last K-step the
   // fragments keep only their elements below K; the NN B operand needs no
   // mask, its rows past K read as zero.
-  auto read_frags = [&](short8v (&fa)[TM], short8v (&fb)[TN], const char* sA_, const char* sB_, int s,
-                        int kstep) {
-#pragma unroll
-    for (int i = 0; i < TN; ++i) {
+  // Piece P of a substep's fragments: B fragment P, then A fragment P - TN.
+  auto read_piece = [&](short8v (&fa)[TM], short8v (&fb)[TN], const char* sA_, const char* sB_, int s, int kstep,
+                        auto P) {
+    constexpr int p = decltype(P)::value;
+    if constexpr (p < TN) {
+      constexpr int i = p;
       if constexpr (NN) {
-        fb[i] = read_nn<BN>(sB_, wn * WN + i * 32, s, lane);
+        fb[i] = read_nn<BN, MI>(sB_, wn * WN + i * MI, s, lane);
       } else if constexpr (BI8) {
-        // 16 int8 weights of row wn WN + 32 i + lane % 32 -> 16 fp16,
+        // 16 int8 weights of row wn WN + MI i + lane % MI -> 16 fp16,
         // exactly, in the even substep: its fragment takes the first 8, the
         // odd substep's the last 8
         if ((s & 1) == 0) {
-          int4v q = __builtin_bit_cast(int4v, *(const short8v*)(sB_ + lofB8[s] + i * 32 * BK));
+          int4v q = __builtin_bit_cast(int4v, *(const short8v*)(sB_ + lofB8[s] + i * MI * BK));
           asm("" : "+v"(q));  // one 16-byte read, not two 8-byte ones
           fb[i] = dequant8(int2v{q[0], q[1]});
           fbo[i] = dequant8(int2v{q[2], q[3]});
@@ -507,30 +555,29 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
           fb[i] = fbo[i];
         }
       } else {
-        fb[i] = *(const short8v*)(sB_ + lofB[s] + i * 32 * RB);
+        fb[i] = *(const short8v*)(sB_ + lofB[s] + i * MI * RB);
       }
+    } else {
+      fa[p - TN] = *(const short8v*)(sA_ + lofA[s] + (p - TN) * MI * RB);
     }
-#pragma unroll
-    for (int j = 0; j < TM; ++j) fa[j] = *(const short8v*)(sA_ + lofA[s] + j * 32 * RB);
     if constexpr (RAGGED) {
       if (kstep == nk - 1) {
         const int nv = K - (kstep * BK + s * 16 + (lane >> 5) * 8);
-#pragma unroll
-        for (int j = 0; j < TM; ++j) fa[j] = keep_first(fa[j], nv);
-        if constexpr (!NN) {
-#pragma unroll
-          for (int i = 0; i < TN; ++i) fb[i] = keep_first(fb[i], nv);
-        }
+        if constexpr (p >= TN) fa[p - TN] = keep_first(fa[p - TN], nv);
+        else if constexpr (!NN) fb[p] = keep_first(fb[p], nv);
       }
     }
   };
+  auto read_frags = [&](short8v (&fa)[TM], short8v (&fb)[TN], const char* sA_, const char* sB_, int s, int kstep) {
+    static_for<TN + TM>([&](auto P) { read_piece(fa, fb, sA_, sB_, s, kstep, P); });
+  };
 
-  float16v acc[TN][TM];
+  Acc acc[TN][TM];
 #pragma unroll
   for (int i = 0; i < TN; ++i)
 #pragma unroll
-    for (int j = 0; j < TM; ++j) acc[i][j] = float16v{};
-  float ss[TM];  // RMS: this lane's sum of squares of row (j*32 + lane%32), its k half
+    for (int j = 0; j < TM; ++j) acc[i][j] = Acc{};
+  float ss[TM];  // RMS: this lane's sum of squares of row (j*MI + lane%MI), its k share
 #pragma unroll
   for (int j = 0; j < TM; ++j) ss[j] = 0.f;
 
@@ -542,7 +589,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
   //   kt), refill step kt's stage with step kt+STAGES;
   //   last substep: MFMAs, with step kt+1's first fragments and the new
   //   step's global loads in between.
-  constexpr int SUBS = BK / 16;
+  constexpr int SUBS = BK / KS;
   constexpr int NDS = (NN ? 2 * TN : TN) + TM;  // LDS read instructions per substep
   constexpr int NVM = IA + IB;                  // global->LDS loads per K-step per wave
   if constexpr (PP) {
@@ -668,8 +715,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
   constexpr int WB = SBS > STAGES ? IB : 0;
 #pragma unroll
   for (int t = -SBS; t < 0; ++t) {
-    if (t + STAGES >= 0) issueA(t + STAGES, t + STAGES);
-    issueB(t + SBS, t + SBS);
+    if (t + STAGES >= 0) issueA(t + STAGES, t + STAGES, kFirst, kAllA);
+    issueB(t + SBS, t + SBS, kFirst, kAllB);
   }
   wait_vmcnt<(STAGES - 1) * NVM + WB>();
   barrier_after_lds_loads();  // (__syncthreads() would wait for every stage)
@@ -699,16 +746,30 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
       constexpr int cur = s % NFB, nxt = t % NFB;
       if constexpr (t < SUBS) {
         read_frags(fa[nxt], fb[nxt], sA_, sB_, t, kt);
-      } else if constexpr (t == SUBS) {
-        wait_vmcnt<(STAGES - 2) * NVM + WB>();
-        barrier_before_refill();
+      } else {
+        if constexpr (t == SUBS) {
+          wait_vmcnt<(STAGES - 2) * NVM + WB>();
+          barrier_before_refill();
+        }
         // fragment reads first, then the refill loads: the same order as the
         // schedule below, so the loads can be spread between the MFMAs
-        read_frags(fa[nxt], fb[nxt], sa(st1), sb(stb1), 0, kt + 1);
-        issueA(kt + STAGES, st);
-        issueB(kt + SBS, stb);
-      } else {
-        read_frags(fa[nxt], fb[nxt], sa(st1), sb(stb1), t - SUBS, kt + 1);
+        if constexpr (MI == 32 || t > SUBS) {
+          read_frags(fa[nxt], fb[nxt], sa(st1), sb(stb1), t - SUBS, kt + 1);
+          if constexpr (t == SUBS) {
+            issueA(kt + STAGES, st, kFirst, kAllA);
+            issueB(kt + SBS, stb, kFirst, kAllB);
+          }
+        } else {  // reads and loads in turn
+          static_for<TN + TM>([&](auto P) {
+            constexpr int p = decltype(P)::value, NP = TN + TM;
+            read_piece(fa[nxt], fb[nxt], sa(st1), sb(stb1), t - SUBS, kt + 1, P);
+            constexpr int lo = p * NVM / NP, hi = (p + 1) * NVM / NP;
+            issueA(kt + STAGES, st, std::integral_constant<int, (lo < IA ? lo : IA)>{},
+                   std::integral_constant<int, (hi < IA ? hi : IA)>{});
+            issueB(kt + SBS, stb, std::integral_constant<int, (lo > IA ? lo - IA : 0)>{},
+                   std::integral_constant<int, (hi > IA ? hi - IA : 0)>{});
+          });
+        }
       }
 #pragma unroll
       for (int i = 0; i < TN; ++i)
@@ -718,7 +779,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
 #pragma unroll
         for (int j = 0; j < TM; ++j) ss[j] = sumsq8<T>(fa[cur][j], ss[j]);
       }
-      schedule_substep<TN * TM, NDS, (t == SUBS) ? NVM : 0, RMS ? TM * 4 : 0>();
+      if constexpr (MI == 32) schedule_substep<TN * TM, NDS, (t == SUBS) ? NVM : 0, RMS ? TM * 4 : 0>();
+      else schedule_pieces<TN * TM, TN, TM, NN ? 2 : (BI8 && t % 2 ? 0 : 1), (t == SUBS) ? NVM : 0, RMS ? TM * 4 : 0>();
       __builtin_amdgcn_sched_barrier(0);
     });
     st = st1;
@@ -729,17 +791,19 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
   __syncthreads();
 
   if constexpr (RMS) {
-    // lanes l and l+32 hold the two k halves of the same row
+    // lanes a multiple of MI apart hold the k shares of the same row
 #pragma unroll
     for (int j = 0; j < TM; ++j) {
-      const float tot = ss[j] + __shfl_xor(ss[j], 32, 64);
+      float tot = ss[j];
+      if constexpr (MI == 16) tot += __shfl_xor(tot, 16, 64);
+      tot += __shfl_xor(tot, 32, 64);
       const float r = rsqrtf(tot / (float)a.K + a.rms_eps);
 #pragma unroll
       for (int i = 0; i < TN; ++i) acc[i][j] *= r;
       // the first column of tiles publishes the row scales for other
       // consumers of the same normalised rows
-      const int m = m0 + wm * WM + j * 32 + lane;
-      if (a.rs_out && tn == 0 && wn == 0 && lane < 32 && m < a.M) a.rs_out[m] = r;
+      const int m = m0 + wm * WM + j * MI + lane;
+      if (a.rs_out && tn == 0 && wn == 0 && lane < MI && m < a.M) a.rs_out[m] = r;
     }
   }
 
@@ -760,9 +824,9 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
 #pragma unroll
         for (int j = 0; j < TM; ++j)
 #pragma unroll
-          for (int g = 0; g < 4; ++g) {
+          for (int g = 0; g < G; ++g) {
             const float4v v = {acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
-            const uint32_t off = (uint32_t)(b * TILE_B + (((i * TM + j) * 4 + g) * NT + threadIdx.x) * 16);
+            const uint32_t off = (uint32_t)(b * TILE_B + (((i * TM + j) * G + g) * NT + threadIdx.x) * 16);
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(int4v, v), rP, off, 0, kCoherent);
           }
       wait_vmcnt0();
@@ -784,7 +848,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
       if (!is_last) return;
       // GS slices' loads in flight at once (the small tiles, whose partial
       // fragments fit in spare registers), then added in slice order
-      constexpr int GS = TN * TM == 1 ? 4 : (TN * TM == 2 ? 2 : 1);
+      constexpr int GS = TN * TM * G == 4 ? 4 : (TN * TM * G == 8 ? 2 : 1);
       if constexpr (GS == 1) {
         for (int sl = 0; sl < a.batch; ++sl) {
 #pragma unroll
@@ -792,8 +856,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
 #pragma unroll
             for (int j = 0; j < TM; ++j)
 #pragma unroll
-              for (int g = 0; g < 4; ++g) {
-                const uint32_t off = (uint32_t)(sl * TILE_B + (((i * TM + j) * 4 + g) * NT + threadIdx.x) * 16);
+              for (int g = 0; g < G; ++g) {
+                const uint32_t off = (uint32_t)(sl * TILE_B + (((i * TM + j) * G + g) * NT + threadIdx.x) * 16);
                 const float4v v =
                     __builtin_bit_cast(float4v, __builtin_amdgcn_raw_buffer_load_b128(rP, off, 0, kCoherent));
 #pragma unroll
@@ -801,7 +865,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
               }
         }
       } else for (int sl0 = 0; sl0 < a.batch; sl0 += GS) {
-        float4v part[GS][TN][TM][4];
+        float4v part[GS][TN][TM][G];
 #pragma unroll
         for (int u = 0; u < GS; ++u)
 #pragma unroll
@@ -809,9 +873,9 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
 #pragma unroll
             for (int j = 0; j < TM; ++j)
 #pragma unroll
-              for (int g = 0; g < 4; ++g) {
+              for (int g = 0; g < G; ++g) {
                 const int sl = sl0 + u;
-                const uint32_t off = (uint32_t)(sl * TILE_B + (((i * TM + j) * 4 + g) * NT + threadIdx.x) * 16);
+                const uint32_t off = (uint32_t)(sl * TILE_B + (((i * TM + j) * G + g) * NT + threadIdx.x) * 16);
                 part[u][i][j][g] = __builtin_bit_cast(
                     float4v, __builtin_amdgcn_raw_buffer_load_b128(rP, sl < a.batch ? off : kOOB, 0, kCoherent));
               }
@@ -823,7 +887,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
 #pragma unroll
             for (int j = 0; j < TM; ++j)
 #pragma unroll
-              for (int g = 0; g < 4; ++g)
+              for (int g = 0; g < G; ++g)
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
                   acc[i][j][4 * g + q] = sl0 + u == 0 ? part[u][i][j][g][q] : acc[i][j][4 * g + q] + part[u][i][j][g][q];
@@ -838,7 +902,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
       // norm weight)
 #pragma unroll
       for (int j = 0; j < TM; ++j) {
-        const int m = m0 + wm * WM + j * 32 + (lane & 31);
+        const int m = m0 + wm * WM + j * MI + (lane & (MI - 1));
         const float r = m < a.M ? a.rs_in[m] : 0.f;
 #pragma unroll
         for (int i = 0; i < TN; ++i) acc[i][j] *= r;
@@ -848,17 +912,17 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
 
   // ---- epilogue -------------------------------------------------------------
   const float alpha = a.alpha;
-  const int hi = lane >> 5;
+  const int hi = lane / MI;  // this lane's columns of a fragment start at 4 hi (+ 8 g)
   if constexpr (OUTF32) {
     char* Cb = a.C + (b * a.sC) * 4;
 #pragma unroll
     for (int i = 0; i < TN; ++i)
 #pragma unroll
       for (int j = 0; j < TM; ++j) {
-        const int m = m0 + wm * WM + j * 32 + (lane & 31);
+        const int m = m0 + wm * WM + j * MI + (lane & (MI - 1));
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int n = n0 + wn * WN + i * 32 + 8 * g + 4 * hi;
+        for (int g = 0; g < G; ++g) {
+          const int n = n0 + wn * WN + i * MI + 8 * g + 4 * hi;
           float v[4];
 #pragma unroll
           for (int q = 0; q < 4; ++q) v[q] = acc[i][j][4 * g + q] * alpha;
@@ -894,26 +958,30 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
     for (int i = 0; i < TN; ++i)
 #pragma unroll
       for (int j = 0; j < TM; ++j) {
-        const int ml = wm * WM + j * 32 + (lane & 31);
+        const int ml = wm * WM + j * MI + (lane & (MI - 1));
         if constexpr (EPI == EPI_SILU_MUL) {
           // packed columns [32q, 32q+16) are gate, [32q+16, 32q+32) are up
-          // for output columns [16q, 16q+16)
+          // for output columns [16q, 16q+16): the two halves of a 32-wide
+          // fragment, or two 16-wide ones
+          if (MI == 16 && i % 2) continue;
 #pragma unroll
-          for (int g = 0; g < 2; ++g) {
+          for (int g = 0; g < (MI == 32 ? 2 : 1); ++g) {
             float v[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
               const float gate = acc[i][j][4 * g + q] * alpha;
-              const float up = acc[i][j][4 * (g + 2) + q] * alpha;
+              float up;
+              if constexpr (MI == 32) up = acc[i][j][4 * (g + 2) + q] * alpha;
+              else up = acc[(i + 1) % TN][j][q] * alpha;
               v[q] = silu(gate) * up;
             }
-            const int ol = (wn * WN + i * 32) / 2 + 8 * g + 4 * hi;
+            const int ol = (wn * WN + i * MI) / 2 + 8 * g + 4 * hi;
             store4<T>(smem + ml * SROW + ol * 2, v[0], v[1], v[2], v[3]);
           }
         } else {
 #pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            const int nl = wn * WN + i * 32 + 8 * g + 4 * hi;
+          for (int g = 0; g < G; ++g) {
+            const int nl = wn * WN + i * MI + 8 * g + 4 * hi;
             float v[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) v[q] = acc[i][j][4 * g + q] * alpha;
@@ -963,6 +1031,7 @@ struct TileShape {
   bool PP = false;
   int SB = 0;  // B stages (0: as many as A)
   int FD = 1;  // substeps between a fragment's LDS read and its MFMAs
+  int MI = 32;  // MFMA: 32x32x16 or 16x16x32
 };
 
 // The small tiles run three LDS stages: their K-steps are short (a 64x64x64
@@ -990,6 +1059,14 @@ struct TileShape {
 // tile: 29.4 and 18.1 us.  It takes k-contiguous B ([N, K]) only: an NN
 // B row of 192 columns (384 bytes) does not divide the 1 KB wave load, and
 // 192 rows do not split into the int8 B loads' 16-row groups over 8 waves.
+// The 8-wave tiles run 16x16x32 MFMAs.  MI355X is power-limited under MFMA
+// load, and per flop these move half the accumulator registers of 32x32x16
+// ones (and twice the operand registers): a loop of nothing else on random
+// operands runs 1975 against 1690 TFLOP/s in fp16, 2100 against 1850 in bf16,
+// and the same 2440 on zeros, where the clock holds.  4096^3 NT 113.6 ->
+// 100.8 us and NN 113.3 -> 102.1 on the 256x256 tile, gate/up 27.8 -> 25.2 us
+// on 128x192.  The 4-wave tiles of at most 128 rows are bound by latency
+// and keep 32x32x16, whose shorter substeps let them read further ahead.
 constexpr TileShape kTiles[TILE_COUNT] = {
     {256, 256, 128, 128, 64, 2},  // TILE_256x256
     {128, 256, 64, 128, 64, 3, false, 0, 3},   // TILE_128x256
@@ -999,13 +1076,13 @@ constexpr TileShape kTiles[TILE_COUNT] = {
     {128, 64, 64, 32, 64, 3, false, 0, 3},     // TILE_128x64
     {64, 64, 32, 32, 64, 3, false, 0, 3},      // TILE_64x64
     {256, 256, 128, 128, 32, 4},  // TILE_256x256_K32S4
-    {256, 256, 128, 64, 64, 2},   // TILE_256x256_W8
+    {256, 256, 128, 64, 64, 2, false, 0, 1, 16},   // TILE_256x256_W8
     {128, 128, 64, 64, 32, 4},    // TILE_128x128_K32S4
     {256, 128, 128, 64, 32, 4},   // TILE_256x128_K32S4
     {256, 256, 128, 64, 32, 3, true},  // TILE_256x256_PP
-    {256, 128, 64, 64, 64, 3},         // TILE_256x128_W8
-    {128, 128, 32, 64, 64, 2, false, 0, 3},    // TILE_128x128_W8
-    {128, 192, 32, 96, 64, 3, false, 0, 3},    // TILE_128x192_W8
+    {256, 128, 64, 64, 64, 3, false, 0, 1, 16},    // TILE_256x128_W8
+    {128, 128, 32, 64, 64, 2, false, 0, 1, 16},    // TILE_128x128_W8
+    {128, 192, 32, 96, 64, 3, false, 0, 1, 16},    // TILE_128x192_W8
     {64, 64, 32, 32, 64, 4, false, 0, 3},      // TILE_64x64_S4
 };
 
@@ -1018,11 +1095,13 @@ hipError_t launch_one(const KArgs& k, hipStream_t stream) {
   // int8 B: BK 64, two A stages (A is L2-resident) and up to six B stages
   // in the LDS that three stages of both took (same workgroups per CU): the
   // weights stream from HBM, so B is prefetched several K-steps ahead
+  // (an NN tile whose loads of one wave lie 8 rows apart keeps 32x32x16)
+  constexpr int MI = NN && threads / 64 * (512 / s.BN) % 16 ? 32 : s.MI;
   constexpr int W8_A = s.BM * 128, W8_B = s.BN * 64;
   constexpr int W8_SB = W8_A / W8_B + 3 > 6 ? 6 : W8_A / W8_B + 3;
   hipLaunchKernelGGL((gemm_mfma<s.BM, s.BN, s.WM, s.WN, (BI8 ? 64 : s.BK), (BI8 || UNAL ? 2 : s.STAGES), NN, T, EPI,
                                 OUTF32, BI8, (s.PP && !BI8 && !RMS), RMS, RAGGED, (BI8 ? W8_SB : s.SB),
-                                (BI8 || s.PP || UNAL ? 1 : s.FD), UNAL>),
+                                (BI8 || s.PP || UNAL ? 1 : s.FD), UNAL, MI>),
                      dim3((unsigned)blocks), dim3(threads), 0, stream, k);
   return hipGetLastError();
 }
