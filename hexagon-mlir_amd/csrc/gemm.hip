@@ -5,6 +5,8 @@
 // K not a multiple of 8 runs the instantiations that mask the last K-step,
 // and rows off the 16-byte grid (leading dimensions not a multiple of 8,
 // misaligned pointers) those that load their tiles through registers.
+#include <algorithm>
+
 #include "gemm_impl.h"
 
 namespace hxmi {
@@ -142,75 +144,40 @@ bool gemm_fast_path_ok(const GemmProblem& p) {
   return gemm::operands_aligned(p) && p.ldc % 8 == 0 && (p.batch <= 1 || p.sC % 8 == 0) && gemm::aligned(p.C, 16);
 }
 
-// Pick the tile that minimises an estimate of makespan: rounds of tiles over
-// the 256 CUs (with the tiles a CU holds at once) times a per-tile cost that
-// reflects each shape's MFMA efficiency.
-int gemm_pick_tile(const GemmProblem& p) {
+// The int8-weight GEMM's tile: the one that minimises an estimate of makespan,
+// rounds of tiles over the 256 CUs (with the tiles a CU holds at once) times a
+// per-tile cost that reflects each shape's MFMA efficiency.
+static int pick_tile_i8(const GemmProblem& p) {
   struct Cand {
     int id, bm, bn, per_cu;
     float eff;
   };
-  // (the 8-wave 128x128 tile at two per CU outruns one 256x128 per CU on the
-  // 512-token LLaMA MLP GEMMs; 64x64 at two per CU outruns 64x128 on the
-  // 512-token O projection; measured on the block shapes)
+  // int8 B converts every weight once per tile row: tall tiles amortise it,
+  // and the latency-bound small shapes want the most workgroups (measured on
+  // the Qwen2.5-0.5B int8 shapes at M = 256: 896 -> 4864 runs 152 tiles of
+  // 128x64 in 11.5 us against 13.4 us for 304 tiles of 64x64; the lm_head at
+  // M = 128 1187 tiles of 128x128 at two per CU in 56.0 us against 72.0 us for
+  // 594 tiles of 128x256)
   static const Cand cands[] = {
-      {TILE_256x256_W8, 256, 256, 1, 1.00f}, {TILE_256x128_W8, 256, 128, 1, 0.85f},
-      {TILE_128x256, 128, 256, 1, 0.80f},    {TILE_128x128_W8, 128, 128, 2, 0.90f},
-      {TILE_64x128, 64, 128, 3, 0.50f},      {TILE_128x64, 128, 64, 3, 0.50f},
-      {TILE_64x64, 64, 64, 4, 0.52f},        {TILE_128x192_W8, 128, 192, 1, 0.80f},
+      {TILE_256x256_W8, 256, 256, 1, 1.00f}, {TILE_256x128_W8, 256, 128, 1, 0.80f},
+      {TILE_128x256, 128, 256, 1, 0.65f},    {TILE_128x128_W8, 128, 128, 2, 0.80f},
+      {TILE_64x128, 64, 128, 3, 0.50f},      {TILE_128x64, 128, 64, 3, 0.62f},
+      {TILE_64x64, 64, 64, 4, 0.60f},
   };
   const int cus = 256;
   int best = TILE_64x64;
   double best_t = 1e300;
-  const bool i8 = p.dtype == DT_W8A16;
   for (const Cand& c : cands) {
-    if (c.bn == 64 && p.epilogue == EPI_SILU_MUL) continue;
-    // 128x192: k-contiguous fp16 / bf16 weights, one round of tiles (where
-    // it was measured: TinyLlama gate/up, ViT-B/16 fc1)
-    if (c.id == TILE_128x192_W8 && (p.dtype == DT_W8A16 || !p.b_nt ||
-                                    ((p.M + 127) / 128) * ((p.N + 191) / 192) * p.batch > cus))
-      continue;
-    // int8 B converts every weight once per tile row: tall tiles amortise
-    // it, and the latency-bound small shapes want the most workgroups
-    // (measured on the Qwen2.5-0.5B int8 shapes at M = 256)
-    float eff = c.eff;
-    // the three-stage 8-wave 256x128 tile pays once K is long enough to keep
-    // its deeper prefetch busy (TinyLlama gate/up, K = 2048: 33.1 -> 30.7 us
-    // against 128x128 at two per CU; ViT fc1, K = 768: 19.4 -> 20.6 us)
-    if (!i8 && c.id == TILE_256x128_W8 && p.K >= 1536) eff = 0.95f;
-    if (i8 && (c.id == TILE_128x128_W8 || c.id == TILE_256x128_W8)) eff = 0.80f;
-    if (i8 && c.id == TILE_64x64) eff = 0.60f;
-    // (the int8 896 -> 4864 projection at M = 256: 152 tiles of 128x64 run
-    // 11.5 us against 13.4 us for 304 tiles of 64x64)
-    if (i8 && c.id == TILE_128x64) eff = 0.62f;
-    // (the int8 lm_head 896 -> 151936 at M = 128: 1187 tiles of 128x128 at
-    // two per CU run 56.0 us against 72.0 us for 594 tiles of 128x256)
-    if (i8 && c.id == TILE_128x256) eff = 0.65f;
-    // an RMSNorm-folded GEMM sums the squares of its A rows in every tile of
-    // a row, so narrow tiles repeat that work more often (the 512-token QKV
-    // projection, 512x2560x2048, in the block sequence: 64x128 1.3 us faster
-    // than 64x64 once the K-step barriers kept the prefetch in flight)
-    if (p.rms && c.id == TILE_64x64) eff = 0.45f;
-    // long K with few tiles: 128x64 (4 waves, three per CU) over 64x64 and
-    // 64x128 (ViT-B/16 fc2, 1576x768x3072: 156 tiles)
-    if (!i8 && p.K >= 3072 && c.id == TILE_128x64) eff = 0.56f;
-    const int64_t tm = (p.M + c.bm - 1) / c.bm, tn = (p.N + c.bn - 1) / c.bn;
-    const int64_t tiles = tm * tn * p.batch;
+    const int64_t tiles = ((p.M + c.bm - 1) / c.bm) * ((p.N + c.bn - 1) / c.bn) * p.batch;
     const int64_t slots = (int64_t)cus * c.per_cu;
     const int64_t rounds = (tiles + slots - 1) / slots;
     const int64_t conc = tiles < slots ? (tiles + cus - 1) / cus : c.per_cu;  // tiles sharing a CU
-    const double t = (double)rounds * c.bm * c.bn * (double)(conc > 0 ? conc : 1) / eff;
+    const double t = (double)rounds * c.bm * c.bn * (double)(conc > 0 ? conc : 1) / c.eff;
     if (t < best_t * 0.999) {
       best_t = t;
       best = c.id;
     }
   }
-  // 64x64 tiles over K >= 2048: a fourth LDS stage (two workgroups still fit
-  // a CU).  The 512-token O projection in the TinyLlama block sequence,
-  // weights from HBM: block 75.46-75.90 -> 74.75-75.04 us (72.8-73.3 against
-  // 74.3-74.6 on another MI355X); the 1024^3 GEMM, its operands in L2, ran
-  // 6.42 -> 6.53 us with it and keeps three stages
-  if (best == TILE_64x64 && !i8 && p.K >= 2048) best = TILE_64x64_S4;
   return best;
 }
 
@@ -223,12 +190,11 @@ int tile_of_two(const GemmProblem& p) {
   return t128 >= 256 ? TILE_128x128 : TILE_64x64;
 }
 
-int tile_for(const GemmProblem& p) {
-  if (p.K % 8) return tile_of_two(p);
+// The tile an override asks for (p.tile, then the knob), or -1: none, or one
+// that does not take p's layout.
+int forced_tile(const GemmProblem& p) {
   int tile = p.tile >= 0 ? p.tile : knob_or(KNOB_GEMM_TILE, -1);
-  // (an override of 128x192 for a layout it does not take: the picker's tile)
-  if (tile < 0 || tile >= TILE_COUNT || (tile == TILE_128x192_W8 && (!p.b_nt || p.dtype == DT_W8A16)))
-    tile = gemm_pick_tile(p);
+  if (tile < 0 || tile >= TILE_COUNT || (tile == TILE_128x192_W8 && (!p.b_nt || p.dtype == DT_W8A16))) return -1;
   if (p.epilogue == EPI_SILU_MUL && kTiles[tile].BN < 128) tile = TILE_64x128;
   return tile;
 }
@@ -275,26 +241,15 @@ hipError_t launch_fast(const GemmProblem& p, int tile, const KArgs& k, hipStream
 }  // namespace
 }  // namespace gemm
 
-// Split K into slices when the output has too few tiles to occupy the 256
-// CUs and K is long enough that each slice still runs many K-steps.  Split
-// problems run 64x128 tiles (4 waves, two per CU at three LDS stages).
-// Slices of >= 2048 of K that already give every CU a workgroup stop at
-// two; otherwise the slice count aims at ~480 workgroups, each slice keeping
-// >= 1024 of K.  With K below 4096 every split measured slower: the
-// 512-token QKV and O projections, and ViT-B/16 fc2 (1576x768x3072) once
-// the K-step barriers kept the prefetch in flight (whole on 128x64 tiles
-// 0.9 us faster per ViT attention + MLP than 3 slices of 64x128).
-// With int8 weights the slices run 64x64 tiles (Qwen2.5-0.5B down
-// projection at M = 256: 105 -> 128 TFLOP/s).
-int gemm_splits(const GemmProblem& p) {
-  const bool i8 = p.dtype == DT_W8A16;
-  if (p.batch != 1 || p.out_f32 || p.rms || p.K < (i8 ? 512 : 2048) || p.K % 8 || !gemm_fast_path_ok(p)) return 1;
-  if (const int64_t e = knob(KNOB_SPLITK); e != KNOB_UNSET) return e < 1 ? 1 : (e > 16 ? 16 : (int)e);
-  if (i8 && p.K < 2048) {
-    // int8 weights at short K with few output tiles (the Qwen2.5-0.5B
-    // 896 -> 896 projection at M = 256: 56 tiles of 64x64): each workgroup's
-    // K-steps wait on memory, so slices of >= 256 of K put the same steps on
-    // more CUs (10.7 -> 9.0 us with 3 slices; 7 slices of 128: 12.1 us)
+// K slices of an int8-weight GEMM: its slices run 64x64 tiles (Qwen2.5-0.5B
+// down projection at M = 256: 105 -> 128 TFLOP/s).
+static int splits_i8(const GemmProblem& p) {
+  if (p.K < 512) return 1;
+  if (p.K < 2048) {
+    // short K with few output tiles (the Qwen2.5-0.5B 896 -> 896 projection
+    // at M = 256: 56 tiles of 64x64): each workgroup's K-steps wait on
+    // memory, so slices of >= 256 of K put the same steps on more CUs (10.7
+    // -> 9.0 us with 3 slices; 7 slices of 128: 12.1 us)
     const int64_t t64 = ((p.M + 63) / 64) * ((p.N + 63) / 64);
     if (t64 >= 128) return 1;
     int s = (int)((240 + t64 / 2) / t64);
@@ -304,22 +259,117 @@ int gemm_splits(const GemmProblem& p) {
   }
   const int64_t tiles = ((p.M + 63) / 64) * ((p.N + 127) / 128);
   if (tiles >= 384 || p.K < 4096) return 1;
-  // long slices: two of them once every CU has a workgroup (measured in the
-  // TinyLlama block sequence, weights not resident in L2: the 512x2048x5632
-  // down projection ran 80.9 us per block with 2 slices, 83.0 with 3, 83.3
-  // with 4, where each slice's fix-up traffic outweighs the extra workgroups)
-  if (p.dtype != DT_W8A16 && tiles * 2 >= 256 && p.K / 2 >= 2048) return 2;
   int s = (int)((480 + tiles / 2) / tiles);
   s = s < 1 ? 1 : (s > 4 ? 4 : s);
   while (s > 1 && p.K / s < 1024) --s;
   return s;
 }
 
+// Tile and K slices of an fp16 / bf16 GEMM: the pair with the least estimated
+// time.  Per 64-deep K-step a tile alone on its CU takes `lat` us (few CUs
+// busy: the loads' latency and its own MFMAs) and, with every CU busy, `thr`
+// us of its CU (memory contention and the power limit slow it), `epi` us for
+// its epilogue; per_cu workgroups share a CU.  Splitting K over s workgroups
+// puts short outputs on more CUs and costs 1.0 + 0.6 s us of fix-up round
+// trips plus the partial tiles' traffic.  Constants fitted to every tile and
+// 1-16 slices on 8 shapes at 20-4096 rows (graph replays, weights rotating);
+// us, the tile rule before it (area over a fixed efficiency, K < 4096 never
+// split) against the pair it takes now:
+//   20 x 80 x 3800 13.6 -> 7.9; 64 x 768 x 3072 12.2 -> 8.6; 64 x 2048 x 5632 18.3 -> 13.2;
+//   256 x 896 x 4864 14.7 -> 11.1; 700 x 2560 x 2048 16.9 -> 13.7; 1028 x 2048 x 5632 54.3 -> 37.2;
+//   2000 x 2048 x 5632 74.8 -> 62.9; 512 x 2048 x 5632 (two slices, as before) 27.3 -> 26.3.
+namespace {
+
+struct TileCost {
+  int id, bm, bn, per_cu;
+  float lat, thr, epi;
+};
+constexpr TileCost kCosts[] = {
+    {TILE_256x256_W8, 256, 256, 1, 1.10f, 1.45f, 3.0f}, {TILE_256x128_W8, 256, 128, 1, 0.68f, 0.92f, 1.8f},
+    {TILE_128x192_W8, 128, 192, 1, 0.55f, 0.72f, 1.6f}, {TILE_128x128_W8, 128, 128, 2, 0.57f, 0.47f, 1.2f},
+    {TILE_64x128, 64, 128, 2, 0.35f, 0.37f, 1.0f},      {TILE_128x64, 128, 64, 2, 0.33f, 0.35f, 1.0f},
+    {TILE_64x64, 64, 64, 2, 0.22f, 0.24f, 0.5f},
+};
+
+struct Plan {
+  int tile, splits;
+  float us;
+};
+
+float plan_us(const GemmProblem& p, const TileCost& c, int splits) {
+  const int64_t tiles = ((p.M + c.bm - 1) / c.bm) * ((p.N + c.bn - 1) / c.bn) * p.batch * splits;
+  const int slots = 256 * c.per_cu;
+  const int64_t full = tiles / slots;
+  const int rem = (int)(tiles - full * slots), conc = (rem + 255) / 256;
+  const float round = std::max(c.lat, c.per_cu * c.thr);
+  const float last = rem ? std::max(c.lat, conc * c.thr * (0.85f + 0.15f * (float)rem / (256.f * conc))) : 0.f;
+  const float steps = (float)((p.K + 64 * splits - 1) / (64 * splits));
+  float t = steps * ((float)full * round + last);
+  // an RMSNorm-folded GEMM sums the squares of its A rows in every tile of a
+  // row, so narrow tiles repeat that work more often
+  if (p.rms) t *= c.bn == 64 ? 1.3f : 1.1f;
+  t += 2.6f + c.epi * ((float)full * c.per_cu + conc);
+  if (splits > 1) t += 1.0f + 0.6f * splits + (float)(p.M * p.N * splits) * (8.f / 6e6f);
+  return t;
+}
+
+// (splits > 0: that many slices; otherwise as many as pay)
+Plan gemm_plan(const GemmProblem& p, int splits) {
+  Plan best{TILE_64x64, 1, 1e30f};
+  for (const TileCost& c : kCosts) {
+    if (c.bn == 64 && p.epilogue == EPI_SILU_MUL) continue;
+    if (c.id == TILE_128x192_W8 && !p.b_nt) continue;  // (k-contiguous weights only)
+    const int64_t tiles = ((p.M + c.bm - 1) / c.bm) * ((p.N + c.bn - 1) / c.bn);
+    const int first = splits > 0 ? splits : 1;
+    // slices of at least four K-steps that stay within two rounds of the
+    // CUs, their partial tiles within 32 MiB
+    const int64_t most = splits > 0 ? splits
+                                    : std::min<int64_t>({8, p.K / 256, 512 / tiles,
+                                                         ((32 << 20) - kWsCounterBytes) / (tiles * c.bm * c.bn * 4)});
+    for (int s = first; s == first || s <= most; s += s < 4 ? 1 : 2) {
+      const float us = plan_us(p, c, s);
+      if (us < (s > 1 ? 0.98f : 1.f) * best.us) best = {c.id, s, us};
+    }
+  }
+  // 64x64 tiles with a CU each and k-contiguous weights: a fourth LDS stage
+  // (64 x 1152 x 896 6.2 -> 5.9 us, 256 x 2560 x 2048 10.5 -> 9.6; with two
+  // tiles a CU 15.2 -> 15.5 us, and the NN 1024^3 GEMM 6.4 -> 6.5)
+  const int64_t t64 = ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch * best.splits;
+  if (best.tile == TILE_64x64 && p.b_nt && t64 <= 256 && p.K >= 768) best.tile = TILE_64x64_S4;
+  return best;
+}
+
+bool may_split(const GemmProblem& p) {
+  return p.batch == 1 && !p.out_f32 && !p.rms && p.K >= 512 && p.K % 8 == 0 && gemm_fast_path_ok(p);
+}
+
+}  // namespace
+
+int gemm_pick_tile(const GemmProblem& p) {
+  if (p.K % 8) return gemm::tile_of_two(p);
+  const int forced = gemm::forced_tile(p);
+  if (forced >= 0) return forced;
+  return p.dtype == DT_W8A16 ? pick_tile_i8(p) : gemm_plan(p, 1).tile;
+}
+
 // The split-K launch of p: K slices of kc (a multiple of the 64-deep K-step)
 // as a batch of GEMMs into the same output (sC = 0), the tile they run and
 // the fix-up workspace they need.  False when p does not split.
 static bool split_plan(const GemmProblem& p, GemmProblem& q, int& tile, int64_t& need) {
-  const int splits = gemm_splits(p);
+  if (!may_split(p)) return false;
+  const bool i8 = p.dtype == DT_W8A16;
+  const int64_t want = knob(KNOB_SPLITK);
+  const int forced_splits = want == KNOB_UNSET ? 0 : (int)std::max<int64_t>(1, std::min<int64_t>(16, want));
+  int splits;
+  tile = gemm::forced_tile(p);
+  if (i8) {
+    splits = forced_splits ? forced_splits : splits_i8(p);
+    if (tile < 0) tile = TILE_64x64;
+  } else {
+    const Plan plan = gemm_plan(p, forced_splits);
+    splits = plan.splits;
+    if (tile < 0) tile = plan.tile;
+  }
   if (splits <= 1) return false;
   q = p;
   const int64_t kc = ((p.K + splits - 1) / splits + 63) / 64 * 64;
@@ -328,12 +378,6 @@ static bool split_plan(const GemmProblem& p, GemmProblem& q, int& tile, int64_t&
   q.sA = kc;
   q.sB = p.b_nt ? kc : kc * p.ldb;
   q.sC = 0;
-  // (fp16: the two long slices of a down projection run 128x64 tiles, the
-  // 512x2048x5632 one 0.65 us faster in the block sequence than 64x128;
-  // ViT fc2's three slices of 1024 measured equal or slower with 128x64)
-  if (q.tile < 0 && gemm::knob_or(KNOB_GEMM_TILE, -1) < 0)
-    q.tile = p.dtype == DT_W8A16 ? TILE_64x64 : (splits == 2 && p.K / 2 >= 2048 ? TILE_128x64 : TILE_64x128);
-  tile = gemm::tile_for(q);
   const gemm::TileShape s = gemm::kTiles[tile];
   const int64_t tiles = ((p.M + s.BM - 1) / s.BM) * ((p.N + s.BN - 1) / s.BN);
   need = kWsCounterBytes + tiles * q.batch * s.BM * s.BN * 4;
@@ -354,7 +398,7 @@ hipError_t launch_gemm(const GemmProblem& p, hipStream_t stream) {
     if (i8) return hipErrorNotSupported;
     if (gemm::any_alignment_ok(p)) {
       if (gemm::operands_aligned(p)) {  // only C is off the 16-byte grid
-        const int tile = gemm::tile_for(p);
+        const int tile = gemm_pick_tile(p);
         return gemm::launch_fast(p, tile, gemm::make_kargs(p, tile), stream);
       }
       const int tile = gemm::tile_of_two(p);
@@ -409,7 +453,7 @@ hipError_t launch_gemm(const GemmProblem& p, hipStream_t stream) {
     return gemm::launch_fast(q, qtile, k, stream);
   }
 
-  const int tile = gemm::tile_for(p);
+  const int tile = gemm_pick_tile(p);
   return gemm::launch_fast(p, tile, gemm::make_kargs(p, tile), stream);
 }
 

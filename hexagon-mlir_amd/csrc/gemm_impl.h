@@ -212,25 +212,18 @@ __device__ __forceinline__ short8v dequant8(int2v raw) {
   return out;
 }
 
-// ss + the sum of squares of 8 packed fp16 / bf16 values (v_dot2 on pairs).
+// ss + the squares of pair q of 8 packed fp16 / bf16 values (v_dot2).
 template <typename T>
-__device__ __forceinline__ float sumsq8(short8v v, float ss) {
+__device__ __forceinline__ float sumsq2(short8v v, int q, float ss) {
   if constexpr (std::is_same_v<T, _Float16>) {
     const half8v h = __builtin_bit_cast(half8v, v);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const half2v p2 = {h[2 * q], h[2 * q + 1]};
-      ss = __builtin_amdgcn_fdot2(p2, p2, ss, false);
-    }
+    const half2v p2 = {h[2 * q], h[2 * q + 1]};
+    return __builtin_amdgcn_fdot2(p2, p2, ss, false);
   } else {
     const bf16x8v h = __builtin_bit_cast(bf16x8v, v);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const bf16x2v p2 = {h[2 * q], h[2 * q + 1]};
-      ss = __builtin_amdgcn_fdot2_f32_bf16(p2, p2, ss, false);
-    }
+    const bf16x2v p2 = {h[2 * q], h[2 * q + 1]};
+    return __builtin_amdgcn_fdot2_f32_bf16(p2, p2, ss, false);
   }
-  return ss;
 }
 
 // The first n (clamped to 0..8) of 8 packed 16-bit values, the rest zero.
@@ -247,7 +240,7 @@ __device__ __forceinline__ short8v keep_first(short8v v, int n) {
 // NVA vector-ALU instructions (the RMSNorm sums of squares of this substep's
 // fragments) go over the second half of the MFMAs, when every fragment has
 // been consumed once and its LDS read has certainly returned.
-template <int NMF, int NDS, int NVM, int NVA = 0>
+template <int NMF, int NDS, int NVM, int NVA>
 __device__ __forceinline__ void schedule_substep() {
   static_assert(NMF > 0, "substep without MFMAs");
   constexpr int kVALU = 0x002, kMFMA = 0x008, kVMEMR = 0x020, kDSR = 0x100;
@@ -273,10 +266,10 @@ __device__ __forceinline__ void schedule_substep() {
 // fragments (NBR reads per B fragment) and, in turn with them, NVM global->LDS
 // loads over the first SPAN MFMAs.  (4096^3 NT on the 8-wave 256x256 tile:
 // loads behind the reads at the substep's end 108.3 us, in turn 100.8.)
-template <int NMF, int NB, int NA, int NBR, int NVM, int NVA>
+template <int NMF, int NB, int NA, int NBR, int NVM>
 __device__ __forceinline__ void schedule_pieces() {
-  constexpr int kVALU = 0x002, kMFMA = 0x008, kVMEMR = 0x020, kDSR = 0x100;
-  constexpr int NP = NB + NA, SPAN = NMF - NMF / 8, HALF = NMF - NMF / 2;
+  constexpr int kMFMA = 0x008, kVMEMR = 0x020, kDSR = 0x100;
+  constexpr int NP = NB + NA, SPAN = NMF - NMF / 8;
   static_for<NMF>([&](auto M) {
     constexpr int m = decltype(M)::value;
     __builtin_amdgcn_sched_group_barrier(kMFMA, 1, 0);
@@ -287,9 +280,6 @@ __device__ __forceinline__ void schedule_pieces() {
       if constexpr (nr > 0) __builtin_amdgcn_sched_group_barrier(kDSR, nr, 0);
       if constexpr (nv > 0) __builtin_amdgcn_sched_group_barrier(kVMEMR, nv, 0);
     });
-    constexpr int ma = m - (NMF - HALF);
-    constexpr int na = (NVA > 0 && ma >= 0) ? (ma + 1) * NVA / HALF - ma * NVA / HALF : 0;
-    if constexpr (na > 0) __builtin_amdgcn_sched_group_barrier(kVALU, na, 0);
   });
 }
 
@@ -303,10 +293,10 @@ __device__ __forceinline__ void pp_barrier() {
 }
 
 // RMS = true: C = epilogue(rmsnorm(A) . B^T) for an NT GEMM whose B already
-// holds the RMSNorm weight folded in (B[n][k] = g[k] * W[n][k]).  Every wave
-// sums the squares of the A fragments it multiplies (its rows, all of K) and
-// scales its accumulators by rsqrt(mean + eps) before the epilogue, so the
-// normalised activations are never written.
+// holds the RMSNorm weight folded in (B[n][k] = g[k] * W[n][k]).  The waves
+// sum the squares of the A fragments they multiply (the waves of a tile row
+// sharing its K-steps) and scale their accumulators by rsqrt(mean + eps)
+// before the epilogue, so the normalised activations are never written.
 //
 // PP = true: ping-pong schedule for 8 waves in two groups of 4 (group =
 // wave / 4 = the tile's upper or lower half of rows, one wave of each group
@@ -577,9 +567,24 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
   for (int i = 0; i < TN; ++i)
 #pragma unroll
     for (int j = 0; j < TM; ++j) acc[i][j] = Acc{};
-  float ss[TM];  // RMS: this lane's sum of squares of row (j*MI + lane%MI), its k share
+  // RMS: this lane's sums of squares of row (j*MI + lane%MI), its k share.
+  // On the 8-wave tiles the NWN waves of a tile row multiply the same A rows
+  // and take turns at the sums, one K-step in NWN each, the two waves of a
+  // SIMD in different ones (the 4096-token QKV projection on 256x256: 58.9 ->
+  // 47.1 us, 43.7 without the norm).  On the 4-wave tiles every wave sums all
+  // of K under its MFMAs: taking turns there measured 0.4 us slower, and four
+  // independent chains of sums the same.
+  constexpr int RS = MI == 16 ? NWN : 1;
+  static_assert(!RMS || (RS & (RS - 1)) == 0, "waves of a tile row");
+  float ss[TM];
 #pragma unroll
   for (int j = 0; j < TM; ++j) ss[j] = 0.f;
+  auto sum_squares = [&](const short8v (&f)[TM]) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) ss[j] = sumsq2<T>(f[j], q, ss[j]);
+  };
 
   // Software pipeline over K-steps: STAGES LDS stages (step kt lives in stage
   // kt % STAGES), fragments double buffered in registers.  Per K-step kt:
@@ -695,10 +700,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
         for (int i = 0; i < TN; ++i)
 #pragma unroll
           for (int j = 0; j < TM; ++j) acc[i][j] = Mfma<T>::run(fb[i], fa[j], acc[i][j]);
-        if constexpr (RMS) {
-#pragma unroll
-          for (int j = 0; j < TM; ++j) ss[j] = sumsq8<T>(fa[j], ss[j]);
-        }
+        if constexpr (RMS) sum_squares(fa);
       });
       if (kt + 1 < nk) {
         commit(kt + 1, (kt + 1) & 1);
@@ -775,13 +777,14 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
       for (int i = 0; i < TN; ++i)
 #pragma unroll
         for (int j = 0; j < TM; ++j) acc[i][j] = Mfma<T>::run(fb[cur][i], fa[cur][j], acc[i][j]);
-      if constexpr (RMS) {
-#pragma unroll
-        for (int j = 0; j < TM; ++j) ss[j] = sumsq8<T>(fa[cur][j], ss[j]);
-      }
-      if constexpr (MI == 32) schedule_substep<TN * TM, NDS, (t == SUBS) ? NVM : 0, RMS ? TM * 4 : 0>();
-      else schedule_pieces<TN * TM, TN, TM, NN ? 2 : (BI8 && t % 2 ? 0 : 1), (t == SUBS) ? NVM : 0, RMS ? TM * 4 : 0>();
+      if constexpr (RMS && RS == 1) sum_squares(fa[cur]);
+      if constexpr (MI == 32) schedule_substep<TN * TM, NDS, (t == SUBS) ? NVM : 0, RMS && RS == 1 ? TM * 4 : 0>();
+      else schedule_pieces<TN * TM, TN, TM, NN ? 2 : (BI8 && t % 2 ? 0 : 1), (t == SUBS) ? NVM : 0>();
       __builtin_amdgcn_sched_barrier(0);
+      if constexpr (RMS && RS > 1) {
+        if (((kt + wm) & (RS - 1)) == wn) sum_squares(fa[cur]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     });
     st = st1;
     stb = stb1;
@@ -791,12 +794,21 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
   __syncthreads();
 
   if constexpr (RMS) {
-    // lanes a multiple of MI apart hold the k shares of the same row
+    // lanes a multiple of MI apart hold k shares of the same row, and so do
+    // the waves of a tile row (through LDS; the operand stages are done)
+    float* const part = (float*)smem;
 #pragma unroll
     for (int j = 0; j < TM; ++j) {
-      float tot = ss[j];
-      if constexpr (MI == 16) tot += __shfl_xor(tot, 16, 64);
-      tot += __shfl_xor(tot, 32, 64);
+      if constexpr (MI == 16) ss[j] += __shfl_xor(ss[j], 16, 64);
+      ss[j] += __shfl_xor(ss[j], 32, 64);
+      if (RS > 1 && lane < MI) part[wn * BM + wm * WM + j * MI + lane] = ss[j];
+    }
+    if constexpr (RS > 1) __syncthreads();
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+      float tot = RS > 1 ? 0.f : ss[j];
+#pragma unroll
+      for (int u = 0; u < (RS > 1 ? RS : 0); ++u) tot += part[u * BM + wm * WM + j * MI + (lane & (MI - 1))];
       const float r = rsqrtf(tot / (float)a.K + a.rms_eps);
 #pragma unroll
       for (int i = 0; i < TN; ++i) acc[i][j] *= r;

@@ -91,9 +91,8 @@ hipError_t launch_fold_rms_weight(int dtype, const void* W, const void* g, void*
 hipError_t launch_quantize_int8_rows(const void* W, int8_t* q, void* s, int64_t N, int64_t K, int64_t ldw,
                                      int64_t ldq, hipStream_t stream);
 
-// Split-K factor the dispatcher uses for p (1 = none) and the workspace bytes
-// it needs; both depend only on shapes and epilogue.
-int gemm_splits(const GemmProblem& p);
+// Workspace bytes of the split-K launch the dispatcher uses for p (0: none),
+// which depends only on shapes and epilogue.
 int64_t gemm_workspace_bytes(const GemmProblem& p);
 
 // Tile shapes the fast kernel is instantiated for.

@@ -1,10 +1,10 @@
 // Native entry of the torch-facing ops (hxmi.py) for their plain form: every
 // tensor an ordinary strided GPU tensor on one device, already in the layout
-// the C ABI takes, no workspace.  Each function checks exactly that,
-// allocates the result and calls the C ABI on the current stream; for
-// anything else, and for a call the library rejects, it returns None and the
-// Python form of the op runs, which converts what it can and names what it
-// cannot.  A launch costs the host 2.7 us; the Python form of these ops took
+// the C ABI takes.  Each function checks exactly that, allocates the result
+// (a split-K workspace comes from hxmi.py's own cache) and calls the C ABI on
+// the current stream; for anything else, and for a call the library rejects,
+// it returns None and the Python form of the op runs, which converts what it
+// can and names what it cannot.  A launch costs the host 2.7 us; the Python form of these ops took
 // 8.2-17.4 us a call (arguments, checks, allocation, ctypes), which is what
 // a decode projection or a norm took eagerly whatever its kernel did.
 #include <Python.h>
@@ -14,6 +14,7 @@
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Device.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -105,9 +106,35 @@ Tensor like(const Tensor& t, at::IntArrayRef shape) { return at::empty(shape, t.
     if (!(cond)) Py_RETURN_NONE; \
   } while (0)
 
-// C[M, nout] of a GEMM without workspace; false when it takes one.
-bool no_workspace(int64_t M, int64_t N, int64_t K, int nt, int epi) {
-  return hxmi_gemm_workspace_bytes(M, N, K, nt, epi) == 0;
+// The split-K workspace of one call: hxmi.py's _workspace(bytes, device), which
+// keeps one per stream and per graph capture.
+PyObject* g_workspace = nullptr;
+
+struct Workspace {
+  PyObject* tensor = nullptr;
+  void* data = nullptr;
+  int64_t bytes = 0;
+  bool ok = true;  // false: a Python error is set
+
+  Workspace(int64_t need, const Tensor& like) {
+    if (need <= 0) return;
+    PyObject* const device = g_workspace ? THPDevice_New(like.device()) : nullptr;
+    tensor = device ? PyObject_CallFunction(g_workspace, "LO", (long long)need, device) : nullptr;
+    Py_XDECREF(device);
+    ok = tensor && THPVariable_Check(tensor);
+    if (!ok) return;
+    const Tensor& t = THPVariable_Unpack(tensor);
+    data = t.data_ptr();
+    bytes = t.nbytes();
+  }
+  ~Workspace() { Py_XDECREF(tensor); }
+};
+
+PyObject* set_workspace(PyObject*, PyObject* fn) {
+  Py_INCREF(fn);
+  Py_XDECREF(g_workspace);
+  g_workspace = fn;
+  Py_RETURN_NONE;
 }
 
 // gemm(a, b, nt, epilogue, bias, alpha, out)
@@ -126,17 +153,18 @@ PyObject* op_gemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const int64_t M = a->size(0), K = a->size(1), N = b->size(nt ? 0 : 1);
   const int64_t nout = epi == kEpiSiluMul ? N / 2 : N;
   const bool takes_bias = epi == kEpiBias || epi == kEpiBiasGelu;
-  NOT_PLAIN_UNLESS(b->size(nt ? 1 : 0) == K && takes_bias == (bias != nullptr) && vec(bias, N, a->scalar_type()) &&
-                   no_workspace(M, N, K, nt, epi));
+  NOT_PLAIN_UNLESS(b->size(nt ? 1 : 0) == K && takes_bias == (bias != nullptr) && vec(bias, N, a->scalar_type()));
   NOT_PLAIN_UNLESS(!o || (o->dim() == 2 && o->size(0) == M && o->size(1) == nout &&
                           o->scalar_type() == a->scalar_type()));
   const Tensor out = o ? *o : like(*a, {M, nout});
   NOT_PLAIN_UNLESS(rows(out, ldc));
   const auto fn = bf16(*a) ? hxmi_gemm_bf16 : hxmi_gemm_f16;
+  const Workspace ws(hxmi_gemm_workspace_bytes(M, N, K, nt, epi), *a);
+  if (!ws.ok) return nullptr;
   void* s = in.stream();
   return result(unlocked([&] {
                   return fn(ptr(a), ptr(b), ptr(&out), ptr(bias), M, N, K, lda, ldb, ldc, nt, epi, (float)alpha,
-                            nullptr, 0, s);
+                            ws.data, ws.bytes, s);
                 }),
                 out);
   END_HANDLE_TH_ERRORS
@@ -206,15 +234,18 @@ PyObject* op_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   NOT_PLAIN_UNLESS(as_rows(*x, M, K, ldx) && rows(*w, ldw) && w->size(1) == K);
   const int64_t N = w->size(0), nout = epi == kEpiSiluMul ? N / 2 : N;
   const bool takes_bias = epi == kEpiBias || epi == kEpiBiasGelu;
-  NOT_PLAIN_UNLESS(takes_bias == (bias != nullptr) && vec(bias, N, x->scalar_type()) && no_workspace(M, N, K, 1, epi));
+  NOT_PLAIN_UNLESS(takes_bias == (bias != nullptr) && vec(bias, N, x->scalar_type()));
   NOT_PLAIN_UNLESS(!o || (o->dim() == 2 && o->size(0) == M && o->size(1) == nout &&
                           o->scalar_type() == x->scalar_type() && rows(*o, ldy)));
   const Tensor out = o ? *o : rows_like(*x, nout);
   if (!o) ldy = std::max<int64_t>(nout, 1);
   const auto fn = bf16(*x) ? hxmi_gemm_bf16 : hxmi_gemm_f16;
+  const Workspace ws(hxmi_gemm_workspace_bytes(M, N, K, 1, epi), *x);
+  if (!ws.ok) return nullptr;
   void* s = in.stream();
   return result(unlocked([&] {
-                  return fn(ptr(x), ptr(w), ptr(&out), ptr(bias), M, N, K, ldx, ldw, ldy, 1, epi, 1.f, nullptr, 0, s);
+                  return fn(ptr(x), ptr(w), ptr(&out), ptr(bias), M, N, K, ldx, ldw, ldy, 1, epi, 1.f, ws.data,
+                            ws.bytes, s);
                 }),
                 out);
   END_HANDLE_TH_ERRORS
@@ -258,15 +289,17 @@ PyObject* op_gemv(PyObject*, PyObject* const* args, Py_ssize_t n) {
   int64_t ldx, ldw, ldy;
   NOT_PLAIN_UNLESS(rows(*x, ldx) && rows(*w, ldw) && w->size(1) == x->size(1));
   const int64_t M = x->size(0), K = x->size(1), N = w->size(0);
-  NOT_PLAIN_UNLESS(vec(bias, N, x->scalar_type()) && hxmi_gemv_workspace_bytes(M, N, K) == 0);
+  NOT_PLAIN_UNLESS(vec(bias, N, x->scalar_type()));
   NOT_PLAIN_UNLESS(!o || (o->dim() == 2 && o->size(0) == M && o->size(1) == N &&
                           o->scalar_type() == x->scalar_type()));
   const Tensor out = o ? *o : like(*x, {M, N});
   NOT_PLAIN_UNLESS(rows(out, ldy));
   const auto fn = bf16(*x) ? hxmi_gemv_bf16 : hxmi_gemv_f16;
+  const Workspace ws(hxmi_gemv_workspace_bytes(M, N, K), *x);
+  if (!ws.ok) return nullptr;
   void* s = in.stream();
   return result(unlocked([&] {
-                  return fn(ptr(x), ptr(w), ptr(bias), ptr(&out), M, N, K, ldx, ldw, ldy, nullptr, 0, s);
+                  return fn(ptr(x), ptr(w), ptr(bias), ptr(&out), M, N, K, ldx, ldw, ldy, ws.data, ws.bytes, s);
                 }),
                 out);
   END_HANDLE_TH_ERRORS
@@ -283,14 +316,16 @@ PyObject* op_w8a16_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   int64_t ldx, ldw, ldy;
   NOT_PLAIN_UNLESS(rows(*x, ldx) && rows(*w, ldw) && w->size(1) == x->size(1));
   const int64_t M = x->size(0), K = x->size(1), N = w->size(0);
-  NOT_PLAIN_UNLESS(vec(scale, N, at::kHalf) && vec(bias, N, at::kHalf) && hxmi_w8a16_workspace_bytes(M, N, K) == 0);
+  NOT_PLAIN_UNLESS(vec(scale, N, at::kHalf) && vec(bias, N, at::kHalf));
   NOT_PLAIN_UNLESS(!o || (o->dim() == 2 && o->size(0) == M && o->size(1) == N && o->scalar_type() == at::kHalf));
   const Tensor out = o ? *o : like(*x, {M, N});
   NOT_PLAIN_UNLESS(rows(out, ldy));
+  const Workspace ws(hxmi_w8a16_workspace_bytes(M, N, K), *x);
+  if (!ws.ok) return nullptr;
   void* s = in.stream();
   return result(unlocked([&] {
                   return hxmi_gemv_w8a16(ptr(x), (const int8_t*)ptr(w), ptr(scale), ptr(bias), ptr(&out), M, N, K, ldx,
-                                         ldw, ldy, nullptr, 0, s);
+                                         ldw, ldy, ws.data, ws.bytes, s);
                 }),
                 out);
   END_HANDLE_TH_ERRORS
@@ -387,6 +422,7 @@ PyObject* op_attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
 #define ENTRY(name) {#name, (PyCFunction)(void (*)(void))op_##name, METH_FASTCALL, nullptr}
 PyMethodDef kMethods[] = {ENTRY(gemm),         ENTRY(bgemm),    ENTRY(linear),  ENTRY(rms_norm_linear), ENTRY(gemv),
                           ENTRY(w8a16_linear), ENTRY(rms_norm), ENTRY(softmax), ENTRY(attention),
+                          {"set_workspace", set_workspace, METH_O, nullptr},
                           {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "hxmi_torch", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 

@@ -114,6 +114,7 @@ class _NativeOps:
         mod = importlib.util.module_from_spec(importlib.util.spec_from_file_location("hxmi_torch", OPS_PATH,
                                                                                      loader=loader))
         loader.exec_module(mod)
+        mod.set_workspace(_workspace)
         _ops = mod
         return getattr(mod, name)
 

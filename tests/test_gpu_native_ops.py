@@ -43,7 +43,7 @@ def calls(pkg, dev):
         ("gemm silu", True, lambda: pkg.gemm(x, w, b_layout="nt", epilogue="silu_mul")),
         ("gemm padded rows", True, lambda: pkg.gemm(wide[:, 8:72], w, b_layout="nt", out=out(40, 104)[:, :96])),
         ("gemm strided bias", False, lambda: pkg.gemm(x, w, b_layout="nt", epilogue="bias", bias=n(dev, 192)[::2])),
-        ("gemm workspace", False, lambda: pkg.gemm(long_x, long_w, b_layout="nt")),
+        ("gemm workspace", True, lambda: pkg.gemm(long_x, long_w, b_layout="nt")),
         ("gemm no rows", True, lambda: pkg.gemm(x[:0], w, b_layout="nt")),
         ("gemm bf16", True, lambda: pkg.gemm(bx, bw, b_layout="nt")),
         ("linear 3-D gelu", True, lambda: pkg.linear(x.view(5, 8, 64), w, b, epilogue="gelu_tanh")),
