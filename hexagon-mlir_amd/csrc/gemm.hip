@@ -6,6 +6,7 @@
 // and rows off the 16-byte grid (leading dimensions not a multiple of 8,
 // misaligned pointers) those that load their tiles through registers.
 #include <algorithm>
+#include <iterator>
 
 #include "gemm_impl.h"
 
@@ -144,43 +145,6 @@ bool gemm_fast_path_ok(const GemmProblem& p) {
   return gemm::operands_aligned(p) && p.ldc % 8 == 0 && (p.batch <= 1 || p.sC % 8 == 0) && gemm::aligned(p.C, 16);
 }
 
-// The int8-weight GEMM's tile: the one that minimises an estimate of makespan,
-// rounds of tiles over the 256 CUs (with the tiles a CU holds at once) times a
-// per-tile cost that reflects each shape's MFMA efficiency.
-static int pick_tile_i8(const GemmProblem& p) {
-  struct Cand {
-    int id, bm, bn, per_cu;
-    float eff;
-  };
-  // int8 B converts every weight once per tile row: tall tiles amortise it,
-  // and the latency-bound small shapes want the most workgroups (measured on
-  // the Qwen2.5-0.5B int8 shapes at M = 256: 896 -> 4864 runs 152 tiles of
-  // 128x64 in 11.5 us against 13.4 us for 304 tiles of 64x64; the lm_head at
-  // M = 128 1187 tiles of 128x128 at two per CU in 56.0 us against 72.0 us for
-  // 594 tiles of 128x256)
-  static const Cand cands[] = {
-      {TILE_256x256_W8, 256, 256, 1, 1.00f}, {TILE_256x128_W8, 256, 128, 1, 0.80f},
-      {TILE_128x256, 128, 256, 1, 0.65f},    {TILE_128x128_W8, 128, 128, 2, 0.80f},
-      {TILE_64x128, 64, 128, 3, 0.50f},      {TILE_128x64, 128, 64, 3, 0.62f},
-      {TILE_64x64, 64, 64, 4, 0.60f},
-  };
-  const int cus = 256;
-  int best = TILE_64x64;
-  double best_t = 1e300;
-  for (const Cand& c : cands) {
-    const int64_t tiles = ((p.M + c.bm - 1) / c.bm) * ((p.N + c.bn - 1) / c.bn) * p.batch;
-    const int64_t slots = (int64_t)cus * c.per_cu;
-    const int64_t rounds = (tiles + slots - 1) / slots;
-    const int64_t conc = tiles < slots ? (tiles + cus - 1) / cus : c.per_cu;  // tiles sharing a CU
-    const double t = (double)rounds * c.bm * c.bn * (double)(conc > 0 ? conc : 1) / c.eff;
-    if (t < best_t * 0.999) {
-      best_t = t;
-      best = c.id;
-    }
-  }
-  return best;
-}
-
 namespace gemm {
 namespace {
 
@@ -195,6 +159,7 @@ int tile_of_two(const GemmProblem& p) {
 int forced_tile(const GemmProblem& p) {
   int tile = p.tile >= 0 ? p.tile : knob_or(KNOB_GEMM_TILE, -1);
   if (tile < 0 || tile >= TILE_COUNT || (tile == TILE_128x192_W8 && (!p.b_nt || p.dtype == DT_W8A16))) return -1;
+  if ((tile == TILE_I8_128x256 || tile == TILE_I8_64x256) && p.dtype != DT_W8A16) return -1;
   if (p.epilogue == EPI_SILU_MUL && kTiles[tile].BN < 128) tile = TILE_64x128;
   return tile;
 }
@@ -241,34 +206,9 @@ hipError_t launch_fast(const GemmProblem& p, int tile, const KArgs& k, hipStream
 }  // namespace
 }  // namespace gemm
 
-// K slices of an int8-weight GEMM: its slices run 64x64 tiles (Qwen2.5-0.5B
-// down projection at M = 256: 105 -> 128 TFLOP/s).
-static int splits_i8(const GemmProblem& p) {
-  if (p.K < 512) return 1;
-  if (p.K < 2048) {
-    // short K with few output tiles (the Qwen2.5-0.5B 896 -> 896 projection
-    // at M = 256: 56 tiles of 64x64): each workgroup's K-steps wait on
-    // memory, so slices of >= 256 of K put the same steps on more CUs (10.7
-    // -> 9.0 us with 3 slices; 7 slices of 128: 12.1 us)
-    const int64_t t64 = ((p.M + 63) / 64) * ((p.N + 63) / 64);
-    if (t64 >= 128) return 1;
-    int s = (int)((240 + t64 / 2) / t64);
-    s = s < 1 ? 1 : (s > 4 ? 4 : s);
-    while (s > 1 && p.K / s < 256) --s;
-    return s;
-  }
-  const int64_t tiles = ((p.M + 63) / 64) * ((p.N + 127) / 128);
-  if (tiles >= 384 || p.K < 4096) return 1;
-  int s = (int)((480 + tiles / 2) / tiles);
-  s = s < 1 ? 1 : (s > 4 ? 4 : s);
-  while (s > 1 && p.K / s < 1024) --s;
-  return s;
-}
-
-// Tile and K slices of an fp16 / bf16 GEMM: the pair with the least estimated
-// time.  Per 64-deep K-step a tile alone on its CU takes `lat` us (few CUs
-// busy: the loads' latency and its own MFMAs) and, with every CU busy, `thr`
-// us of its CU (memory contention and the power limit slow it), `epi` us for
+// Tile and K slices of a GEMM: the pair with the least estimated time.  Per
+// 64-deep K-step a tile alone on its CU takes `lat` us (few CUs busy: the
+// loads' latency and its own MFMAs) and, with every CU busy, `thr` us of its CU (memory contention and the power limit slow it), `epi` us for
 // its epilogue; per_cu workgroups share a CU.  Splitting K over s workgroups
 // puts short outputs on more CUs and costs 1.0 + 0.6 s us of fix-up round
 // trips plus the partial tiles' traffic.  Constants fitted to every tile and
@@ -278,6 +218,8 @@ static int splits_i8(const GemmProblem& p) {
 //   20 x 80 x 3800 13.6 -> 7.9; 64 x 768 x 3072 12.2 -> 8.6; 64 x 2048 x 5632 18.3 -> 13.2;
 //   256 x 896 x 4864 14.7 -> 11.1; 700 x 2560 x 2048 16.9 -> 13.7; 1028 x 2048 x 5632 54.3 -> 37.2;
 //   2000 x 2048 x 5632 74.8 -> 62.9; 512 x 2048 x 5632 (two slices, as before) 27.3 -> 26.3.
+// int8 weights (fitted the same way): 256 x 151936 x 896 98 -> 86; 150 x 151936 x 896 101 -> 74;
+//   64 x 151936 x 896 48.5 -> 39.7; 256 x 11264 x 2048 26.4 -> 20.6; 17 x 2048 x 2048 14.6 -> 9.5.
 namespace {
 
 struct TileCost {
@@ -289,6 +231,15 @@ constexpr TileCost kCosts[] = {
     {TILE_128x192_W8, 128, 192, 1, 0.55f, 0.72f, 1.6f}, {TILE_128x128_W8, 128, 128, 2, 0.57f, 0.47f, 1.2f},
     {TILE_64x128, 64, 128, 2, 0.35f, 0.37f, 1.0f},      {TILE_128x64, 128, 64, 2, 0.33f, 0.35f, 1.0f},
     {TILE_64x64, 64, 64, 2, 0.22f, 0.24f, 0.5f},
+};
+// int8 B: a tile's waves convert every weight they multiply, so the two tiles
+// of one wave row convert each once; two workgroups a CU cover each other's
+// first loads and epilogue
+constexpr TileCost kCostsI8[] = {
+    {TILE_256x256_W8, 256, 256, 1, 2.00f, 2.10f, 3.0f}, {TILE_I8_128x256, 128, 256, 2, 1.10f, 1.00f, 2.5f},
+    {TILE_I8_64x256, 64, 256, 2, 0.53f, 0.72f, 1.5f},   {TILE_128x128, 128, 128, 2, 0.64f, 0.80f, 1.2f},
+    {TILE_64x128, 64, 128, 2, 0.50f, 0.42f, 0.8f},      {TILE_128x64, 128, 64, 2, 0.45f, 0.37f, 0.8f},
+    {TILE_64x64, 64, 64, 2, 0.36f, 0.25f, 0.5f},
 };
 
 struct Plan {
@@ -305,18 +256,22 @@ float plan_us(const GemmProblem& p, const TileCost& c, int splits) {
   const float last = rem ? std::max(c.lat, conc * c.thr * (0.85f + 0.15f * (float)rem / (256.f * conc))) : 0.f;
   const float steps = (float)((p.K + 64 * splits - 1) / (64 * splits));
   float t = steps * ((float)full * round + last);
+  if (p.dtype == DT_W8A16) t = std::max(t, (float)(p.N * p.K) * (1.f / 4.2e6f));  // (the weights from HBM)
   // an RMSNorm-folded GEMM sums the squares of its A rows in every tile of a
   // row, so narrow tiles repeat that work more often
   if (p.rms) t *= c.bn == 64 ? 1.3f : 1.1f;
   t += 2.6f + c.epi * ((float)full * c.per_cu + conc);
-  if (splits > 1) t += 1.0f + 0.6f * splits + (float)(p.M * p.N * splits) * (8.f / 6e6f);
+  if (splits > 1) t += 1.0f + 0.6f * splits + (float)tiles * (float)(c.bm * c.bn) * (8.f / 6e6f);
   return t;
 }
 
 // (splits > 0: that many slices; otherwise as many as pay)
 Plan gemm_plan(const GemmProblem& p, int splits) {
   Plan best{TILE_64x64, 1, 1e30f};
-  for (const TileCost& c : kCosts) {
+  const bool i8 = p.dtype == DT_W8A16;
+  static_assert(std::size(kCosts) == std::size(kCostsI8), "one loop over either");
+  for (const TileCost* e = i8 ? kCostsI8 : kCosts, *const end = e + std::size(kCosts); e != end; ++e) {
+    const TileCost& c = *e;
     if (c.bn == 64 && p.epilogue == EPI_SILU_MUL) continue;
     if (c.id == TILE_128x192_W8 && !p.b_nt) continue;  // (k-contiguous weights only)
     const int64_t tiles = ((p.M + c.bm - 1) / c.bm) * ((p.N + c.bn - 1) / c.bn);
@@ -335,7 +290,7 @@ Plan gemm_plan(const GemmProblem& p, int splits) {
   // (64 x 1152 x 896 6.2 -> 5.9 us, 256 x 2560 x 2048 10.5 -> 9.6; with two
   // tiles a CU 15.2 -> 15.5 us, and the NN 1024^3 GEMM 6.4 -> 6.5)
   const int64_t t64 = ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch * best.splits;
-  if (best.tile == TILE_64x64 && p.b_nt && t64 <= 256 && p.K >= 768) best.tile = TILE_64x64_S4;
+  if (best.tile == TILE_64x64 && !i8 && p.b_nt && t64 <= 256 && p.K >= 768) best.tile = TILE_64x64_S4;
   return best;
 }
 
@@ -349,7 +304,7 @@ int gemm_pick_tile(const GemmProblem& p) {
   if (p.K % 8) return gemm::tile_of_two(p);
   const int forced = gemm::forced_tile(p);
   if (forced >= 0) return forced;
-  return p.dtype == DT_W8A16 ? pick_tile_i8(p) : gemm_plan(p, 1).tile;
+  return gemm_plan(p, 1).tile;
 }
 
 // The split-K launch of p: K slices of kc (a multiple of the 64-deep K-step)
@@ -357,19 +312,12 @@ int gemm_pick_tile(const GemmProblem& p) {
 // the fix-up workspace they need.  False when p does not split.
 static bool split_plan(const GemmProblem& p, GemmProblem& q, int& tile, int64_t& need) {
   if (!may_split(p)) return false;
-  const bool i8 = p.dtype == DT_W8A16;
   const int64_t want = knob(KNOB_SPLITK);
-  const int forced_splits = want == KNOB_UNSET ? 0 : (int)std::max<int64_t>(1, std::min<int64_t>(16, want));
-  int splits;
+  const Plan plan =
+      gemm_plan(p, want == KNOB_UNSET ? 0 : (int)std::max<int64_t>(1, std::min<int64_t>(16, want)));
+  const int splits = plan.splits;
   tile = gemm::forced_tile(p);
-  if (i8) {
-    splits = forced_splits ? forced_splits : splits_i8(p);
-    if (tile < 0) tile = TILE_64x64;
-  } else {
-    const Plan plan = gemm_plan(p, forced_splits);
-    splits = plan.splits;
-    if (tile < 0) tile = plan.tile;
-  }
+  if (tile < 0) tile = plan.tile;
   if (splits <= 1) return false;
   q = p;
   const int64_t kc = ((p.K + splits - 1) / splits + 63) / 64 * 64;

@@ -315,8 +315,8 @@ __device__ __forceinline__ void pp_barrier() {
 // elements and shifted, which leaves zeros past K.
 template <int BM, int BN, int WM, int WN, int BK, int STAGES, bool NN, typename T, int EPI, bool OUTF32,
           bool BI8 = false, bool PP = false, bool RMS = false, bool RAGGED = false, int SB = 0, int FD = 1,
-          bool UNAL = false, int MI = 32>
-__global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a) {
+          bool UNAL = false, int MI = 32, bool OCC2 = false>
+__global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, (OCC2 ? (BM / WM) * (BN / WN) / 2 : 1)) void gemm_mfma(KArgs a) {
   constexpr int NWM = BM / WM, NWN = BN / WN, NW = NWM * NWN, NT = NW * 64;
   constexpr int TM = WM / MI, TN = WN / MI;
   constexpr int KS = 512 / MI;          // k per MFMA: one substep
@@ -341,7 +341,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
   // start, so they cost no registers through the main loop and the
   // epilogue (the 8-wave 256x256 tile holds 256 accumulator VGPRs a lane).
   constexpr bool HAS_BIAS = EPI == EPI_BIAS || EPI == EPI_BIAS_GELU_TANH;
-  constexpr int NCV = (HAS_BIAS ? 1 : 0) + (BI8 ? 1 : 0);
+  // (OCC2: two workgroups of 80 KB a CU leave no room for them)
+  constexpr int NCV = OCC2 ? 0 : (HAS_BIAS ? 1 : 0) + (BI8 ? 1 : 0);
   constexpr int SMEM = SMEM_OPS + NCV * 1024;
   static_assert(BK == 32 || BK == 64, "BK");
   static_assert(STAGES >= 2 && STAGES <= 4, "STAGES");
@@ -381,7 +382,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_mfma(KArgs a)
   const bool cv_lds = NCV > 0 && !UNAL && (a.N % 8) == 0;
   char* const cv_bias = smem + SMEM_OPS;
   char* const cv_scale = smem + SMEM_OPS + (HAS_BIAS ? 1024 : 0);
-  if (cv_lds && w == 0) {
+  if (NCV > 0 && cv_lds && w == 0) {
     const uint32_t off = (uint32_t)(n0 + lane * 8) * 2u;
     if constexpr (HAS_BIAS) load_lds16(make_rsrc(a.bias, (uint32_t)a.N * 2u), (HXMI_LDS void*)to_lds(cv_bias), off);
     if constexpr (BI8) load_lds16(make_rsrc(a.scale, (uint32_t)a.N * 2u), (HXMI_LDS void*)to_lds(cv_scale), off);
@@ -1044,6 +1045,7 @@ struct TileShape {
   int SB = 0;  // B stages (0: as many as A)
   int FD = 1;  // substeps between a fragment's LDS read and its MFMAs
   int MI = 32;  // MFMA: 32x32x16 or 16x16x32
+  bool OCC2 = false;  // int8 B only: two workgroups of 80 KB of LDS and at most 128 registers a CU
 };
 
 // The small tiles run three LDS stages: their K-steps are short (a 64x64x64
@@ -1096,6 +1098,8 @@ constexpr TileShape kTiles[TILE_COUNT] = {
     {128, 128, 32, 64, 64, 2, false, 0, 1, 16},    // TILE_128x128_W8
     {128, 192, 32, 96, 64, 3, false, 0, 1, 16},    // TILE_128x192_W8
     {64, 64, 32, 32, 64, 4, false, 0, 3},      // TILE_64x64_S4
+    {128, 256, 128, 32, 64, 2, false, 0, 1, 32, true},  // TILE_I8_128x256
+    {64, 256, 64, 32, 64, 2, false, 0, 1, 32, true},    // TILE_I8_64x256
 };
 
 template <int TILE, bool NN, typename T, int EPI, bool OUTF32, bool BI8, bool RMS = false, bool RAGGED = false,
@@ -1110,10 +1114,10 @@ hipError_t launch_one(const KArgs& k, hipStream_t stream) {
   // (an NN tile whose loads of one wave lie 8 rows apart keeps 32x32x16)
   constexpr int MI = NN && threads / 64 * (512 / s.BN) % 16 ? 32 : s.MI;
   constexpr int W8_A = s.BM * 128, W8_B = s.BN * 64;
-  constexpr int W8_SB = W8_A / W8_B + 3 > 6 ? 6 : W8_A / W8_B + 3;
+  constexpr int W8_SB = s.OCC2 ? (81920 - 2 * W8_A) / W8_B : W8_A / W8_B + 3 > 6 ? 6 : W8_A / W8_B + 3;
   hipLaunchKernelGGL((gemm_mfma<s.BM, s.BN, s.WM, s.WN, (BI8 ? 64 : s.BK), (BI8 || UNAL ? 2 : s.STAGES), NN, T, EPI,
                                 OUTF32, BI8, (s.PP && !BI8 && !RMS), RMS, RAGGED, (BI8 ? W8_SB : s.SB),
-                                (BI8 || s.PP || UNAL ? 1 : s.FD), UNAL, MI>),
+                                (BI8 || s.PP || UNAL ? 1 : s.FD), UNAL, MI, s.OCC2>),
                      dim3((unsigned)blocks), dim3(threads), 0, stream, k);
   return hipGetLastError();
 }
@@ -1137,6 +1141,12 @@ hipError_t launch_tile(int tile, const KArgs& k, hipStream_t stream) {
     case TILE_128x192_W8:
       if constexpr (BI8 || NN) return hipErrorNotSupported;  // (k-contiguous fp16 / bf16 B only)
       else return launch_one<TILE_128x192_W8, NN, T, EPI, OUTF32, BI8, RMS>(k, stream);
+    case TILE_I8_128x256:
+      if constexpr (BI8) return launch_one<TILE_I8_128x256, NN, T, EPI, OUTF32, BI8, RMS>(k, stream);
+      else return hipErrorNotSupported;
+    case TILE_I8_64x256:
+      if constexpr (BI8) return launch_one<TILE_I8_64x256, NN, T, EPI, OUTF32, BI8, RMS>(k, stream);
+      else return hipErrorNotSupported;
     case TILE_64x64_S4: return launch_one<TILE_64x64_S4, NN, T, EPI, OUTF32, BI8, RMS>(k, stream);
     default: return launch_one<TILE_64x64, NN, T, EPI, OUTF32, BI8, RMS>(k, stream);
   }

@@ -113,6 +113,8 @@ enum TileId {
   TILE_128x128_W8,  // 8 waves of 32x64
   TILE_128x192_W8,  // 8 waves of 32x96, 3 stages; k-contiguous fp16 / bf16 B only (not NN, not int8)
   TILE_64x64_S4,    // TILE_64x64 with 4 LDS stages
+  TILE_I8_128x256,  // 8 waves of 128x32, two workgroups a CU; int8 B only
+  TILE_I8_64x256,   // 8 waves of 64x32, two workgroups a CU; int8 B only
   TILE_COUNT
 };
 

@@ -506,3 +506,22 @@ def test_w8a16_gemm_integer_exact_every_tile(pkg, dev, tile, splits):
         torch.cuda.synchronize()
     exact = x.double() @ q.double().T
     assert np.array_equal(y.cpu().numpy(), exact.numpy().astype(np.float16))
+
+
+@pytest.mark.parametrize("tile", [16, 17])  # 128x256 and 64x256, one wave row, two workgroups a CU
+@pytest.mark.parametrize("M,N,K", [(17, 8, 16), (64, 256, 64), (65, 264, 784), (129, 520, 192), (256, 1000, 896)])
+@pytest.mark.parametrize("splits", [1, 2])
+def test_w8a16_gemm_wide_tiles_exact(pkg, dev, tile, M, N, K, splits):
+    """The int8-only tiles at their edges, with the scales and bias they read
+    from global memory in the epilogue: powers of two as scales and small
+    integers keep every value exact (|sum| <= 896 * 2 * 7)."""
+    g = torch.Generator().manual_seed(65)
+    x = torch.randint(-2, 3, (M, K), generator=g).half()
+    q = torch.randint(-7, 8, (N, K), generator=g, dtype=torch.int8)
+    s = torch.exp2(torch.randint(-2, 2, (N,), generator=g).float()).half()
+    b = torch.randint(-8, 9, (N,), generator=g).half()
+    with pkg.tuning(w8_tile=tile, splitk=splits):
+        y = pkg.w8a16_linear(x.to(dev), q.to(dev), s.to(dev), b.to(dev))
+        torch.cuda.synchronize()
+    exact = (x.double() @ q.double().T) * s.double() + b.double()
+    assert np.array_equal(y.cpu().numpy(), exact.numpy().astype(np.float16))
