@@ -29,7 +29,13 @@ int pick_cfg(const AttnProblem& p) {
   // pair up, so the causal lines lie at about twice the others.
   const bool few_keys = p.skv <= 384;
   const int64_t wg128 = p.bh * ((p.s + 127) / 128), wg64 = p.bh * ((p.s + 63) / 64);
-  if (wg128 >= (p.causal ? 320 : few_keys ? 192 : 144)) return p.d <= 64 && !few_keys ? 42 : 41;
+  // A mask's entries take registers that eight waves do not have: 128
+  // queries run four waves, and pay only from 320 on (8 waves / 4 waves / 64
+  // queries: 32 x 1024 full 23.7 / 25.5 / 20.8, 64 x 500 15.3 / 15.7 / 14.1,
+  // 64 x 1000 39.1 / 38.7 / 40.3, 128 x 2048 causal 135 / 131 / 142).
+  const bool masked64 = p.mask && p.d <= 64;
+  if (wg128 >= (p.causal ? 320 : few_keys ? 192 : masked64 ? 320 : 144))
+    return p.d <= 64 && !few_keys && !p.mask ? 42 : 41;
   return wg64 >= (few_keys ? 144 : p.causal ? 288 : 192) ? 22 : 14;
 }
 
@@ -50,7 +56,6 @@ hipError_t launch_attention(const AttnProblem& p, hipStream_t stream) {
   a.kv_group = (int)p.kv_group;
   a.mask_group = (int)(p.mask_group > 0 ? p.mask_group : 1);
   a.causal_off = p.causal == 1 ? 0 : p.causal == 2 ? (int)(p.skv - p.s) : (int)p.skv;
-  a.mask_vec = p.mask && p.ldm % 4 == 0 && p.sm % 4 == 0 && ((uintptr_t)p.mask & 7) == 0;
   a.ldq = p.ldq;
   a.ldk = p.ldk;
   a.ldv = p.ldv;

@@ -35,6 +35,11 @@
 //     2048 x 2048 at head dim 64 went 53.0 -> 42.9 us (800 TFLOP/s), causal
 //     33.2 -> 26.3, head dim 128 x 4096 312 -> 277 us (994 TFLOP/s) against one
 //     stage of twice the keys, waited for whole, and one block at a time;
+//   * mask entries are read one stage ahead, 32 contiguous bytes a lane
+//     wherever the rows start; loaded as a stage began, 8 bytes (rows off the
+//     8-byte grid: 2) at a time, they took longer than the rest of the kernel
+//     (32 x 1024 x 1024, D 64: 31.9 -> 20.8 us, causal 22.0 -> 15.5, unmasked
+//     14.0 and 11.4; 64 x 1000, D 128 causal 72.6 -> 35.9, unmasked 27);
 //   * O = D[d][query] accumulates in registers and is divided by the sum of
 //     the same 16-bit weights once at the end.  A query whose every key is
 //     masked divides 0 by 0 (NaN), as the reference's decomposition does.
@@ -63,7 +68,6 @@ struct AArgs {
   int kv_group;    // query slices per K/V slice
   int mask_group;  // query slices per mask slice
   int causal_off;  // key > query + causal_off is masked (skv: no causal rule)
-  int mask_vec;    // mask rows allow aligned 8-byte loads
   int order;       // OrderId: workgroup -> (slice, query block)
   int64_t ldq, ldk, ldv, ldo, ldm;  // row strides, elements
   int64_t bq, bk, bv, bo, bm;       // slice strides, elements
@@ -177,6 +181,12 @@ struct AttnShape {
   static constexpr bool ok = NT <= 1024 && (KS - 1) * QG * NV * 64 * 4 <= 2 * ST * CHUNK;
 };
 
+typedef uint32_t uint2v __attribute__((ext_vector_type(2)));
+typedef int int4u __attribute__((ext_vector_type(4), aligned(2)));  // (mask rows start anywhere)
+struct MaskBlock {
+  int4v v[2];
+};
+
 // DT: 32-wide output tiles computed (fewer than D / 32 for head dims 72-96).
 // PART: the head dim a.d is below D; rows fill up with zeros.
 template <typename T, int D, int DT, bool PART, int QG, int KS, bool MASK>
@@ -216,9 +226,10 @@ __global__ __launch_bounds__(64 * QG * KS, (AttnShape<D, QG, KS, MASK>::WPE)) vo
   const int wkend = q0 < a.sq ? max(0, min(a.skv, min(q0 + 31, a.sq - 1) + a.causal_off + 1)) : 0;
   const int nchunk = kend > 0 ? (kend + KC - 1) / KC : 0;
 
+  // this lane's mask row (queries past the sequence read the last one's)
   const _Float16* mrow = nullptr;
-  if (MASK && qme < a.sq)
-    mrow = (const _Float16*)a.mask + ((int64_t)(bh / a.mask_group) * a.bm + (int64_t)qme * a.ldm);
+  if constexpr (MASK)
+    mrow = (const _Float16*)a.mask + ((int64_t)(bh / a.mask_group) * a.bm + (int64_t)min(qme, a.sq - 1) * a.ldm);
 
   // Q fragments of this wave's 32 queries (zero past the sequence).  The
   // loads take no branch (an offset past the buffer reads zeros).
@@ -279,23 +290,26 @@ __global__ __launch_bounds__(64 * QG * KS, (AttnShape<D, QG, KS, MASK>::WPE)) vo
     vbase[dt] = CHUNK + v_off<D>(4 * h + (L >> 2), d >> 3) + (d & 7) * 2;
   }
 
-  // mask entries of the 32-key block at kb for this lane's 16 scores: keys kb + 8g + 4h + j
-  auto mask_vals = [&](int kb, half4v (&mk)[4]) {
+  // Mask entries of the 32-key block at kb < skv, keys kb + 16h to + 16h + 15
+  // of this lane's query as they lie in memory.  A lane's scores are keys
+  // kb + 8g + 4h + j: the halves change places between the two lanes of a
+  // query when they are used (8-byte loads in the scores' own order touch
+  // every line of the mask twice as often).
+  auto mask_vals = [&](int kb, MaskBlock& mk) {
+    if (kb + 32 <= a.skv) {  // (wave-uniform)
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int kk = kb + 8 * g + 4 * h;
-      if (mrow && a.mask_vec && kk + 4 <= a.skv) {
-        mk[g] = *(const half4v*)(mrow + kk);
-      } else {
+      for (int x = 0; x < 2; ++x) mk.v[x] = *(const int4u*)(mrow + kb + 16 * h + 8 * x);
+    } else {
+      _Float16 e[16];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) mk[g][j] = (mrow && kk + j < a.skv) ? mrow[kk + j] : (_Float16)0.f;
-      }
+      for (int i = 0; i < 16; ++i) e[i] = mrow[min(kb + 16 * h + i, a.skv - 1)];
+      __builtin_memcpy(mk.v, e, 32);
     }
   };
 
   // The group of keys from kb on, its K rows at `rows` in LDS.  EDGE: some
   // of the keys may be past the sequence or the causal limit.
-  auto group = [&](auto EDGE_, int kb, const char* rows, half4v (&mk)[MASK ? NB : 1][4]) {
+  auto group = [&](auto EDGE_, int kb, const char* rows, const MaskBlock (&mk)[MASK ? NB : 1]) {
     constexpr int N = NB;
     constexpr bool SCALED = decltype(EDGE_)::value;  // scores multiplied by a.c before the maximum
     // S: D[key][query], lane holds query lane%32, keys 8g + 4h + j of each
@@ -330,12 +344,24 @@ __global__ __launch_bounds__(64 * QG * KS, (AttnShape<D, QG, KS, MASK>::WPE)) vo
     }
     if constexpr (SCALED) {
 #pragma unroll
-      for (int n = 0; n < N; ++n)
+      for (int n = 0; n < N; ++n) {
+        half4v me[4];  // by the g of the scores' keys
+        if constexpr (MASK) {
+#pragma unroll
+          for (int x = 0; x < 2; ++x) {
+            const int4v v = mk[n].v[x];
+            const auto e0 = __builtin_amdgcn_permlane32_swap(v[0], v[2], false, false);
+            const auto e1 = __builtin_amdgcn_permlane32_swap(v[1], v[3], false, false);
+            me[x] = __builtin_bit_cast(half4v, uint2v{(uint32_t)e0[0], (uint32_t)e1[0]});
+            me[2 + x] = __builtin_bit_cast(half4v, uint2v{(uint32_t)e0[1], (uint32_t)e1[1]});
+          }
+        }
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
           s[n][i] *= a.c;
-          if constexpr (MASK) s[n][i] = fmaf((float)mk[n][i >> 2][i & 3], kLog2e, s[n][i]);
+          if constexpr (MASK) s[n][i] = fmaf((float)me[i >> 2][i & 3], kLog2e, s[n][i]);
         }
+      }
       if (kb + N * 32 > min(a.skv, q0 + a.causal_off + 1)) {  // (wave-uniform)
         const int last = min(a.skv - 1, qme + a.causal_off) - kb - 4 * h;
 #pragma unroll
@@ -400,8 +426,6 @@ __global__ __launch_bounds__(64 * QG * KS, (AttnShape<D, QG, KS, MASK>::WPE)) vo
   // takes the loads of stage c + 1 while stage c is computed.  The first two
   // stages are issued together.  (One stage: its loads wait until every wave
   // is done with it, and only the other workgroup of the CU covers them.)
-  if (nchunk > 0) issue(0, 0);
-  if (ST == 2 && nchunk > 1) issue(1, 1);
   auto stage_in = [&](int c) {
     if (ST == 1 && c > 0) {
       barrier_before_refill();
@@ -419,7 +443,24 @@ __global__ __launch_bounds__(64 * QG * KS, (AttnShape<D, QG, KS, MASK>::WPE)) vo
   // the waves meet at the barriers), then the rest.
   int nfull = 0;
   if constexpr (!MASK) nfull = max(0, min(a.skv, qb0 + a.causal_off + 1) / KC);
-  half4v mk[MASK ? GPC : 1][MASK ? NB : 1][4];
+  // A stage's mask entries are loaded one stage ahead (before that stage's K
+  // and V: loads return in order), so their latency passes under a stage's
+  // MFMAs.
+  MaskBlock mk[MASK ? GPC : 1][MASK ? NB : 1], mk_next[MASK ? GPC : 1][MASK ? NB : 1];
+  auto load_mask = [&](int c, auto& m) {
+    if constexpr (MASK) {
+#pragma unroll
+      for (int g = 0; g < GPC; ++g)
+#pragma unroll
+        for (int n = 0; n < NB; ++n) {
+          const int kb = c * KC + ((g * KS + kh) * NB + n) * 32;
+          if (kb < wkend) mask_vals(kb, m[g][n]);
+        }
+    }
+  };
+  load_mask(0, mk);
+  if (nchunk > 0) issue(0, 0);
+  if (ST == 2 && nchunk > 1) issue(1, 1);
   int c = 0;
   for (; c < min(nfull, nchunk); ++c) {
     stage_in(c);
@@ -432,21 +473,19 @@ __global__ __launch_bounds__(64 * QG * KS, (AttnShape<D, QG, KS, MASK>::WPE)) vo
   }
   for (; c < nchunk; ++c) {
     stage_in(c);
-    if constexpr (MASK) {  // before the next stage's loads: loads return in order
-#pragma unroll
-      for (int g = 0; g < GPC; ++g)
-#pragma unroll
-        for (int n = 0; n < NB; ++n) {
-          const int kb = c * KC + ((g * KS + kh) * NB + n) * 32;
-          if (kb < wkend) mask_vals(kb, mk[g][n]);
-        }
-    }
+    load_mask(c + 1, mk_next);
     stage_out(c);
 #pragma unroll
     for (int g = 0; g < GPC; ++g) {
       const int row = (g * KS + kh) * NB * 32;
       if (c * KC + row < wkend)
         group(std::true_type{}, c * KC + row, stage_at(c) + row * RB, mk[MASK ? g : 0]);
+    }
+    if constexpr (MASK) {
+#pragma unroll
+      for (int g = 0; g < GPC; ++g)
+#pragma unroll
+        for (int n = 0; n < NB; ++n) mk[g][n] = mk_next[g][n];
     }
   }
 

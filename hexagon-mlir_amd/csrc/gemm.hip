@@ -208,7 +208,8 @@ hipError_t launch_fast(const GemmProblem& p, int tile, const KArgs& k, hipStream
 
 // Tile and K slices of a GEMM: the pair with the least estimated time.  Per
 // 64-deep K-step a tile alone on its CU takes `lat` us (few CUs busy: the
-// loads' latency and its own MFMAs) and, with every CU busy, `thr` us of its CU (memory contention and the power limit slow it), `epi` us for
+// loads' latency and its own MFMAs) and, with every CU busy, `thr` us of its
+// CU (memory contention and the power limit slow it), `epi` us for
 // its epilogue; per_cu workgroups share a CU.  Splitting K over s workgroups
 // puts short outputs on more CUs and costs 1.0 + 0.6 s us of fix-up round
 // trips plus the partial tiles' traffic.  Constants fitted to every tile and

@@ -389,12 +389,43 @@ bool slices(const Tensor& t, int64_t& ld, int64_t& slice) {
          (t.size(d - 2) - 1) * ld + t.size(d - 1) <= int64_t(1) << 30;
 }
 
-// attention(q, k, v, scale or None, causal): no mask, no out
+// An additive fp16 mask with q's leading dimensions (or 1 in their place, or
+// none of the outer ones): rows ld apart, `group` query slices a mask slice, those `slice` apart.
+bool mask_slices(const Tensor& m, const Tensor& q, int64_t Skv, int64_t& ld, int64_t& slice, int64_t& group) {
+  const int64_t r = q.dim(), off = r - m.dim();
+  if (m.scalar_type() != at::kHalf || off < 0 || off > r - 2 || m.size(-1) != Skv || m.size(-2) != q.size(-2) ||
+      (m.stride(-1) != 1 && Skv > 1) || (uintptr_t)m.data_ptr() % 2)
+    return false;
+  ld = m.stride(-2);
+  slice = 0;
+  group = 1;
+  int64_t next = -1;  // stride the next outer dimension must have
+  bool broadcast = false;
+  for (int64_t i = r - 3; i >= 0; --i) {
+    const int64_t sz = i < off ? 1 : m.size(i - off);
+    if (sz != 1 && sz != q.size(i)) return false;
+    if (q.size(i) == 1) continue;
+    const int64_t st = sz == 1 ? 0 : m.stride(i - off);
+    if (st == 0 && next < 0) {  // (the innermost ones only)
+      group *= q.size(i);
+      broadcast = true;
+      continue;
+    }
+    if (st <= 0 || (next >= 0 && st != next)) return false;
+    if (next < 0) slice = st;
+    next = st * q.size(i);
+  }
+  if (next < 0 && broadcast) group = 1;  // one slice for all
+  return ld >= Skv;
+}
+
+// attention(q, k, v, scale or None, causal, mask or None, out or None)
 PyObject* op_attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  NOT_PLAIN_UNLESS(n == 5);
+  NOT_PLAIN_UNLESS(n == 7);
   Operands in;
-  const Tensor *q = in.get(args[0]), *k = in.get(args[1]), *v = in.get(args[2]);
+  const Tensor *q = in.get(args[0]), *k = in.get(args[1]), *v = in.get(args[2]), *m = in.get(args[5], true),
+               *o = in.get(args[6], true);
   NOT_PLAIN_UNLESS(in.ok && half_type(*q) && k->scalar_type() == q->scalar_type() &&
                    v->scalar_type() == q->scalar_type());
   const int64_t r = q->dim();
@@ -408,11 +439,16 @@ PyObject* op_attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
   NOT_PLAIN_UNLESS(scale > 0 && std::isfinite((float)scale) && causal >= 0 && causal <= 2);
   int64_t ldq, ldk, ldv, sq, sk, sv;
   NOT_PLAIN_UNLESS(slices(*q, ldq, sq) && slices(*k, ldk, sk) && slices(*v, ldv, sv));
-  const Tensor out = like(*q, q->sizes());
+  int64_t ldm = 0, sm = 0, mg = 1;
+  NOT_PLAIN_UNLESS(!m || mask_slices(*m, *q, Skv, ldm, sm, mg));
+  int64_t ldo = D, so = S * D;
+  NOT_PLAIN_UNLESS(!o || (o->sizes() == q->sizes() && o->scalar_type() == q->scalar_type() && slices(*o, ldo, so) &&
+                          (o->is_contiguous() || (!bf16(*q) && (D == 64 || D == 128)))));
+  const Tensor out = o ? *o : like(*q, q->sizes());
   void* s = in.stream();
   return result(unlocked([&] {
                   return hxmi_attention_ex(bf16(*q), ptr(q), ptr(k), ptr(v), ptr(&out), q->numel() / (S * D), S, Skv, D,
-                                           ldq, ldk, ldv, D, sq, sk, sv, S * D, H / Hkv, nullptr, 0, 0, 1, (int)causal,
+                                           ldq, ldk, ldv, ldo, sq, sk, sv, so, H / Hkv, ptr(m), ldm, sm, mg, (int)causal,
                                            (float)scale, s);
                 }),
                 out);

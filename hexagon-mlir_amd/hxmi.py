@@ -617,16 +617,14 @@ def _mask_slices(mask: torch.Tensor, lead: tuple, S: int, Skv: int) -> tuple[tor
 
 def _fused_attention_ok(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float,
                         out: Optional[torch.Tensor]) -> bool:
-    """Whether attention() runs the fused kernel.  fp16 at head dims 64 and
-    128 always does; the others where the three steps take nothing more: at
+    """Whether attention() runs the fused kernel where its own test (fp16 at
+    head dims 64 and 128) fails: where the three steps take nothing more, at
     least one key, K / V slices of at most 2 GiB, a finite scale, operands on
     the 16-byte grid and an out whose rows take the kernel's 8-byte stores."""
     D = q.shape[-1]
     if q.dtype not in (torch.float16, torch.bfloat16) or k.dtype != q.dtype or v.dtype != q.dtype \
             or v.shape[-1] != D or D % 8 or not 8 <= D <= 128 or not scale > 0:
         return False
-    if q.dtype == torch.float16 and D in (64, 128):
-        return True
     S, Skv = q.shape[-2], k.shape[-2]
     if not 0 < Skv < 1 << 30 or S >= 1 << 30 or scale == float("inf"):
         return False
@@ -647,10 +645,9 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional
     query + S_kv - S.  fp16 and bf16 with D a multiple of 8 up to 128 and scale > 0 run the fused kernel
     (hxmi_attention_ex); every other case (other head dims, v of another width) runs the reference's three
     steps as bmm(Q, K^T) -> softmax (with the mask and causal rule: hxmi_softmax_masked_*) -> bmm(P, V)."""
-    if out is None and mask is None:
-        y = _ops.attention(q, k, v, scale, causal)
-        if y is not None:
-            return y
+    y = _ops.attention(q, k, v, scale, causal, mask, out)
+    if y is not None:
+        return out if out is not None else y
     if scale is None:
         scale = q.shape[-1] ** -0.5
     S, D = q.shape[-2:]
@@ -665,7 +662,8 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional
     q3 = q.reshape(-1, S, D)
     k3 = k.reshape(-1, Skv, D)
     v3 = v.reshape(-1, Skv, v.shape[-1])
-    if _fused_attention_ok(q, k, v, scale, out):
+    if (q.dtype == torch.float16 and D in (64, 128) and v.shape[-1] == D and k.dtype == v.dtype == q.dtype
+            and scale > 0) or _fused_attention_ok(q, k, v, scale, out):
         _require_gpu(q3, k3, v3)
         q3, k3, v3 = (t if t.stride(-1) == 1 and t.stride(1) % 8 == 0 and t.stride(0) % 8 == 0
                       and t.data_ptr() % 16 == 0 else t.contiguous() for t in (q3, k3, v3))

@@ -361,6 +361,22 @@ def test_attention_causal_block_orders(pkg, dev, bh, s):
     _check_nan_tol(out, ref.sdpa(np32(q), np32(k), np32(v), 0.125, causal=1), RMS[torch.float16])
 
 
+@pytest.mark.parametrize("off", [0, 3])
+@pytest.mark.parametrize("cfg,s,skv,d", [(41, 130, 31, 64), (42, 129, 300, 64), (22, 65, 289, 128), (14, 33, 545, 64),
+                                         (14, 31, 385, 128), (22, 1, 3, 64)])
+def test_attention_mask_tails(pkg, dev, knobs, cfg, s, skv, d, off):
+    """Mask rows that start anywhere, key counts around the 32-key block and
+    the stages, the mask of every query slice its own; rows past the last
+    query and keys past the last one lie outside the mask's storage."""
+    q, k, v = uniform((2, 3, s, d), 91), uniform((2, 3, skv, d), 92), uniform((2, 3, skv, d), 93)
+    full = normal((2, 3, s, skv + off), 94, 4.0)
+    m = full.cuda()[..., off:]
+    knobs(attn_cfg=cfg)
+    out = pkg.attention(q.cuda(), k.cuda(), v.cuda(), 0.125, mask=m).cpu()
+    exp = ref.sdpa(np32(q), np32(k), np32(v), 0.125, mask=np32(full[..., off:]))
+    assert ref.max_err_vs_scale(np32(out), exp) <= TOL
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_attention_three_step_value_width(pkg, dev, dtype):
     """A value width other than the head dim stays on the three steps: mask,

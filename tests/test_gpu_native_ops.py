@@ -29,6 +29,13 @@ def calls(pkg, dev):
     q, k, v = (qkv[:, :, i].transpose(1, 2) for i in range(3))  # [2, 4, 50, 64], heads 64 apart
     one = [t[:1] for t in (q, k, v)]
     kx = n(dev, 2, 1, 50, 64, seed=5).expand(2, 4, 50, 64)
+    q3 = n(dev, 2, 3, 4, 50, 64, seed=12)
+    masks = [(n(dev, *sh, seed=13), True) for sh in
+             ((1, 1, 1, 50, 50), (2, 1, 1, 50, 50), (2, 3, 1, 50, 50), (2, 3, 4, 50, 50))]
+    masks += [(n(dev, *sh, seed=13), False) for sh in ((1, 3, 1, 50, 50), (1, 1, 4, 50, 50), (2, 1, 4, 50, 50))]
+    masks += [(n(dev, *sh, seed=13), True) for sh in ((1, 50, 50), (1, 1, 50, 50))]
+    masks += [(n(dev, *sh, seed=13), False) for sh in ((4, 50, 50), (3, 1, 50, 50))]
+    masks += [(n(dev, 2, 3, 1, 50, 64, seed=13)[..., 7:57], True), (n(dev, 2, 3, 1, 50, 50) > 0, False)]
     s, g = n(dev, 64, 96, 40, seed=6), n(dev, 40, seed=7)
     wq = torch.randint(-127, 128, (96, 64), dtype=torch.int8, generator=torch.Generator().manual_seed(8)).to(dev)
     sc = (torch.rand(96, generator=torch.Generator().manual_seed(9)) * 9e-3 + 1e-3).half().to(dev)
@@ -70,7 +77,12 @@ def calls(pkg, dev):
         ("attention grouped bf16", True, lambda: pkg.attention(q.bfloat16().contiguous(), kx[:, :1].bfloat16(),
                                                                kx[:, 1:2].bfloat16())),
         ("attention negative scale", False, lambda: pkg.attention(*one, -0.2)),
-        ("attention masked", False, lambda: pkg.attention(*one, mask=n(dev, 50, 50))),
+        ("attention masked", True, lambda: pkg.attention(*one, mask=n(dev, 50, 50))),
+        ("attention out", True, lambda: pkg.attention(*one, out=out(1, 4, 50, 64))),
+        ("attention padded out", True, lambda: pkg.attention(*one, out=out(1, 4, 50, 72)[..., 8:])),
+        ("attention out off the grid", False, lambda: pkg.attention(*one, out=out(1, 4, 50, 72)[..., 4:68])),
+        *((f"attention mask of {tuple(m.shape)} {m.stride()}", plain, lambda m=m: pkg.attention(q3, q3, q3, mask=m))
+          for m, plain in masks),
     ]
 
 
