@@ -1,12 +1,14 @@
-// Row reductions: RMSNorm and (scaled) softmax, one wave64 per row.
+// Row reductions: RMSNorm and (scaled) softmax, one wave64 per row (several
+// for the long rows of RMSNorm).
 //
 // The reference turns these into HVX split reductions (a 32-wide partial
 // accumulator generic plus linalg.reduce, SplitReductionUtils.cpp,
-// TilingPass.cpp:261-289) over VTCM tiles.  On CDNA the row lives in the
-// registers of one wave: 16-byte loads (or 2-byte loads for unaligned rows)
-// spread the row across the 64 lanes, the reduction is a butterfly over
-// lanes, and every element is read from HBM once and written once.  All
-// arithmetic is fp32.
+// TilingPass.cpp:261-289) over VTCM tiles.  On CDNA the row lives in
+// registers: 16-byte loads (2-byte ones for softmax) spread it across the
+// lanes, the reduction is a butterfly over lanes, and every element is read
+// from HBM once and written once.  All arithmetic is fp32.
+#include <type_traits>
+
 #include "hxmi_common.h"
 #include "hxmi_internal.h"
 
@@ -45,21 +47,30 @@ __device__ __forceinline__ int4v pack8(const float* f) {
 // (the normalised value is rounded to the I/O type before the weight multiply,
 // as in the HF LlamaRMSNorm forward the TinyLlama benchmark runs)
 
-// Row held in registers: CPL 16-byte chunks per lane (cols <= 512 * CPL).
-template <typename T, int CPL>
-__global__ __launch_bounds__(128) void rmsnorm_vec(RArgs a) {
-  const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * 2 + (threadIdx.x >> 6);
+// Row held in registers: CPL 16-byte chunks per lane of the WPR waves that
+// share it (cols < 512 * CPL * WPR + 8).  GRID: rows on the 16-byte grid and
+// whole chunks; otherwise the accesses are as wide but start anywhere, and
+// the cols % 8 elements left over go one to a lane.
+typedef int int4u __attribute__((ext_vector_type(4), aligned(2)));
+
+template <typename T, int CPL, int WPR, bool GRID>
+__global__ __launch_bounds__(WPR == 1 ? 128 : 64 * WPR) void rmsnorm_vec(RArgs a) {
+  using V = std::conditional_t<GRID, int4v, int4u>;
+  const int lane = WPR == 1 ? threadIdx.x & 63 : threadIdx.x;
+  const int64_t row = WPR == 1 ? (int64_t)blockIdx.x * 2 + (threadIdx.x >> 6) : (int64_t)blockIdx.x;
   if (row >= a.rows) return;
-  const int nch = a.cols >> 3;
-  const __amdgpu_buffer_rsrc_t rx = make_rsrc(a.x + row * a.ldx * 2, 0x7fffffff);
+  const int nch = a.cols >> 3, left = GRID ? 0 : a.cols & 7;
+  const char* xrow = a.x + row * a.ldx * 2;
+  const __amdgpu_buffer_rsrc_t rx = make_rsrc(xrow, (uint32_t)a.cols * 2);
   int4v v[CPL];
 #pragma unroll
   for (int i = 0; i < CPL; ++i) {
-    const int c = lane + 64 * i;
-    v[i] = load16(rx, c < nch ? (uint32_t)c * 16 : kOOB);
+    const int c = lane + 64 * WPR * i;
+    if constexpr (GRID) v[i] = load16(rx, c < nch ? (uint32_t)c * 16 : kOOB);  // (zeros, and no branch)
+    else v[i] = c < nch ? (int4v)*(const V*)(xrow + (int64_t)c * 16) : int4v{};
   }
-  float ss = 0.f;
+  const T last = lane < left ? ((const T*)xrow)[nch * 8 + lane] : (T)0.f;
+  float ss = (float)last * (float)last;
 #pragma unroll
   for (int i = 0; i < CPL; ++i) {
     float f[8];
@@ -68,23 +79,35 @@ __global__ __launch_bounds__(128) void rmsnorm_vec(RArgs a) {
     for (int e = 0; e < 8; ++e) ss += f[e] * f[e];
   }
   ss = wave_sum_dpp(ss);
+  if constexpr (WPR > 1) {
+    __shared__ float part[WPR];
+    part[threadIdx.x >> 6] = ss;  // (every lane holds the sum)
+    __syncthreads();
+    ss = 0.f;
+#pragma unroll
+    for (int w = 0; w < WPR; ++w) ss += part[w];
+  }
   const float r = __builtin_amdgcn_rsqf(ss / (float)a.cols + a.eps);
   char* yrow = a.y + row * a.ldy * 2;
 #pragma unroll
   for (int i = 0; i < CPL; ++i) {
-    const int c = lane + 64 * i;
+    const int c = lane + 64 * WPR * i;
     if (c < nch) {
       float f[8], gf[8];
       unpack8<T>(v[i], f);
-      unpack8<T>(*(const int4v*)(a.g + (int64_t)c * 16), gf);
+      unpack8<T>((int4v)*(const V*)(a.g + (int64_t)c * 16), gf);
 #pragma unroll
       for (int e = 0; e < 8; ++e) f[e] = gf[e] * (float)(T)(f[e] * r);
-      *(int4v*)(yrow + (int64_t)c * 16) = pack8<T>(f);
+      *(V*)(yrow + (int64_t)c * 16) = (V)pack8<T>(f);
     }
+  }
+  if (lane < left) {
+    const int c = nch * 8 + lane;
+    ((T*)yrow)[c] = (T)((float)((const T*)a.g)[c] * (float)(T)((float)last * r));
   }
 }
 
-// Any width / alignment: two passes over the row, element at a time.
+// Any width: two passes over the row, element at a time.
 template <typename T>
 __global__ __launch_bounds__(128) void rmsnorm_any(RArgs a) {
   const int lane = threadIdx.x & 63;
@@ -209,20 +232,49 @@ RArgs make_args(const RowProblem& p) {
   return a;
 }
 
+// The waves of a row: as many as have a chunk for each lane, up to eight,
+// while all rows' waves fit the chip at once (32 a CU); fewer for more rows,
+// which then only wait on each other.  us, graph replays on MI355X:
+//   512 x 2048     1 / 2 / 4 / 8 waves 3.1 / 2.9 / 2.7 / 2.8;  4096 x 2048  8.5 / 8.2 / 8.5 / 9.7
+//   512 x 4096     4.4 / 4.0 / 3.7 / 3.7;  2048 x 4096  8.9 / 8.4 / 8.2 / 8.4;  4096 x 4096  12.9 / 12.1 / 14.3 / 14.0
+//   512 x 8192     4 / 8 waves 5.3 / 5.0;  2048 x 8192  12.6 / 14.6;  4096 x 8192  26.6 / 25.0
+// (4096 x 8192 in two passes of 2-byte loads, as all widths over 4096 and
+// odd ones ran before: 94.7; 512 x 8192 49.2; 4096 x 2049 27.2).  Rows off the
+// 16-byte grid, whose waves share lines, run one wave a row where many rows
+// allow it (4096 x 2049: 9.5, two waves 10.9; 4096 x 4097: 14.6, two 19.3).
+template <typename T, bool GRID>
+void rms_launch_vec(const RArgs& a, hipStream_t stream) {
+  auto rows = [&](auto CPL, auto WPR) {
+    constexpr int W = decltype(WPR)::value;
+    const dim3 grid((unsigned)(W == 1 ? (a.rows + 1) / 2 : a.rows)), block(W == 1 ? 128 : 64 * W);
+    hipLaunchKernelGGL((rmsnorm_vec<T, decltype(CPL)::value, W, GRID>), grid, block, 0, stream, a);
+  };
+  constexpr std::integral_constant<int, 1> one;
+  constexpr std::integral_constant<int, 2> two;
+  constexpr std::integral_constant<int, 4> four;
+  constexpr std::integral_constant<int, 8> eight;
+  const int64_t nch = a.cols / 8, most = 8192 / a.rows;  // waves a row that fit at once
+  if (nch <= 64) rows(one, one);
+  else if (nch <= 128) most >= 2 ? rows(one, two) : rows(two, one);
+  else if (nch <= 256) most >= 4 ? rows(one, four) : GRID ? rows(two, two) : rows(four, one);
+  else if (nch <= 512) {
+    if (most >= 8) rows(one, eight);
+    else if (GRID) most >= 4 ? rows(two, four) : rows(four, two);
+    else rows(eight, one);
+  } else if (nch <= 1024) most >= 8 ? rows(two, eight) : rows(four, four);
+  else if (nch <= 2048) rows(four, eight);
+  else rows(eight, eight);
+}
+
 template <typename T>
 hipError_t rms_launch(const RowProblem& p, hipStream_t stream) {
   const RArgs a = make_args(p);
-  // two rows (waves) a workgroup: [512, 2048] then spans 256 workgroups, one
-  // per CU (2.96 -> 2.88 us against four rows a workgroup; one row: 3.01)
-  const dim3 grid((unsigned)((p.rows + 1) / 2)), block(128);
-  const bool vec = (p.cols % 8 == 0) && (p.ldx % 8 == 0) && (p.ldy % 8 == 0) && ((uintptr_t)p.x % 16 == 0) &&
-                   ((uintptr_t)p.y % 16 == 0) && ((uintptr_t)p.g % 16 == 0) && p.ldx * 2 * 4 < (1ll << 31);
-  const int64_t nch = p.cols / 8;
-  if (vec && nch <= 64) hipLaunchKernelGGL((rmsnorm_vec<T, 1>), grid, block, 0, stream, a);
-  else if (vec && nch <= 128) hipLaunchKernelGGL((rmsnorm_vec<T, 2>), grid, block, 0, stream, a);
-  else if (vec && nch <= 256) hipLaunchKernelGGL((rmsnorm_vec<T, 4>), grid, block, 0, stream, a);
-  else if (vec && nch <= 512) hipLaunchKernelGGL((rmsnorm_vec<T, 8>), grid, block, 0, stream, a);
-  else hipLaunchKernelGGL((rmsnorm_any<T>), grid, block, 0, stream, a);
+  const bool grid16 = (p.cols % 8 == 0) && (p.ldx % 8 == 0) && (p.ldy % 8 == 0) && ((uintptr_t)p.x % 16 == 0) &&
+                      ((uintptr_t)p.y % 16 == 0) && ((uintptr_t)p.g % 16 == 0);
+  if (p.cols >= 8 * 4096 + 8)
+    hipLaunchKernelGGL((rmsnorm_any<T>), dim3((unsigned)((p.rows + 1) / 2)), dim3(128), 0, stream, a);
+  else if (grid16) rms_launch_vec<T, true>(a, stream);
+  else rms_launch_vec<T, false>(a, stream);
   return hipGetLastError();
 }
 

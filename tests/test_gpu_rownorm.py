@@ -23,6 +23,27 @@ def test_rmsnorm(pkg, dev, rows, cols):
     assert np.max(np.abs(y.astype(np.float32) - hf) / np.maximum(np.abs(hf), 1e-3)) <= 2 ** -9
 
 
+@pytest.mark.parametrize("rows", [1, 1030, 2050, 4100])  # each side of the lines between waves a row
+@pytest.mark.parametrize("cols", [7, 512, 519, 1016, 1031, 2048, 2055, 4088, 4103, 8199, 16391, 32775, 32776])
+def test_rmsnorm_row_shapes(pkg, dev, rows, cols):
+    """Whole and odd widths at the edges of the row shapes, on and off the
+    16-byte grid, nothing written past the rows."""
+    rows = min(rows, 2 ** 25 // cols)
+    g = (1 + normal((cols,), 2, 0.02, torch.float32)).half()
+    picks = sorted({0, rows // 2, rows - 1})
+    for off in (0, 5):
+        x = torch.empty(rows * cols + 16, dtype=torch.float16, device=dev).normal_(
+            generator=torch.Generator(dev).manual_seed(cols))[off:off + rows * cols].view(rows, cols)
+        buf = torch.full((rows * cols + 16,), 7.0, dtype=torch.float16, device=dev)
+        y = pkg.rms_norm(x, g.to(dev), 1e-5, out=buf[off:off + rows * cols].view(rows, cols))
+        assert torch.all(buf[:off] == 7.0) and torch.all(buf[off + rows * cols:] == 7.0)
+        hf = ref.rms_norm_hf(x[picks].cpu().numpy(), g.numpy(), 1e-5).astype(np.float32)
+        err = np.abs(np32(y[picks].cpu()) - hf)
+        assert np.max(err / np.maximum(np.abs(hf), 1e-3)) <= 2 ** -9  # (one ulp, as above)
+        want = x.float() * torch.rsqrt(x.float().square().mean(1, keepdim=True) + 1e-5) * g.to(dev).float()
+        assert (y.float() - want).abs().max() <= 2 ** -9 * want.abs().max()
+
+
 def test_rmsnorm_reference_test_shape_uniform(pkg, dev):
     # test_rms_norm.py:19-20, 65-67: 127 x 513, rand inputs and weights
     x = uniform((127, 513), 3, 0, 1)
