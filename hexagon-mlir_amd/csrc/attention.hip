@@ -36,6 +36,10 @@ int pick_cfg(const AttnProblem& p) {
   const bool masked64 = p.mask && p.d <= 64;
   if (wg128 >= (p.causal ? 320 : few_keys ? 192 : masked64 ? 320 : 144))
     return p.d <= 64 && !few_keys && !p.mask ? 42 : 41;
+  // (64-192 keys at head dims over 64: the merge of four key splits takes as
+  // long as the keys; 4 x 157 causal 6.4 us against 7.2, 32 x 155 full 7.4
+  // against 7.5, 64 x 201 8.3 against 7.6)
+  if (p.d > 64 && p.skv <= 192) return 22;
   return wg64 >= (few_keys ? 144 : p.causal ? 288 : 192) ? 22 : 14;
 }
 

@@ -168,16 +168,17 @@ __device__ __forceinline__ int v_off(int r, int c) {
 // Head dims up to 64 run in LDS rows of D = 64, others in rows of 128.  K and
 // V pass through ST LDS stages of KC keys, 64 KB in all (two workgroups a
 // CU); a wave takes NB 32-key blocks at a time (a group), GPC groups a stage.
-template <int D, int QG, int KS, bool MASK>
+// DEEP: two stages also where one fills 64 KB (one workgroup a CU).
+template <int D, int QG, int KS, bool MASK, bool DEEP>
 struct AttnShape {
   static constexpr int NT = 64 * QG * KS;
   static constexpr int KC = D == 64 || KS == 4 ? 128 : 64;
-  static constexpr int ST = KC * D > 8192 ? 1 : 2;
+  static constexpr int ST = KC * D > 8192 && !DEEP ? 1 : 2;
   static constexpr int NB = KC / 32 / KS >= 2 && !MASK ? 2 : 1;  // (two blocks' mask entries would not fit)
   static constexpr int GPC = KC / 32 / KS / NB;
   static constexpr int CHUNK = KC * 2 * D;    // bytes of K (and of V) per stage: 16 or 32 KB
   static constexpr int NV = D / 32 * 16 + 2;  // floats per lane in the key-split merge
-  static constexpr int WPE = QG * KS / 2;     // waves per SIMD that two workgroups a CU make
+  static constexpr int WPE = QG * KS / (DEEP ? 4 : 2);  // waves per SIMD that one / two workgroups a CU make
   static constexpr bool ok = NT <= 1024 && (KS - 1) * QG * NV * 64 * 4 <= 2 * ST * CHUNK;
 };
 
@@ -189,9 +190,9 @@ struct MaskBlock {
 
 // DT: 32-wide output tiles computed (fewer than D / 32 for head dims 72-96).
 // PART: the head dim a.d is below D; rows fill up with zeros.
-template <typename T, int D, int DT, bool PART, int QG, int KS, bool MASK>
-__global__ __launch_bounds__(64 * QG * KS, (AttnShape<D, QG, KS, MASK>::WPE)) void attention_fwd(AArgs a) {
-  using Sh = AttnShape<D, QG, KS, MASK>;
+template <typename T, int D, int DT, bool PART, int QG, int KS, bool MASK, bool DEEP>
+__global__ __launch_bounds__(64 * QG * KS, (AttnShape<D, QG, KS, MASK, DEEP>::WPE)) void attention_fwd(AArgs a) {
+  using Sh = AttnShape<D, QG, KS, MASK, DEEP>;
   static_assert(Sh::ok, "attention shape");
   constexpr int NW = QG * KS;
   constexpr int KC = Sh::KC, NB = Sh::NB, GPC = Sh::GPC, ST = Sh::ST;
@@ -539,9 +540,9 @@ __global__ __launch_bounds__(64 * QG * KS, (AttnShape<D, QG, KS, MASK>::WPE)) vo
   }
 }
 
-template <typename T, int D, int DT, bool PART, int QG, int KS>
+template <typename T, int D, int DT, bool PART, int QG, int KS, bool DEEP = false>
 hipError_t launch_cfg(AArgs a, const AttnProblem& p, bool mask, hipStream_t stream) {
-  if constexpr (!AttnShape<D, QG, KS, false>::ok) {
+  if constexpr (!AttnShape<D, QG, KS, false, DEEP>::ok) {
     return hipErrorNotSupported;
   } else {
     a.nqb = (int)((p.s + 32 * QG - 1) / (32 * QG));
@@ -550,9 +551,9 @@ hipError_t launch_cfg(AArgs a, const AttnProblem& p, bool mask, hipStream_t stre
     a.order = !p.causal ? ORDER_SLICES : (blocks <= 512 ? ORDER_PAIRED : ORDER_HEAVY);
     const dim3 grid((unsigned)blocks), block(64 * QG * KS);
     if (mask)
-      hipLaunchKernelGGL((attention_fwd<T, D, DT, PART, QG, KS, true>), grid, block, 0, stream, a);
+      hipLaunchKernelGGL((attention_fwd<T, D, DT, PART, QG, KS, true, DEEP>), grid, block, 0, stream, a);
     else
-      hipLaunchKernelGGL((attention_fwd<T, D, DT, PART, QG, KS, false>), grid, block, 0, stream, a);
+      hipLaunchKernelGGL((attention_fwd<T, D, DT, PART, QG, KS, false, DEEP>), grid, block, 0, stream, a);
     return hipGetLastError();
   }
 }
@@ -564,7 +565,13 @@ hipError_t launch_d(const AArgs& a, const AttnProblem& p, int cfg, hipStream_t s
   const bool m = p.mask != nullptr;
   switch (cfg) {
     case 41: return launch_cfg<T, D, DT, PART, 4, 1>(a, p, m, stream);
-    case 14: return launch_cfg<T, D, DT, PART, 1, 4>(a, p, m, stream);
+    case 14:
+      // One workgroup a CU at most: its loads need a second stage to pass
+      // under its MFMAs (2 x 1968 x 1968 causal, D 128: 22.9 -> 20.9 us, 16 x
+      // 458 10.5 -> 9.8); from 257 workgroups on two share a CU, which only
+      // one stage each allows (8 x 1132: 20.0 us, two stages 27.6).
+      if (D > 64 && p.bh * ((p.s + 31) / 32) <= 256) return launch_cfg<T, D, DT, PART, 1, 4, (D > 64)>(a, p, m, stream);
+      return launch_cfg<T, D, DT, PART, 1, 4>(a, p, m, stream);
     case 42: return launch_cfg<T, D, DT, PART, 4, 2>(a, p, m, stream);
     case 22: return launch_cfg<T, D, DT, PART, 2, 2>(a, p, m, stream);
     default: break;

@@ -361,6 +361,16 @@ def test_attention_causal_block_orders(pkg, dev, bh, s):
     _check_nan_tol(out, ref.sdpa(np32(q), np32(k), np32(v), 0.125, causal=1), RMS[torch.float16])
 
 
+@pytest.mark.parametrize("d", [80, 128])
+@pytest.mark.parametrize("bh,s,skv", [(64, 128, 129), (257, 32, 385), (2, 33, 640), (2, 33, 1), (43, 185, 256)])
+def test_attention_key_split_stages(pkg, dev, knobs, bh, s, skv, d):
+    """Four key-split waves at head dims over 64: two stages up to 256
+    workgroups, one beyond, with one key, whole stages and a key after one."""
+    knobs(attn_cfg=14)
+    q, k, v = uniform((bh, s, d), 141), uniform((bh, skv, d), 142), uniform((bh, skv, d), 143)
+    _check(pkg.attention(q.cuda(), k.cuda(), v.cuda(), 0.1).cpu(), q, k, v, 0.1)
+
+
 @pytest.mark.parametrize("off", [0, 3])
 @pytest.mark.parametrize("cfg,s,skv,d", [(41, 130, 31, 64), (42, 129, 300, 64), (22, 65, 289, 128), (14, 33, 545, 64),
                                          (14, 31, 385, 128), (22, 1, 3, 64)])
