@@ -1054,7 +1054,7 @@ struct TileShape {
 // flight while two or three workgroups still fit per CU.  Measured on the
 // TinyLlama block in sequence (weights not resident in L2): 91.0 -> 79.3 us;
 // four stages, at half the workgroups per CU, gave 87.1 us.
-// The tiles of at most 128 rows read their fragments three substeps ahead
+// The 4-wave tiles of at most 128 rows read their fragments three substeps ahead
 // (FD = 3): with one or two waves per SIMD and one to four MFMAs per wave
 // and substep, an LDS read issued one substep ahead had not returned by its
 // MFMA.  1024^3 NN on 64x64 tiles: 7.3 -> 6.3 us; the block's GEMMs and the
@@ -1081,6 +1081,10 @@ struct TileShape {
 // 100.8 us and NN 113.3 -> 102.1 on the 256x256 tile, gate/up 27.8 -> 25.2 us
 // on 128x192.  The 4-wave tiles of at most 128 rows are bound by latency
 // and keep 32x32x16, whose shorter substeps let them read further ahead.
+// The int8 tiles of one wave row convert each weight once, and their 80 KB of
+// LDS leave room for a second workgroup, which covers the first loads and the
+// epilogue: lm_head 896 -> 151936 at M = 256 98 us on 256x256 -> 86 on 128x256
+// (256x128 the same way: 91), M = 64 48.5 -> 40 on the tiles the plan takes.
 constexpr TileShape kTiles[TILE_COUNT] = {
     {256, 256, 128, 128, 64, 2},  // TILE_256x256
     {128, 256, 64, 128, 64, 3, false, 0, 3},   // TILE_128x256
