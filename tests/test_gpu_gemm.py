@@ -510,3 +510,18 @@ def test_hexkl_compat_matmul(pkg, dev):
     out = pkg.hexkl_matmul(act.to(dev), w.to(dev)).cpu()
     assert out.dtype == torch.float32
     assert np.max(np.abs(out.numpy() - ref.matmul(act.numpy(), w.numpy()))) <= 1e-2
+
+
+@pytest.mark.parametrize("left", range(1, 8))
+@pytest.mark.parametrize("off", [0, 3])  # rows of C on and off the 16-byte grid
+def test_gemm_last_columns_exact(pkg, dev, left, off):
+    """The last N % 8 columns of C, and nothing beyond them."""
+    m, n, k = 70, 64 + left, 64
+    g = torch.Generator().manual_seed(left)
+    a = torch.randint(-4, 5, (m, k), generator=g).half()
+    b = torch.randint(-4, 5, (n, k), generator=g).half()
+    buf = torch.full((m, 88), 7.0, dtype=torch.float16, device=dev)
+    pkg.gemm(a.to(dev), b.to(dev), b_layout="nt", out=buf[:, off:off + n])
+    got = buf.cpu()
+    assert torch.equal(got[:, off:off + n].float(), a.float() @ b.float().t())
+    assert torch.all(got[:, :off] == 7.0) and torch.all(got[:, off + n:] == 7.0)
