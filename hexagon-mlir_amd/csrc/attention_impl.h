@@ -233,16 +233,19 @@ __global__ __launch_bounds__(64 * QG * KS, (AttnShape<D, QG, KS, MASK, DEEP>::WP
     mrow = (const _Float16*)a.mask + ((int64_t)(bh / a.mask_group) * a.bm + (int64_t)min(qme, a.sq - 1) * a.ldm);
 
   // Q fragments of this wave's 32 queries (zero past the sequence).  The
-  // loads take no branch (an offset past the buffer reads zeros).
+  // loads take no branch (an offset past the buffer reads zeros).  The buffer
+  // starts at the wave's first row, so its 32-bit offsets span 32 rows (the
+  // host checks those) and a slice may be of any length.
   short8v qf[DS];
   {
-    const __amdgpu_buffer_rsrc_t rQ = make_rsrc(Q, 0x7fffffffu);
+    const int left = min(32, a.sq - q0), r = lane & 31;
+    const __amdgpu_buffer_rsrc_t rQ =
+        make_rsrc(Q + (int64_t)q0 * a.ldq * 2, left > 0 ? (uint32_t)(((left - 1) * a.ldq + a.d) * 2) : 0u);
+    const uint32_t row = (uint32_t)r * (uint32_t)a.ldq + h * 8;
 #pragma unroll
     for (int s = 0; s < DS; ++s)
       qf[s] = __builtin_bit_cast(
-          short8v, load16(rQ, qme < a.sq && !(PART && s * 16 + h * 8 >= a.d)
-                                  ? (uint32_t)(((int64_t)qme * a.ldq + s * 16 + h * 8) * 2)
-                                  : kOOB));
+          short8v, load16(rQ, r < left && !(PART && s * 16 + h * 8 >= a.d) ? (row + s * 16) * 2 : kOOB));
   }
 
   // Direct loads: wave w's load i fills LDS bytes [(i*NW + w) KB, +1 KB) of

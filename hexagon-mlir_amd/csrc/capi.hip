@@ -431,6 +431,8 @@ int attention_common(const char* name, int dtype, const void* q, const void* k, 
   REQUIRE(s_q < (1ll << 30) && s_kv < (1ll << 30), "%s: sequence too long", name);
   REQUIRE(((s_kv - 1) * ldk + d) * 2 <= (1ll << 31) && ((s_kv - 1) * ldv + d) * 2 <= (1ll << 31),
           "%s: one K or V slice must span at most 2 GiB", name);
+  REQUIRE((((s_q < 32 ? s_q : 32) - 1) * ldq + d) * 2 <= (1ll << 31), "%s: 32 rows of q must span at most 2 GiB",
+          name);
   if (mask) {
     REQUIRE(ldm >= s_kv && stride_m >= 0, "%s: mask row stride %lld below s_kv", name, (long long)ldm);
     REQUIRE(mask_group >= 1 && bh % mask_group == 0, "%s: mask_group %lld must divide bh", name,

@@ -667,6 +667,8 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional
         _require_gpu(q3, k3, v3)
         q3, k3, v3 = (t if t.stride(-1) == 1 and t.stride(1) % 8 == 0 and t.stride(0) % 8 == 0
                       and t.data_ptr() % 16 == 0 else t.contiguous() for t in (q3, k3, v3))
+        if (min(S, 32) - 1) * q3.stride(1) + D > 1 << 30:  # (a wave's 32 rows in one 2 GiB buffer)
+            q3 = q3.contiguous()
         if out is None:
             o = torch.empty((q3.shape[0], S, D), dtype=q.dtype, device=q.device)
         else:

@@ -308,7 +308,8 @@ int hxmi_quantize_int8_rows_f16(const void* W, int8_t* q, void* s, int64_t N, in
  *   O[i] = softmax(scale * Q[i] . K^T) . V  over s_kv keys,
  * Q/O [s_q, d], K/V [s_kv, d] row-major (leading dims ld*, slice strides
  * stride_*, elements), d = 64 or 128, scale > 0, fp32 softmax and accumulation,
- * no mask.
+ * no mask.  A K or V slice and any 32 consecutive rows of Q span at most 2 GiB;
+ * Q and O slices may be longer.
  * Replaces: tm_tensor.attention as LowerTmTensor.cpp:52-250 lowers it
  * (batch_matmul(Q, K^T) -> scale -> softmax -> batch_matmul(P, V), semantics
  * of qcom_hexagon_backend/test/Conversion/TmTensorToLinalg/SDPA.mlir:18-59)

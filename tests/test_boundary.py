@@ -182,6 +182,28 @@ def test_tuning_overrides_are_per_thread_and_restorable(pkg):
         pkg.set_tuning("no_such_knob", 1)
 
 
+def test_attention_rejects_rows_its_offsets_do_not_reach(pkg):
+    """A wave reads its 32 query rows through one buffer of at most 2 GiB, a
+    K or V slice through another: rows further apart are refused before
+    anything is launched, and named."""
+    lib = pkg.load_library()
+    P = 1 << 12  # aligned, never dereferenced: every call below fails a check first
+
+    def call(fn, *head, s_q=64, s_kv=64, d=64, ldq=64, ldk=64):
+        lds = (ldq, ldk, 64, 64)
+        tail = (0, 0, 0, 0) + ((0.125, None) if fn == "hxmi_attention_f16" else (1, None, 0, 0, 1, 0, 0.125, None))
+        return getattr(lib, fn)(*head, P, P, P, P, 1, s_q, s_kv, d, *lds, *tail)
+
+    for fn, head in (("hxmi_attention_f16", ()), ("hxmi_attention_ex_f16", ()), ("hxmi_attention_ex", (1,)),
+                     ("hxmi_attention_ex", (0,))):
+        assert call(fn, *head, ldq=(1 << 30) // 31 // 8 * 8) == 1, fn  # 31 of these and one row's 64 elements
+        assert "32 rows of q" in lib.hxmi_last_error().decode()
+        assert call(fn, *head, s_q=2, ldq=1 << 30) == 1, fn
+        assert "32 rows of q" in lib.hxmi_last_error().decode()
+        assert call(fn, *head, ldk=1 << 25) == 1, fn
+        assert "K or V slice" in lib.hxmi_last_error().decode()
+
+
 def test_plan_tile_applies_to_its_own_runs_only(pkg):
     from hexagon_mlir_amd.backend.graph import Plan
 

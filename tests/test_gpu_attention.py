@@ -351,6 +351,22 @@ def test_attention_fused_head_dims(pkg, dev, dtype, d, masked):
     _check_nan_tol(out, exp, RMS[dtype])
 
 
+@pytest.mark.parametrize("dtype,d", [(torch.float16, 64), (torch.float16, 128), (torch.bfloat16, 64),
+                                     (torch.bfloat16, 128), (torch.float16, 80), (torch.bfloat16, 40)])
+@pytest.mark.parametrize("s,ld", [(70, 1 << 25),  # a slice of 4.4 GiB, 32 rows of which stay within 2 GiB
+                                  (33, 3 << 24)])  # 32 rows of 2.9 GiB
+def test_attention_long_query_slices(pkg, dev, dtype, d, s, ld):
+    """Query rows so far apart that a slice passes 2 and 4 GiB: the same
+    results as from the same rows side by side."""
+    q, k, v = (uniform((1, n, d), 241 + i, dtype=dtype).to(dev) for i, n in enumerate((s, 200, 200)))
+    far = torch.empty((s - 1) * ld + d, dtype=dtype, device=dev).as_strided((1, s, d), (0, ld, 1))
+    far.copy_(q)
+    got = pkg.attention(far, k, v, causal=2)
+    assert torch.equal(got, pkg.attention(q, k, v, causal=2))
+    exp = ref.sdpa(*(np32(t.cpu()) for t in (q, k, v)), d**-0.5, causal=2)
+    _check_nan_tol(got.cpu(), exp, RMS[dtype])
+
+
 @pytest.mark.parametrize("bh,s", [(3, 200), (12, 700), (50, 512), (72, 512), (75, 512), (130, 512), (136, 512)])
 def test_attention_causal_block_orders(pkg, dev, bh, s):
     """Every query block is computed once whatever order the causal rule gives
