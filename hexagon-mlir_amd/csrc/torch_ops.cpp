@@ -71,12 +71,17 @@ struct Operands {
 bool half_type(const Tensor& t) { return t.scalar_type() == at::kHalf || t.scalar_type() == at::kBFloat16; }
 bool bf16(const Tensor& t) { return t.scalar_type() == at::kBFloat16; }
 
-// A 2-D view with unit last stride; its leading dimension.
-bool rows(const Tensor& t, int64_t& ld) {
-  if (t.dim() != 2 || (t.stride(1) != 1 && t.size(1) > 1)) return false;
-  ld = std::max<int64_t>({t.stride(0), t.size(1), 1});
+// Rows over the last two dimensions, with unit last stride and no elements in
+// common; their leading dimension (a single row may have any stride).
+bool lead(const Tensor& t, int64_t& ld) {
+  const int64_t d = t.dim(), stride = t.stride(d - 2), width = t.size(d - 1);
+  if ((t.stride(d - 1) != 1 && width > 1) || (t.size(d - 2) > 1 && stride < width)) return false;
+  ld = std::max<int64_t>({stride, t.size(d - 2) > 1 ? 1 : width, 1});
   return true;
 }
+
+// A 2-D view of such rows.
+bool rows(const Tensor& t, int64_t& ld) { return t.dim() == 2 && lead(t, ld); }
 
 // A contiguous vector of n elements.
 bool vec(const Tensor* t, int64_t n, at::ScalarType type) {
@@ -181,21 +186,21 @@ PyObject* op_bgemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const int epi = (int)PyLong_AsLong(args[3]);
   const double alpha = PyFloat_AsDouble(args[5]);
   if (PyErr_Occurred()) return nullptr;
-  const auto unit = [](const Tensor& t) { return t.stride(2) == 1 || t.size(2) <= 1; };
-  const auto lead = [](const Tensor& t) { return std::max<int64_t>({t.stride(1), t.size(2), 1}); };
+  int64_t lda, ldb, ldc;
   const int64_t batch = a->size(0), M = a->size(1), K = a->size(2), N = b->size(nt ? 1 : 2);
   const int64_t nout = epi == kEpiSiluMul ? N / 2 : N;
   const bool takes_bias = epi == kEpiBias || epi == kEpiBiasGelu;
-  NOT_PLAIN_UNLESS(unit(*a) && unit(*b) && b->size(0) == batch && b->size(nt ? 2 : 1) == K &&
+  NOT_PLAIN_UNLESS(lead(*a, lda) && lead(*b, ldb) && b->size(0) == batch && b->size(nt ? 2 : 1) == K &&
                    takes_bias == (bias != nullptr) && vec(bias, N, a->scalar_type()));
   NOT_PLAIN_UNLESS(!o || (o->dim() == 3 && o->size(0) == batch && o->size(1) == M && o->size(2) == nout &&
-                          o->scalar_type() == a->scalar_type() && unit(*o)));
+                          o->scalar_type() == a->scalar_type()));
   const Tensor out = o ? *o : like(*a, {batch, M, nout});
+  NOT_PLAIN_UNLESS(lead(out, ldc));
   const auto fn = bf16(*a) ? hxmi_bgemm_bf16 : hxmi_bgemm_f16;
   void* s = in.stream();
   return result(unlocked([&] {
-                  return fn(ptr(a), ptr(b), ptr(&out), ptr(bias), batch, M, N, K, lead(*a), lead(*b), lead(out),
-                            a->stride(0), b->stride(0), out.stride(0), nt, epi, (float)alpha, s);
+                  return fn(ptr(a), ptr(b), ptr(&out), ptr(bias), batch, M, N, K, lda, ldb, ldc, a->stride(0),
+                            b->stride(0), out.stride(0), nt, epi, (float)alpha, s);
                 }),
                 out);
   END_HANDLE_TH_ERRORS

@@ -182,13 +182,30 @@ def _require_gpu(*ts: Optional[torch.Tensor]) -> None:
             raise HxmiError(f"tensors on different devices: {dev} and {t.device}")
 
 
+def _own_rows(t: torch.Tensor) -> torch.Tensor:
+    """t, or a copy where its rows share elements: expanded rows, overlapping
+    windows.  The kernels take a row stride of at least a row."""
+    if t.dim() < 2 or (t.stride(-1) != 1 and t.size(-1) > 1):
+        return t  # (refused where it matters)
+    return t.contiguous() if t.size(-2) > 1 and t.stride(-2) < t.size(-1) else t
+
+
+def _lead(t: torch.Tensor, name: str) -> int:
+    """Row stride of the last two dims; a single row may have any."""
+    if t.size(-2) > 1:
+        if t.stride(-2) < t.size(-1):
+            raise HxmiError(f"the rows of {name} must not share elements (row stride {t.stride(-2)})")
+        return max(t.stride(-2), 1)
+    return max(t.stride(-2), t.size(-1), 1)
+
+
 def _rowmajor(t: torch.Tensor, name: str) -> int:
     """Leading dimension of a 2-D view with unit stride in the last dim."""
     if t.dim() != 2:
         raise HxmiError(f"{name} must be 2-D, got shape {tuple(t.shape)}")
     if t.stride(1) != 1 and t.size(1) > 1:
         raise HxmiError(f"{name} must have unit stride in its last dimension")
-    return max(t.stride(0), t.size(1), 1)
+    return _lead(t, name)
 
 
 def _vec(t: Optional[torch.Tensor], n: int, dtype: torch.dtype, name: str) -> Optional[torch.Tensor]:
@@ -310,6 +327,7 @@ def gemm(
         raise HxmiError(f"b_layout must be 'nn' or 'nt', got {b_layout!r}")
     if epilogue not in EPILOGUES:
         raise HxmiError(f"unknown epilogue {epilogue!r}")
+    a, b = _own_rows(a), _own_rows(b)
     lda, ldb = _rowmajor(a, "a"), _rowmajor(b, "b")
     M, K = a.shape
     nt = b_layout == "nt"
@@ -341,7 +359,7 @@ def _batched(t: torch.Tensor, name: str) -> tuple[int, int]:
         raise HxmiError(f"{name} must be 3-D, got shape {tuple(t.shape)}")
     if t.stride(2) != 1 and t.size(2) > 1:
         raise HxmiError(f"{name} must have unit stride in its last dimension")
-    return max(t.stride(1), t.size(2), 1), t.stride(0)
+    return _lead(t, name), t.stride(0)
 
 
 def bgemm(
@@ -364,6 +382,7 @@ def bgemm(
         raise HxmiError("bgemm takes fp16 or bf16 operands of one dtype")
     if epilogue not in EPILOGUES:
         raise HxmiError(f"unknown epilogue {epilogue!r}")
+    a, b = _own_rows(a), _own_rows(b)
     lda, sa = _batched(a, "a")
     ldb, sb = _batched(b, "b")
     batch, M, K = a.shape
@@ -422,6 +441,7 @@ def fold_rms_weight(w: torch.Tensor, g: torch.Tensor) -> torch.Tensor:
     if w.dim() != 2:
         raise HxmiError("fold_rms_weight takes a 2-D weight")
     N, K = w.shape
+    w = _own_rows(w)
     ldw = _rowmajor(w, "w")
     g = _vec(g, K, w.dtype, "g")
     out = torch.empty((N, K), dtype=w.dtype, device=w.device)
@@ -440,6 +460,7 @@ def quantize_int8(w: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     if w.dtype != torch.float16 or w.dim() != 2:
         raise HxmiError("quantize_int8 takes a 2-D fp16 weight")
     N, K = w.shape
+    w = _own_rows(w)
     ldw = _rowmajor(w, "w")
     q = torch.empty((N, K), dtype=torch.int8, device=w.device)
     s = torch.empty(N, dtype=torch.float16, device=w.device)
@@ -473,7 +494,7 @@ def rms_norm_linear(x: torch.Tensor, w_folded: torch.Tensor, eps: float = 1e-5, 
     if bias is not None and epilogue is not None:
         raise HxmiError("rms_norm_linear takes a bias only without an epilogue")
     lead = x.shape[:-1]
-    x2 = x.reshape(-1, x.shape[-1])
+    x2, w_folded = _own_rows(x.reshape(-1, x.shape[-1])), _own_rows(w_folded)
     M, K = x2.shape
     N = w_folded.shape[0]
     if w_folded.dim() != 2 or w_folded.shape[1] != K:
@@ -503,6 +524,7 @@ def gemv(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
     _require_gpu(x, w, bias, out)
     if x.dtype not in (torch.float16, torch.bfloat16) or w.dtype != x.dtype:
         raise HxmiError("gemv takes fp16 or bf16 x and w of one dtype")
+    x, w = _own_rows(x), _own_rows(w)
     ldx, ldw = _rowmajor(x, "x"), _rowmajor(w, "w")
     M, K = x.shape
     N = w.shape[0]
@@ -529,6 +551,7 @@ def w8a16_linear(x: torch.Tensor, wq: torch.Tensor, scale: torch.Tensor, bias: O
     _require_gpu(x, wq, scale, bias, out)
     if x.dtype != torch.float16 or wq.dtype != torch.int8:
         raise HxmiError("w8a16_linear takes fp16 x and int8 wq")
+    x, wq = _own_rows(x), _own_rows(wq)
     ldx, ldw = _rowmajor(x, "x"), _rowmajor(wq, "wq")
     M, K = x.shape
     N = wq.shape[0]
@@ -556,7 +579,7 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5,
     if x.dtype not in (torch.float16, torch.bfloat16) or weight.dtype != x.dtype:
         raise HxmiError("rms_norm takes fp16 or bf16 x and weight of the same dtype")
     lead = x.shape[:-1]
-    x2 = x.reshape(-1, x.shape[-1])
+    x2 = _own_rows(x.reshape(-1, x.shape[-1]))
     ldx = _rowmajor(x2, "x")
     rows, cols = x2.shape
     weight = _vec(weight, cols, x.dtype, "weight")
@@ -578,7 +601,7 @@ def softmax(x: torch.Tensor, scale: float = 1.0, out: Optional[torch.Tensor] = N
     if x.dtype not in (torch.float16, torch.bfloat16):
         raise HxmiError("softmax takes fp16 or bf16 input")
     lead = x.shape[:-1]
-    x2 = x.reshape(-1, x.shape[-1])
+    x2 = _own_rows(x.reshape(-1, x.shape[-1]))
     ldx = _rowmajor(x2, "x")
     rows, cols = x2.shape
     if out is None:
@@ -665,7 +688,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional
     if (q.dtype == torch.float16 and D in (64, 128) and v.shape[-1] == D and k.dtype == v.dtype == q.dtype
             and scale > 0) or _fused_attention_ok(q, k, v, scale, out):
         _require_gpu(q3, k3, v3)
-        q3, k3, v3 = (t if t.stride(-1) == 1 and t.stride(1) % 8 == 0 and t.stride(0) % 8 == 0
+        q3, k3, v3 = (t if _own_rows(t) is t and t.stride(-1) == 1 and t.stride(1) % 8 == 0 and t.stride(0) % 8 == 0
                       and t.data_ptr() % 16 == 0 else t.contiguous() for t in (q3, k3, v3))
         if (min(S, 32) - 1) * q3.stride(1) + D > 1 << 30:  # (a wave's 32 rows in one 2 GiB buffer)
             q3 = q3.contiguous()

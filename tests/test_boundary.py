@@ -268,3 +268,26 @@ def test_decode_step_rejects_before_launch(pkg):
     assert call_ov(layers=0) == 1 and "positive" in lib.hxmi_last_error().decode()
     assert call_ov(b_ov=P + 1) == 1 and "b_ov" in lib.hxmi_last_error().decode()
     assert call_ov(w_ov=P + 2) == 1 and "16-byte" in lib.hxmi_last_error().decode()
+
+
+def test_row_strides_below_a_row(pkg):
+    """Rows that share elements (expanded, or windows of one vector) are
+    copied for a kernel that reads them and refused where one would write
+    them; every other view keeps its storage and its row stride."""
+    hx, base = pkg.hxmi, torch.arange(60, dtype=torch.float16)
+    for t in (base[:6].expand(4, 6), base.as_strided((4, 6), (2, 1)), base[:1].view(1, 1).expand(4, 1),
+              base.as_strided((2, 4, 6), (30, 5, 1)), base[:6].expand(2, 4, 6)):
+        own = hx._own_rows(t)
+        assert own.is_contiguous() and torch.equal(own, t)
+        assert hx._lead(own, "x") == t.size(-1)
+        with pytest.raises(pkg.HxmiError, match="share elements"):
+            (hx._rowmajor if t.dim() == 2 else hx._batched)(t, "out")
+    x = base.view(6, 10)
+    for t, ld in ((x, 10), (x[:, 3:7], 10), (x[:1].expand(1, 10), 10), (x[:1, :4], 10), (x[2:2], 10),
+                  (base.as_strided((1, 6), (0, 1)), 6), (base.as_strided((1, 6), (2, 1)), 6), (x[:, :1], 10),
+                  (base[:0].view(4, 0), 1)):
+        assert hx._own_rows(t) is t and hx._rowmajor(t, "x") == ld
+    assert hx._own_rows(x.t()).data_ptr() == x.data_ptr()  # (not copied: refused, as it was)
+    with pytest.raises(pkg.HxmiError, match="unit stride"):
+        hx._rowmajor(x.t(), "x")
+    assert hx._batched(base.view(2, 3, 10)[:1].expand(5, 3, 10), "x") == (10, 0)  # one slice for a whole batch

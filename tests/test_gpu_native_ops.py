@@ -134,3 +134,66 @@ def test_native_form_leaves_errors_to_python(pkg, dev):
                 lambda: pkg.rms_norm(x, w[:, :8]), lambda: pkg.attention(x, x, x)):
         with pytest.raises((pkg.HxmiError, IndexError)):
             bad()
+
+
+def shared_rows(pkg, dev):
+    """(name, call, operands whose rows share elements): each operand in turn,
+    expanded from one row or a window that moves less than a row."""
+    x, w, b = n(dev, 40, 64), n(dev, 96, 64, seed=2), n(dev, 96, seed=3)
+    one, window = x[:1].expand(40, 64), n(dev, 1000, seed=21).as_strided((40, 64), (8, 1))
+    w1, ww = w[:1].expand(96, 64), n(dev, 1000, seed=22).as_strided((96, 64), (8, 1))
+    x3, w3 = window.view(40, 64).as_strided((4, 10, 64), (80, 8, 1)), ww.as_strided((4, 24, 64), (200, 8, 1))
+    wq = torch.randint(-127, 128, (96, 64), dtype=torch.int8, generator=torch.Generator().manual_seed(8)).to(dev)
+    q1 = wq[:1].expand(96, 64)
+    sc = (torch.rand(96, generator=torch.Generator().manual_seed(9)) * 9e-3 + 1e-3).half().to(dev)
+    q, k = n(dev, 4, 50, 64, seed=4), n(dev, 4, 1, 64, seed=5).expand(4, 50, 64)
+    for xx in (one, window):
+        yield "gemm a", lambda a: pkg.gemm(a, w, b_layout="nt"), xx
+        yield "linear x", lambda a: pkg.linear(a, w, b), xx
+        yield "rms_norm_linear x", lambda a: pkg.rms_norm_linear(a, w, 1e-5), xx
+        yield "gemv x", lambda a: pkg.gemv(a, w), xx[:3]
+        yield "w8a16 x", lambda a: pkg.w8a16_linear(a, wq, sc), xx[:3]
+        yield "w8a16 x, many rows", lambda a: pkg.w8a16_linear(a, wq, sc), xx
+        yield "rms_norm x", lambda a: pkg.rms_norm(a, w[0], 1e-5), xx
+        yield "softmax x", lambda a: pkg.softmax(a, 0.3), xx
+    for yy in (w1, ww):
+        yield "gemm b", lambda a: pkg.gemm(x, a, b_layout="nt"), yy
+        yield "linear w", lambda a: pkg.linear(x, a, b), yy
+        yield "rms_norm_linear w", lambda a: pkg.rms_norm_linear(x, a, 1e-5), yy
+        yield "gemv w", lambda a: pkg.gemv(x[:3], a), yy
+        yield "fold_rms_weight w", lambda a: pkg.fold_rms_weight(a, x[0]), yy
+        yield "quantize_int8 w", lambda a: pkg.hxmi.quantize_int8(a)[0], yy
+        yield "gemm nn b", lambda a: pkg.gemm(n(dev, 40, 96), a), yy
+    yield "w8a16 wq", lambda a: pkg.w8a16_linear(x[:3], a, sc), q1
+    yield "bgemm a", lambda a: pkg.bgemm(a, w.view(4, 24, 64), b_layout="nt"), x3
+    yield "bgemm b", lambda a: pkg.bgemm(x.view(4, 10, 64), a, b_layout="nt"), w3
+    for dt in (torch.float16, torch.bfloat16):
+        yield "attention k", lambda a: pkg.attention(q.to(a.dtype), a, q.to(a.dtype)), k.to(dt)[:, :1].expand(4, 50, 64)
+        yield "attention q", lambda a: pkg.attention(a, q.to(a.dtype), q.to(a.dtype)), k.to(dt)[:, :1].expand(4, 50, 64)
+
+
+def test_rows_that_share_elements(pkg, dev):
+    """The results are those of a copy with rows of its own, on the native
+    entry's way and on the Python form's."""
+    for name, call, t in shared_rows(pkg, dev):
+        print(name, tuple(t.shape), t.stride(), flush=True)
+        assert t.stride(-2) < t.size(-1)
+        want = call(t.clone(memory_format=torch.contiguous_format))
+        assert torch.equal(call(t), want), name
+        with PythonForm():
+            assert torch.equal(call(t), want), name
+
+
+def test_out_rows_that_share_elements_are_refused(pkg, dev):
+    x, w, b = n(dev, 8, 64), n(dev, 96, 64, seed=2), n(dev, 1, 96)
+    wq = torch.ones(96, 64, dtype=torch.int8, device=dev)
+    out = b.expand(8, 96)
+    for bad in (lambda: pkg.gemm(x, w, b_layout="nt", out=out), lambda: pkg.linear(x, w, out=out),
+                lambda: pkg.gemv(x, w, out=out), lambda: pkg.w8a16_linear(x, wq, b[0], out=out),
+                lambda: pkg.rms_norm_linear(x, w, 1e-5, out=out), lambda: pkg.softmax(x, out=x[:1].expand(8, 64)),
+                lambda: pkg.rms_norm(x, w[0], out=x[:1].expand(8, 64)),
+                lambda: pkg.bgemm(x.view(1, 8, 64), w.view(1, 96, 64), b_layout="nt", out=out.unsqueeze(0)),
+                lambda: pkg.attention(x.view(1, 8, 64), x.view(1, 8, 64), x.view(1, 8, 64),
+                                      out=x[:1].expand(1, 8, 64))):
+        with pytest.raises(pkg.HxmiError):
+            bad()
