@@ -90,6 +90,23 @@ bool vec(const Tensor* t, int64_t n, at::ScalarType type) {
 
 void* ptr(const Tensor* t) { return t ? t->data_ptr() : nullptr; }
 
+// The value of a Python float or int; false, with no Python error left, for
+// anything else (which the Python form converts or names).
+bool number(PyObject* o, long& v) {
+  if (!PyLong_Check(o)) return false;
+  v = PyLong_AsLong(o);
+  if (v != -1 || !PyErr_Occurred()) return true;
+  PyErr_Clear();  // (out of range)
+  return false;
+}
+bool number(PyObject* o, double& v) {
+  long i;
+  if (PyFloat_Check(o)) v = PyFloat_AS_DOUBLE(o);
+  else if (number(o, i)) v = (double)i;
+  else return false;
+  return true;
+}
+
 template <typename F>
 int unlocked(F&& f) {
   int rc;
@@ -150,9 +167,9 @@ PyObject* op_gemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const Tensor *a = in.get(args[0]), *b = in.get(args[1]), *bias = in.get(args[4], true), *o = in.get(args[6], true);
   NOT_PLAIN_UNLESS(in.ok && half_type(*a) && b->scalar_type() == a->scalar_type());
   const int nt = PyObject_IsTrue(args[2]);
-  const int epi = (int)PyLong_AsLong(args[3]);
-  const double alpha = PyFloat_AsDouble(args[5]);
-  if (PyErr_Occurred()) return nullptr;
+  long epi;
+  double alpha;
+  NOT_PLAIN_UNLESS(number(args[3], epi) && number(args[5], alpha));
   int64_t lda, ldb, ldc;
   NOT_PLAIN_UNLESS(rows(*a, lda) && rows(*b, ldb));
   const int64_t M = a->size(0), K = a->size(1), N = b->size(nt ? 0 : 1);
@@ -168,7 +185,7 @@ PyObject* op_gemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (!ws.ok) return nullptr;
   void* s = in.stream();
   return result(unlocked([&] {
-                  return fn(ptr(a), ptr(b), ptr(&out), ptr(bias), M, N, K, lda, ldb, ldc, nt, epi, (float)alpha,
+                  return fn(ptr(a), ptr(b), ptr(&out), ptr(bias), M, N, K, lda, ldb, ldc, nt, (int)epi, (float)alpha,
                             ws.data, ws.bytes, s);
                 }),
                 out);
@@ -183,9 +200,9 @@ PyObject* op_bgemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const Tensor *a = in.get(args[0]), *b = in.get(args[1]), *bias = in.get(args[4], true), *o = in.get(args[6], true);
   NOT_PLAIN_UNLESS(in.ok && half_type(*a) && b->scalar_type() == a->scalar_type() && a->dim() == 3 && b->dim() == 3);
   const int nt = PyObject_IsTrue(args[2]);
-  const int epi = (int)PyLong_AsLong(args[3]);
-  const double alpha = PyFloat_AsDouble(args[5]);
-  if (PyErr_Occurred()) return nullptr;
+  long epi;
+  double alpha;
+  NOT_PLAIN_UNLESS(number(args[3], epi) && number(args[5], alpha));
   int64_t lda, ldb, ldc;
   const int64_t batch = a->size(0), M = a->size(1), K = a->size(2), N = b->size(nt ? 1 : 2);
   const int64_t nout = epi == kEpiSiluMul ? N / 2 : N;
@@ -200,7 +217,7 @@ PyObject* op_bgemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
   void* s = in.stream();
   return result(unlocked([&] {
                   return fn(ptr(a), ptr(b), ptr(&out), ptr(bias), batch, M, N, K, lda, ldb, ldc, a->stride(0),
-                            b->stride(0), out.stride(0), nt, epi, (float)alpha, s);
+                            b->stride(0), out.stride(0), nt, (int)epi, (float)alpha, s);
                 }),
                 out);
   END_HANDLE_TH_ERRORS
@@ -233,8 +250,8 @@ PyObject* op_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   Operands in;
   const Tensor *x = in.get(args[0]), *w = in.get(args[1]), *bias = in.get(args[2], true), *o = in.get(args[4], true);
   NOT_PLAIN_UNLESS(in.ok && half_type(*x) && w->scalar_type() == x->scalar_type());
-  const int epi = (int)PyLong_AsLong(args[3]);
-  if (PyErr_Occurred()) return nullptr;
+  long epi;
+  NOT_PLAIN_UNLESS(number(args[3], epi));
   int64_t M, K, ldx, ldw, ldy;
   NOT_PLAIN_UNLESS(as_rows(*x, M, K, ldx) && rows(*w, ldw) && w->size(1) == K);
   const int64_t N = w->size(0), nout = epi == kEpiSiluMul ? N / 2 : N;
@@ -264,9 +281,9 @@ PyObject* op_rms_norm_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const Tensor *x = in.get(args[0]), *w = in.get(args[1]), *rs_out = in.get(args[4], true),
                *rs_in = in.get(args[5], true), *bias = in.get(args[6], true);
   NOT_PLAIN_UNLESS(in.ok && half_type(*x) && w->scalar_type() == x->scalar_type());
-  const double eps = PyFloat_AsDouble(args[2]);
-  int epi = (int)PyLong_AsLong(args[3]);
-  if (PyErr_Occurred()) return nullptr;
+  double eps;
+  long epi;
+  NOT_PLAIN_UNLESS(number(args[2], eps) && number(args[3], epi));
   int64_t M, K, ldx, ldw;
   NOT_PLAIN_UNLESS(as_rows(*x, M, K, ldx) && rows(*w, ldw) && w->size(1) == K);
   const int64_t N = w->size(0), nout = epi == kEpiSiluMul ? N / 2 : N;
@@ -343,8 +360,8 @@ PyObject* op_rms_norm(PyObject*, PyObject* const* args, Py_ssize_t n) {
   Operands in;
   const Tensor *x = in.get(args[0]), *w = in.get(args[1]), *o = in.get(args[3], true);
   NOT_PLAIN_UNLESS(in.ok && half_type(*x) && x->is_contiguous() && x->dim() >= 1 && x->numel() > 0);
-  const double eps = PyFloat_AsDouble(args[2]);
-  if (PyErr_Occurred()) return nullptr;
+  double eps;
+  NOT_PLAIN_UNLESS(number(args[2], eps));
   const int64_t cols = x->size(-1), nrows = x->numel() / cols;
   NOT_PLAIN_UNLESS(w && vec(w, cols, x->scalar_type()));
   NOT_PLAIN_UNLESS(!o || (o->sizes() == x->sizes() && o->scalar_type() == x->scalar_type() && o->is_contiguous()));
@@ -363,8 +380,8 @@ PyObject* op_softmax(PyObject*, PyObject* const* args, Py_ssize_t n) {
   Operands in;
   const Tensor *x = in.get(args[0]), *o = in.get(args[2], true);
   NOT_PLAIN_UNLESS(in.ok && half_type(*x) && x->is_contiguous() && x->dim() >= 1 && x->numel() > 0);
-  const double scale = PyFloat_AsDouble(args[1]);
-  if (PyErr_Occurred()) return nullptr;
+  double scale;
+  NOT_PLAIN_UNLESS(number(args[1], scale));
   const int64_t cols = x->size(-1), nrows = x->numel() / cols;
   NOT_PLAIN_UNLESS(!o || (o->sizes() == x->sizes() && o->scalar_type() == x->scalar_type() && o->is_contiguous()));
   const Tensor out = o ? *o : like(*x, x->sizes());
@@ -438,9 +455,9 @@ PyObject* op_attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const int64_t S = q->size(-2), Skv = k->size(-2), D = q->size(-1), H = q->size(-3), Hkv = k->size(-3);
   NOT_PLAIN_UNLESS(k->size(-1) == D && D % 8 == 0 && D <= 128 && H % Hkv == 0 &&
                    q->sizes().slice(0, r - 3) == k->sizes().slice(0, r - 3));
-  const double scale = args[3] == Py_None ? 1.0 / std::sqrt((double)D) : PyFloat_AsDouble(args[3]);
-  const long causal = PyLong_AsLong(args[4]);
-  if (PyErr_Occurred()) return nullptr;
+  double scale = 1.0 / std::sqrt((double)D);
+  long causal;
+  NOT_PLAIN_UNLESS((args[3] == Py_None || number(args[3], scale)) && number(args[4], causal));
   NOT_PLAIN_UNLESS(scale > 0 && std::isfinite((float)scale) && causal >= 0 && causal <= 2);
   int64_t ldq, ldk, ldv, sq, sk, sv;
   NOT_PLAIN_UNLESS(slices(*q, ldq, sq) && slices(*k, ldk, sk) && slices(*v, ldv, sv));

@@ -3,6 +3,7 @@ Python form: the same calls, once as they are and once under an empty torch
 function mode, which sends every op down its Python form.  Results have to be
 the same bits, whether a call's operands are plain (the native entry takes
 it) or not (views, ranks, strides and workspaces it leaves alone)."""
+import numpy as np
 import pytest
 import torch
 from torch.overrides import TorchFunctionMode
@@ -196,4 +197,32 @@ def test_out_rows_that_share_elements_are_refused(pkg, dev):
                 lambda: pkg.attention(x.view(1, 8, 64), x.view(1, 8, 64), x.view(1, 8, 64),
                                       out=x[:1].expand(1, 8, 64))):
         with pytest.raises(pkg.HxmiError):
+            bad()
+
+
+class Half:
+    def __float__(self):
+        return 0.5
+
+
+def test_numbers_that_only_the_python_form_takes(pkg, dev):
+    """causal and scale in other forms than int and float: what the Python
+    form converts gives its results, what it refuses is refused by its name."""
+    q = n(dev, 2, 50, 64)
+    for dt in (torch.float16, torch.bfloat16):
+        t = q.to(dt)
+        want = pkg.attention(t, t, t, causal=1)
+        for causal in (1.0, True, np.bool_(True), np.int64(1), np.float32(1)):
+            assert torch.equal(pkg.attention(t, t, t, causal=causal), want)
+        assert torch.equal(pkg.attention(t, t, t, np.float32(0.5)), pkg.attention(t, t, t, 0.5))
+        for causal in (None, 1.5, "1", 3, -1, 1 << 70):
+            with pytest.raises(pkg.HxmiError):
+                pkg.attention(t, t, t, causal=causal)
+    x, w = n(dev, 8, 64), n(dev, 96, 64, seed=2)
+    assert torch.equal(pkg.gemm(x, w, b_layout="nt", alpha=Half()), pkg.gemm(x, w, b_layout="nt", alpha=0.5))
+    assert torch.equal(pkg.gemm(x, w, b_layout="nt", alpha=2), pkg.gemm(x, w, b_layout="nt", alpha=2.0))
+    assert torch.equal(pkg.softmax(x, Half()), pkg.softmax(x, 0.5))
+    for bad in (lambda: pkg.gemm(x, w, b_layout="nt", alpha="one"), lambda: pkg.softmax(x, None),
+                lambda: pkg.rms_norm(x, w[0], None), lambda: pkg.rms_norm_linear(x, w, "eps")):
+        with pytest.raises((TypeError, ValueError)):
             bad()
