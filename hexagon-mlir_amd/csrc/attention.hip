@@ -1,4 +1,6 @@
 // Fused attention dispatch: the workgroup shape and the launch arguments.
+#include <algorithm>
+
 #include "attention_impl.h"
 
 namespace hxmi {
@@ -11,8 +13,6 @@ namespace {
 
 // Launch shape: query waves x key-split waves per workgroup.
 int pick_cfg(const AttnProblem& p) {
-  const int64_t forced = knob(KNOB_ATTN_CFG);
-  if (forced != KNOB_UNSET) return (int)forced;
   // Queries per workgroup: the most that still spread over the chip, since
   // each workgroup reads its K and V through LDS once; 128 queries are split
   // over two halves of the keys to have eight waves (four with few keys, and
@@ -72,8 +72,14 @@ hipError_t launch_attention(const AttnProblem& p, hipStream_t stream) {
   a.bm = p.sm;
   a.c = p.scale * attn::kLog2e;
   if (p.d % 8 || p.d < 8 || p.d > 128) return hipErrorNotSupported;
-  const int cfg = pick_cfg(p);
-  return p.dtype == DT_BF16 ? attn::launch_bf16(a, p, cfg, stream) : attn::launch_f16(a, p, cfg, stream);
+  const auto launch = [&](int cfg) {
+    return p.dtype == DT_BF16 ? attn::launch_bf16(a, p, cfg, stream) : attn::launch_f16(a, p, cfg, stream);
+  };
+  // an override that has no instantiation for this type and head dim gives
+  // way to the picked shape (nothing has been launched then)
+  const int64_t forced = knob(KNOB_ATTN_CFG);
+  const hipError_t e = forced == KNOB_UNSET ? hipErrorNotSupported : launch((int)std::clamp<int64_t>(forced, 0, 999));
+  return e == hipErrorNotSupported ? launch(pick_cfg(p)) : e;
 }
 
 }  // namespace hxmi

@@ -235,6 +235,18 @@ def test_attention_launch_shapes_d128(pkg, dev, knobs, cfg):
     _check_nan(out, ref.sdpa(np32(q), np32(k), np32(v), 0.09, causal=2))
 
 
+@pytest.mark.parametrize("dtype,d,cfg", [(torch.bfloat16, 64, 24), (torch.bfloat16, 128, 21), (torch.float16, 80, 12),
+                                         (torch.float16, 128, 42), (torch.float16, 128, 24), (torch.float16, 64, 99),
+                                         (torch.bfloat16, 40, 0), (torch.float16, 64, 1 << 32 | 41)])
+def test_attention_override_without_an_instantiation(pkg, dev, knobs, dtype, d, cfg):
+    """The knob changes how a result is computed, never whether: a shape that
+    does not exist for the type and head dim is not taken."""
+    q, k, v = (uniform((3, n, d), 131 + i, dtype=dtype).to(dev) for i, n in enumerate((77, 300, 300)))
+    want = pkg.attention(q, k, v, causal=2)
+    knobs(attn_cfg=cfg)
+    assert torch.equal(pkg.attention(q, k, v, causal=2), want)
+
+
 def test_attention_ex_rejects_bad_arguments(pkg, dev):
     lib = pkg.hxmi.load_library()
     x = torch.zeros(4, 64, dtype=torch.float16, device="cuda")
