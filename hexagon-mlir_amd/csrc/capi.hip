@@ -113,6 +113,7 @@ int gemm_common(int dtype, const void* A, const void* B, void* C, const void* bi
   p.rs_out = rs_out;
   p.rs_in = rs_in;
   if (noalloc) {
+    p.lib_scratch = 1;
     // the split-K partials go to this device's scratch array
     const int64_t need = hxmi::gemm_workspace_bytes(p);
     REQUIRE(need <= (int64_t)HXMI_NOALLOC_SCRATCH_BYTES,

@@ -296,6 +296,13 @@ Plan gemm_plan(const GemmProblem& p, int splits) {
 }
 
 bool may_split(const GemmProblem& p) {
+  // The library's own scratch serves one call of a GPU at a time.  Callers on
+  // several streams only order the products that have always used it: those
+  // of a long K into few tiles, and forced splits.
+  if (p.lib_scratch && (knob(KNOB_SPLITK) != KNOB_UNSET
+                            ? p.K < 2048
+                            : p.K < 4096 || ((p.M + 63) / 64) * ((p.N + 127) / 128) >= 384))
+    return false;
   return p.batch == 1 && !p.out_f32 && !p.rms && p.K >= 512 && p.K % 8 == 0 && gemm_fast_path_ok(p);
 }
 

@@ -73,6 +73,7 @@ struct GemmProblem {
   int tile;      // forced tile id (< 0: heuristic)
   void* ws;      // split-K workspace (fp32 partial sums) or null
   int64_t ws_bytes;
+  int lib_scratch;    // 1: ws is the library's own, which all calls on a GPU share
   const void* scale;  // int8 B only: per-column fp16 scale
   int rms;            // 1: C = epilogue(rmsnorm(A) . B^T), B holds the folded norm weight
   float rms_eps;

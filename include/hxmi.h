@@ -125,13 +125,15 @@ int64_t hxmi_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int b_is_nt, 
  * arguments, results and epilogues as hxmi_gemm_f16; where that call would
  * split K, the fp32 partial tiles go to a library-owned array of
  * HXMI_NOALLOC_SCRATCH_BYTES in each GPU's memory (held until the process
- * ends) instead of a caller workspace.  A shape whose partials need more is
- * rejected with HXMI_ERR_INVALID_ARGUMENT before anything is launched.  The
- * array's arrival counters start zero and every call leaves them zero.  All
- * calls on one GPU share its array: two calls whose executions overlap on
- * one GPU (different streams, or concurrent graph replays) race and give
- * wrong results; calls ordered on one stream are safe.  `stream` must
- * belong to the current device.
+ * ends) instead of a caller workspace, for K of at least 4096 and fewer than
+ * 384 tiles of 64 x 128 (with a splitk override: K of at least 2048); other
+ * shapes run whole.  A shape whose partials need more is rejected with
+ * HXMI_ERR_INVALID_ARGUMENT before anything is launched.  The array's arrival
+ * counters start zero and every call leaves them zero.  All calls on one GPU
+ * that split K share its array: two of them whose executions overlap on one
+ * GPU (different streams, or concurrent graph replays) race and give wrong
+ * results; calls ordered on one stream, and calls that run whole, are safe.
+ * `stream` must belong to the current device.
  * No counterpart in the reference (its kernels allocate VTCM from a runtime
  * pool, VTCMPool.cpp:62-106); it exists for the callers named above.
  */

@@ -58,3 +58,24 @@ def test_noalloc_gemm_epilogue_on_current_stream(pkg, dev):
     s.synchronize()
     exp = ref.silu_mul_linear(x.cpu().numpy(), wg.cpu().numpy(), wu.cpu().numpy())
     assert ref.max_rel_err(np32(y.cpu()), exp) <= TOL
+
+
+@pytest.mark.parametrize("M,N,K", [(64, 768, 3072), (20, 80, 3800), (256, 896, 1024), (3072, 2048, 5632)])
+def test_noalloc_gemm_runs_whole_beside_the_long_products(pkg, dev, M, N, K):
+    """Shapes other than long K into few tiles keep off the shared array,
+    whatever the call with a workspace does: the same bits as a call without
+    one, and no refusal where a forced split would need more than the array."""
+    lib = pkg.load_library()
+    x, w = _operands(M, N, K, 95, dev)
+    y = torch.full((2, M, N), 7.0, dtype=torch.float16, device=dev)
+    args = (None, M, N, K, K, K, N, 1, 0, 1.0)
+    assert lib.hxmi_gemm_f16(x.data_ptr(), w.data_ptr(), y[0].data_ptr(), *args, None, 0, None) == 0
+    assert lib.hxmi_gemm_f16_noalloc(x.data_ptr(), w.data_ptr(), y[1].data_ptr(), *args, None) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(y[0], y[1])
+    if K < 2048:
+        with pkg.tuning(splitk=4, gemm_tile=6):  # 64x64 tiles
+            assert lib.hxmi_gemm_f16_noalloc(x.data_ptr(), w.data_ptr(), y[1].data_ptr(), *args, None) == 0
+            assert lib.hxmi_gemm_f16(x.data_ptr(), w.data_ptr(), y[0].data_ptr(), *args, None, 0, None) == 0
+        torch.cuda.synchronize()
+        assert torch.equal(y[0], y[1])
