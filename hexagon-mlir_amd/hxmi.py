@@ -642,9 +642,11 @@ def _fused_attention_ok(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale
                         out: Optional[torch.Tensor]) -> bool:
     """Whether attention() runs the fused kernel where its own test (fp16 at
     head dims 64 and 128) fails: where the three steps take nothing more, at
-    least one key, K / V slices of at most 2 GiB, a finite scale, operands on
-    the 16-byte grid and an out whose rows take the kernel's 8-byte stores."""
+    least one key, K / V slices of at most 2 GiB, a scale positive and finite
+    in 32 bits, operands on the 16-byte grid and an out whose rows take the
+    kernel's 8-byte stores."""
     D = q.shape[-1]
+    scale = ctypes.c_float(scale).value
     if q.dtype not in (torch.float16, torch.bfloat16) or k.dtype != q.dtype or v.dtype != q.dtype \
             or v.shape[-1] != D or D % 8 or not 8 <= D <= 128 or not scale > 0:
         return False

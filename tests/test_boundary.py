@@ -270,6 +270,16 @@ def test_decode_step_rejects_before_launch(pkg):
     assert call_ov(w_ov=P + 2) == 1 and "16-byte" in lib.hxmi_last_error().decode()
 
 
+def test_scales_the_fused_attention_takes(pkg):
+    """Zero or infinite once in 32 bits: left to the three steps, which take
+    any scale."""
+    q = torch.zeros(2, 8, 80, dtype=torch.float16)
+    ok = lambda s: pkg.hxmi._fused_attention_ok(q, q, q, s, None)  # noqa: E731
+    assert ok(0.125) and ok(1) and ok(torch.tensor(0.5)) and ok(2.0 ** -149) and ok(3e38)
+    for s in (0.0, -1.0, 2.0 ** -151, 1e-60, 3.5e38, 1e300, float("inf"), float("nan")):
+        assert not ok(s), s
+
+
 def test_row_strides_below_a_row(pkg):
     """Rows that share elements (expanded, or windows of one vector) are
     copied for a kernel that reads them and refused where one would write

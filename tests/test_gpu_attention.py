@@ -415,6 +415,15 @@ def test_attention_mask_tails(pkg, dev, knobs, cfg, s, skv, d, off):
     assert ref.max_err_vs_scale(np32(out), exp) <= TOL
 
 
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 64), (torch.float16, 80)])
+def test_attention_scale_below_32_bits(pkg, dev, dtype, d):
+    """A scale that is zero in 32 bits weighs every key the same."""
+    q, k, v = (uniform((2, n, d), 251 + i, dtype=dtype).to(dev) for i, n in enumerate((40, 64, 64)))
+    out = pkg.attention(q, k, v, 1e-50)
+    exp = np.broadcast_to(np32(v.cpu()).mean(1, keepdims=True), (2, 40, d))
+    _check_nan_tol(out.cpu(), exp, RMS[dtype])
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_attention_three_step_value_width(pkg, dev, dtype):
     """A value width other than the head dim stays on the three steps: mask,
