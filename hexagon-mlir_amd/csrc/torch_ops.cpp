@@ -441,6 +441,16 @@ bool mask_slices(const Tensor& m, const Tensor& q, int64_t Skv, int64_t& ld, int
   return ld >= Skv;
 }
 
+// Whether the address ranges of two tensors' elements meet (neither is empty).
+bool overlap(const Tensor& a, const Tensor& b) {
+  const auto end = [](const Tensor& t) {
+    int64_t last = 0;
+    for (int64_t i = 0; i < t.dim(); ++i) last += (t.size(i) - 1) * t.stride(i);
+    return (uintptr_t)t.data_ptr() + (last + 1) * t.element_size();
+  };
+  return (uintptr_t)a.data_ptr() < end(b) && (uintptr_t)b.data_ptr() < end(a);
+}
+
 // attention(q, k, v, scale or None, causal, mask or None, out or None)
 PyObject* op_attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -465,7 +475,9 @@ PyObject* op_attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
   NOT_PLAIN_UNLESS(!m || mask_slices(*m, *q, Skv, ldm, sm, mg));
   int64_t ldo = D, so = S * D;
   NOT_PLAIN_UNLESS(!o || (o->sizes() == q->sizes() && o->scalar_type() == q->scalar_type() && slices(*o, ldo, so) &&
-                          (o->is_contiguous() || (!bf16(*q) && (D == 64 || D == 128)))));
+                          ((!bf16(*q) && (D == 64 || D == 128)) ||
+                           (o->is_contiguous() && !overlap(*o, *k) && !overlap(*o, *v) && !(m && overlap(*o, *m)) &&
+                            (!overlap(*o, *q) || (q->data_ptr() == o->data_ptr() && q->is_contiguous()))))));
   const Tensor out = o ? *o : like(*q, q->sizes());
   void* s = in.stream();
   return result(unlocked([&] {

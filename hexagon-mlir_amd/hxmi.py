@@ -638,13 +638,22 @@ def _mask_slices(mask: torch.Tensor, lead: tuple, S: int, Skv: int) -> tuple[tor
     return m, Skv, S * Skv, 1
 
 
+def _overlap(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether the address ranges of two tensors' elements meet."""
+    ends = [(t.data_ptr(), t.data_ptr() + (sum((n - 1) * st for n, st in zip(t.shape, t.stride())) + 1) * t.element_size())
+            for t in (a, b)]
+    return a.numel() > 0 and b.numel() > 0 and ends[0][0] < ends[1][1] and ends[1][0] < ends[0][1]
+
+
 def _fused_attention_ok(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float,
-                        out: Optional[torch.Tensor]) -> bool:
+                        out: Optional[torch.Tensor], mask: Optional[torch.Tensor] = None) -> bool:
     """Whether attention() runs the fused kernel where its own test (fp16 at
     head dims 64 and 128) fails: where the three steps take nothing more, at
     least one key, K / V slices of at most 2 GiB, a scale positive and finite
     in 32 bits, operands on the 16-byte grid and an out whose rows take the
-    kernel's 8-byte stores."""
+    kernel's 8-byte stores, apart from the operands: the three steps have read
+    q, k and the mask before they write out, the kernel's workgroups have not
+    (each has read its own rows of q, so out may be q itself)."""
     D = q.shape[-1]
     scale = ctypes.c_float(scale).value
     if q.dtype not in (torch.float16, torch.bfloat16) or k.dtype != q.dtype or v.dtype != q.dtype \
@@ -657,7 +666,12 @@ def _fused_attention_ok(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale
         return False
     if any(t.data_ptr() % 16 or (t.is_contiguous() and any(st % 8 for st in t.stride()[:-1])) for t in (q, k, v)):
         return False  # (other tensors off the 16-byte grid are copied)
-    return out is None or (out.is_contiguous() and out.data_ptr() % 8 == 0)
+    if out is None:
+        return True
+    if any(t is not None and _overlap(t, out) for t in (k, v, mask)) or \
+            (_overlap(q, out) and (q.data_ptr() != out.data_ptr() or q.stride() != out.stride())):
+        return False
+    return out.is_contiguous() and out.data_ptr() % 8 == 0
 
 
 def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional[float] = None,
@@ -688,7 +702,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional
     k3 = k.reshape(-1, Skv, D)
     v3 = v.reshape(-1, Skv, v.shape[-1])
     if (q.dtype == torch.float16 and D in (64, 128) and v.shape[-1] == D and k.dtype == v.dtype == q.dtype
-            and scale > 0) or _fused_attention_ok(q, k, v, scale, out):
+            and scale > 0) or _fused_attention_ok(q, k, v, scale, out, mask):
         _require_gpu(q3, k3, v3)
         q3, k3, v3 = (t if _own_rows(t) is t and t.stride(-1) == 1 and t.stride(1) % 8 == 0 and t.stride(0) % 8 == 0
                       and t.data_ptr() % 16 == 0 else t.contiguous() for t in (q3, k3, v3))

@@ -1,6 +1,7 @@
 """CPU checks of the C ABI boundary: the library loads, exports exactly what
 include/hxmi.h declares, and rejects invalid arguments before any launch."""
 import ctypes
+import math
 import re
 
 import pytest
@@ -278,6 +279,22 @@ def test_scales_the_fused_attention_takes(pkg):
     assert ok(0.125) and ok(1) and ok(torch.tensor(0.5)) and ok(2.0 ** -149) and ok(3e38)
     for s in (0.0, -1.0, 2.0 ** -151, 1e-60, 3.5e38, 1e300, float("inf"), float("nan")):
         assert not ok(s), s
+
+
+def test_out_that_the_fused_attention_would_overwrite(pkg):
+    """An out over K, V, the mask or other rows of Q is left to the three
+    steps, which have read Q, K and the mask by then; Q itself is not."""
+    buf = torch.zeros(6 * 512, dtype=torch.float16)
+    part = lambda at, *sh: buf[at:at + math.prod(sh)].view(*sh)  # noqa: E731
+    q, k, v, o, m = (part(i * 512, 2, 8, 32) for i in range(5))
+    m = m.view(-1)[:64].view(8, 8)
+    ok = lambda out, q=q: pkg.hxmi._fused_attention_ok(q, k, v, 0.2, out, m)  # noqa: E731
+    assert ok(None) and ok(o) and ok(q) and ok(q.view(2, 8, 32))
+    assert not ok(k) and not ok(v) and not ok(m.as_strided((2, 8, 32), (256, 32, 1)))
+    assert not ok(part(256, 2, 8, 32)) and not ok(part(508, 2, 8, 32)) and not ok(part(8, 2, 8, 32))
+    rows = part(3 * 512, 8, 2, 32).transpose(0, 1)  # out over q's elements in another order
+    assert not ok(o, rows) and ok(q, rows)
+    assert ok(part(0, 2, 8, 32)[:0], q[:0])
 
 
 def test_row_strides_below_a_row(pkg):

@@ -424,6 +424,24 @@ def test_attention_scale_below_32_bits(pkg, dev, dtype, d):
     _check_nan_tol(out.cpu(), exp, RMS[dtype])
 
 
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 64), (torch.bfloat16, 128), (torch.float16, 80)])
+@pytest.mark.parametrize("over", ["q", "k", "mask"])
+def test_attention_out_over_an_operand(pkg, dev, dtype, d, over):
+    """out in q's memory, in k's, and in the mask's: each was read before the
+    three steps wrote it, and still is."""
+    bh, s = 12, 384
+    q, k, v = (uniform((bh, s, d), 261 + i, dtype=dtype).to(dev) for i in range(3))
+    m = normal((bh, s, s), 264).to(dev) if over == "mask" else None
+    want = pkg.attention(q, k, v, mask=m)
+    out = {"q": q, "k": k}.get(over)
+    if out is None:
+        out = m.view(dtype).view(-1)[:bh * s * d].view(bh, s, d)
+    got = pkg.attention(q, k, v, mask=m, out=out)
+    assert got is out
+    assert (got.float() - want.float()).square().mean().sqrt() <= RMS[dtype] * want.float().square().mean().sqrt()
+    assert (got.float() - want.float()).abs().max() <= TOL * want.float().abs().max()
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_attention_three_step_value_width(pkg, dev, dtype):
     """A value width other than the head dim stays on the three steps: mask,
