@@ -248,14 +248,15 @@ struct Plan {
   float us;
 };
 
-float plan_us(const GemmProblem& p, const TileCost& c, int splits) {
-  const int64_t tiles = ((p.M + c.bm - 1) / c.bm) * ((p.N + c.bn - 1) / c.bn) * p.batch * splits;
-  const int slots = 256 * c.per_cu;
-  const int64_t full = tiles / slots;
+// (mn: output tiles of one batch entry)
+float plan_us(const GemmProblem& p, const TileCost& c, int64_t mn, int splits) {
+  const int64_t tiles = mn * p.batch * splits;
+  const int slots = 256 * c.per_cu;  // (per_cu: 1 or 2)
+  const int64_t full = c.per_cu == 1 ? tiles / 256 : tiles / 512;
   const int rem = (int)(tiles - full * slots), conc = (rem + 255) / 256;
   const float round = std::max(c.lat, c.per_cu * c.thr);
   const float last = rem ? std::max(c.lat, conc * c.thr * (0.85f + 0.15f * (float)rem / (256.f * conc))) : 0.f;
-  const float steps = (float)((p.K + 64 * splits - 1) / (64 * splits));
+  const float steps = (float)(((uint32_t)((p.K + 63) / 64) + splits - 1) / (uint32_t)splits);
   float t = steps * ((float)full * round + last);
   if (p.dtype == DT_W8A16) t = std::max(t, (float)(p.N * p.K) * (1.f / 4.2e6f));  // (the weights from HBM)
   // an RMSNorm-folded GEMM sums the squares of its A rows in every tile of a
@@ -279,11 +280,12 @@ Plan gemm_plan(const GemmProblem& p, int splits) {
     const int first = splits > 0 ? splits : 1;
     // slices of at least four K-steps that stay within two rounds of the
     // CUs, their partial tiles within 32 MiB
-    const int64_t most = splits > 0 ? splits
-                                    : std::min<int64_t>({8, p.K / 256, 512 / tiles,
-                                                         ((32 << 20) - kWsCounterBytes) / (tiles * c.bm * c.bn * 4)});
+    const int64_t most = splits > 0    ? splits
+                         : tiles > 256 ? 1
+                                       : std::min<int64_t>({8, p.K / 256, 512 / tiles,
+                                                            ((32 << 20) - kWsCounterBytes) / (tiles * c.bm * c.bn * 4)});
     for (int s = first; s == first || s <= most; s += s < 4 ? 1 : 2) {
-      const float us = plan_us(p, c, s);
+      const float us = plan_us(p, c, tiles, s);
       if (us < (s > 1 ? 0.98f : 1.f) * best.us) best = {c.id, s, us};
     }
   }
@@ -317,8 +319,9 @@ int gemm_pick_tile(const GemmProblem& p) {
 
 // The split-K launch of p: K slices of kc (a multiple of the 64-deep K-step)
 // as a batch of GEMMs into the same output (sC = 0), the tile they run and
-// the fix-up workspace they need.  False when p does not split.
-static bool split_plan(const GemmProblem& p, GemmProblem& q, int& tile, int64_t& need) {
+// the fix-up workspace they need.  False when p does not split; where the
+// plan was to run it whole, `whole` receives the tile (gemm_pick_tile's).
+static bool split_plan(const GemmProblem& p, GemmProblem& q, int& tile, int64_t& need, int& whole) {
   if (!may_split(p)) return false;
   const int64_t want = knob(KNOB_SPLITK);
   const Plan plan =
@@ -326,7 +329,10 @@ static bool split_plan(const GemmProblem& p, GemmProblem& q, int& tile, int64_t&
   const int splits = plan.splits;
   tile = gemm::forced_tile(p);
   if (tile < 0) tile = plan.tile;
-  if (splits <= 1) return false;
+  if (splits <= 1) {
+    whole = tile;
+    return false;
+  }
   q = p;
   const int64_t kc = ((p.K + splits - 1) / splits + 63) / 64 * 64;
   q.K = kc;
@@ -342,9 +348,9 @@ static bool split_plan(const GemmProblem& p, GemmProblem& q, int& tile, int64_t&
 
 int64_t gemm_workspace_bytes(const GemmProblem& p) {
   GemmProblem q;
-  int tile;
+  int tile, whole;
   int64_t need;
-  return split_plan(p, q, tile, need) ? need : 0;
+  return split_plan(p, q, tile, need, whole) ? need : 0;
 }
 
 hipError_t launch_gemm(const GemmProblem& p, hipStream_t stream) {
@@ -398,19 +404,19 @@ hipError_t launch_gemm(const GemmProblem& p, hipStream_t stream) {
   }
 
   GemmProblem q;
-  int qtile;
+  int tile, whole = -1;
   int64_t need;
-  if (split_plan(p, q, qtile, need) && p.ws && p.ws_bytes >= need && ((uintptr_t)p.ws % 256) == 0) {
+  if (p.ws && split_plan(p, q, tile, need, whole) && p.ws_bytes >= need && ((uintptr_t)p.ws % 256) == 0) {
     // K slices as a batch into one output; the last slice to finish a tile
     // adds the fp32 partials (in the workspace) and runs the epilogue
-    gemm::KArgs k = gemm::make_kargs(q, qtile);
+    gemm::KArgs k = gemm::make_kargs(q, tile);
     k.k_last = (int)(p.K - (q.batch - 1) * q.K);
     k.fix = (char*)p.ws;
-    return gemm::launch_fast(q, qtile, k, stream);
+    return gemm::launch_fast(q, tile, k, stream);
   }
 
-  const int tile = gemm_pick_tile(p);
-  return gemm::launch_fast(p, tile, gemm::make_kargs(p, tile), stream);
+  if (whole < 0) whole = gemm_pick_tile(p);
+  return gemm::launch_fast(p, whole, gemm::make_kargs(p, whole), stream);
 }
 
 GemmProblem w8a16_as_gemm(const GemvProblem& p) {
