@@ -522,13 +522,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, (OCC2 ? (BM / WM) * (BN
     lofB8[s] = (uint32_t)((wn * WN + l) * BK + (((MI == 32 ? 2 * (s >> 1) + h : h) ^ ((l >> 2) & 3)) << 4));
   }
   short8v fbo[BI8 ? TN : 1];  // BI8: the odd substep's B fragments, dequantised with the even one's
-  // RAGGED (K % 8 != 0): the 16-byte chunk that straddles K brings in
-  // elements past K (row padding, or the next row).  In the last K-step the
-  // fragments keep only their elements below K; the NN B operand needs no
-  // mask, its rows past K read as zero.
   // Piece P of a substep's fragments: B fragment P, then A fragment P - TN.
-  auto read_piece = [&](short8v (&fa)[TM], short8v (&fb)[TN], const char* sA_, const char* sB_, int s, int kstep,
-                        auto P) {
+  auto read_piece = [&](short8v (&fa)[TM], short8v (&fb)[TN], const char* sA_, const char* sB_, int s, auto P) {
     constexpr int p = decltype(P)::value;
     if constexpr (p < TN) {
       constexpr int i = p;
@@ -552,16 +547,25 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, (OCC2 ? (BM / WM) * (BN
     } else {
       fa[p - TN] = *(const short8v*)(sA_ + lofA[s] + (p - TN) * MI * RB);
     }
+  };
+  // RAGGED (K % 8 != 0): the 16-byte chunk that straddles K brings in
+  // elements past K (row padding, or the next row).  In the last K-step the
+  // fragments keep only their elements below K; the NN B operand needs no
+  // mask, its rows past K read as zero.  One test behind all the reads: a
+  // branch after each of them waits for it (20 x 81 x 3801 30.8 us, 18.4 so).
+  auto read_frags = [&](short8v (&fa)[TM], short8v (&fb)[TN], const char* sA_, const char* sB_, int s, int kstep) {
+    static_for<TN + TM>([&](auto P) { read_piece(fa, fb, sA_, sB_, s, P); });
     if constexpr (RAGGED) {
       if (kstep == nk - 1) {
         const int nv = K - (kstep * BK + s * 16 + (lane >> 5) * 8);
-        if constexpr (p >= TN) fa[p - TN] = keep_first(fa[p - TN], nv);
-        else if constexpr (!NN) fb[p] = keep_first(fb[p], nv);
+#pragma unroll
+        for (int j = 0; j < TM; ++j) fa[j] = keep_first(fa[j], nv);
+        if constexpr (!NN) {
+#pragma unroll
+          for (int i = 0; i < TN; ++i) fb[i] = keep_first(fb[i], nv);
+        }
       }
     }
-  };
-  auto read_frags = [&](short8v (&fa)[TM], short8v (&fb)[TN], const char* sA_, const char* sB_, int s, int kstep) {
-    static_for<TN + TM>([&](auto P) { read_piece(fa, fb, sA_, sB_, s, kstep, P); });
   };
 
   Acc acc[TN][TM];
@@ -766,7 +770,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, (OCC2 ? (BM / WM) * (BN
         } else {  // reads and loads in turn
           static_for<TN + TM>([&](auto P) {
             constexpr int p = decltype(P)::value, NP = TN + TM;
-            read_piece(fa[nxt], fb[nxt], sa(st1), sb(stb1), t - SUBS, kt + 1, P);
+            read_piece(fa[nxt], fb[nxt], sa(st1), sb(stb1), t - SUBS, P);
             constexpr int lo = p * NVM / NP, hi = (p + 1) * NVM / NP;
             issueA(kt + STAGES, st, std::integral_constant<int, (lo < IA ? lo : IA)>{},
                    std::integral_constant<int, (hi < IA ? hi : IA)>{});
