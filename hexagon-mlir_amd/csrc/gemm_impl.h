@@ -466,22 +466,14 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, (OCC2 ? (BM / WM) * (BN
     const int k0 = kt * BK;
     const bool live = kt < nk;
     char* sB_ = sb(stage);
-    const char* base;
-    uint32_t bytes, vB;
-    if constexpr (NN) {
-      base = Bb + (int64_t)k0 * a.ldb * 2;
-      bytes = (uint32_t)min(BK, K - k0) * bytesB;
-      vB = voffB;
-    } else if constexpr (BI8) {
-      base = Bb + k0;
-      bytes = bytesB - (uint32_t)k0;
-      vB = (k0 + cB8 * 16) < K ? voffB : kOOB;
-    } else {
-      base = Bb + (int64_t)k0 * 2;
-      bytes = bytesB - 2u * k0;
-      vB = (k0 + cA * 8) < K ? voffB : kOOB;
-    }
-    const __amdgpu_buffer_rsrc_t rB = make_rsrc(base, live ? bytes : 0u);
+    // (the resource before the lane offsets: in the other order the scalar
+    // work of both operands' resources lands ahead of the MFMAs of a substep,
+    // RMS 700 x 2048 x 5632 on 128x64 tiles 34.7 -> 37.6 us)
+    const __amdgpu_buffer_rsrc_t rB =
+        NN    ? make_rsrc(Bb + (int64_t)k0 * a.ldb * 2, live ? (uint32_t)min(BK, K - k0) * bytesB : 0u)
+        : BI8 ? make_rsrc(Bb + k0, live ? bytesB - (uint32_t)k0 : 0u)
+              : make_rsrc(Bb + (int64_t)k0 * 2, live ? bytesB - 2u * k0 : 0u);
+    const uint32_t vB = NN || (k0 + (BI8 ? cB8 * 16 : cA * 8)) < K ? voffB : kOOB;
 #pragma unroll
     for (int i = decltype(LO)::value; i < decltype(HI)::value; ++i)
       load_lds16(rB, (HXMI_LDS void*)to_lds(sB_ + (i * NW + w) * 1024), vB + i * stepB);
@@ -587,9 +579,9 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, (OCC2 ? (BM / WM) * (BN
   for (int j = 0; j < TM; ++j) ss[j] = 0.f;
   auto sum_squares = [&](const short8v (&f)[TM]) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
+    for (int j = 0; j < TM; ++j)
 #pragma unroll
-      for (int j = 0; j < TM; ++j) ss[j] = sumsq2<T>(f[j], q, ss[j]);
+      for (int q = 0; q < 4; ++q) ss[j] = sumsq2<T>(f[j], q, ss[j]);
   };
 
   // Software pipeline over K-steps: STAGES LDS stages (step kt lives in stage
