@@ -1117,13 +1117,16 @@ hipError_t launch_one(const KArgs& k, hipStream_t stream) {
   // int8 B: BK 64, two A stages (A is L2-resident) and up to six B stages
   // in the LDS that three stages of both took (same workgroups per CU): the
   // weights stream from HBM, so B is prefetched several K-steps ahead
-  // (an NN tile whose loads of one wave lie 8 rows apart keeps 32x32x16)
-  constexpr int MI = NN && threads / 64 * (512 / s.BN) % 16 ? 32 : s.MI;
+  // (an NN tile whose loads of one wave lie 8 rows apart keeps 32x32x16, and
+  // so does the 8-wave 128x128 NN tile: 256 x 1024 x 1024 10.2 -> 9.8 us,
+  // 700 x 2048 x 5632 57.5 -> 55.8; k-contiguous B 9.3 us against 9.6)
+  constexpr bool W16 = s.MI == 16 && !(NN && (TILE == TILE_128x128_W8 || threads / 64 * (512 / s.BN) % 16));
+  constexpr int MI = W16 ? 16 : 32, FD = TILE == TILE_128x128_W8 && !W16 ? 3 : s.FD;
   constexpr int W8_A = s.BM * 128, W8_B = s.BN * 64;
   constexpr int W8_SB = s.OCC2 ? (81920 - 2 * W8_A) / W8_B : W8_A / W8_B + 3 > 6 ? 6 : W8_A / W8_B + 3;
   hipLaunchKernelGGL((gemm_mfma<s.BM, s.BN, s.WM, s.WN, (BI8 ? 64 : s.BK), (BI8 || UNAL ? 2 : s.STAGES), NN, T, EPI,
                                 OUTF32, BI8, (s.PP && !BI8 && !RMS), RMS, RAGGED, (BI8 ? W8_SB : s.SB),
-                                (BI8 || s.PP || UNAL ? 1 : s.FD), UNAL, MI, s.OCC2>),
+                                (BI8 || s.PP || UNAL ? 1 : FD), UNAL, MI, s.OCC2>),
                      dim3((unsigned)blocks), dim3(threads), 0, stream, k);
   return hipGetLastError();
 }
