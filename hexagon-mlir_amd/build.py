@@ -1,5 +1,6 @@
 """Build libhxmi.so (the C-ABI kernel library) in-tree with hipcc for gfx950,
-and hxmi_torch.so (the native entry of the torch-facing ops) on top of it.
+and hxmi_torch.so (the native entry of the torch-facing ops) on top of it
+where torch and its headers are there.
 
     python hexagon-mlir_amd/build.py [--jobs N]
 
@@ -61,6 +62,7 @@ def _compile(src: pathlib.Path) -> pathlib.Path:
 def _build_ops() -> None:
     """torch_ops.cpp is host code only: g++ against torch's headers, linked to
     the libhxmi.so beside it."""
+    OPS.unlink(missing_ok=True)  # (one of another libhxmi.so)
     import sysconfig
 
     import torch
@@ -79,6 +81,17 @@ def _build_ops() -> None:
     os.replace(tmp, OPS)
 
 
+def build_ops() -> bool:
+    """hxmi_torch.so, or False with the reason on stderr: libhxmi.so and the
+    ops work without it (no torch or no ROCm torch headers here)."""
+    try:
+        _build_ops()
+    except (ImportError, OSError, RuntimeError) as e:
+        print(f"[hxmi] {OPS.name} is not built, the ops take their Python forms: {e}", file=sys.stderr, flush=True)
+        return False
+    return True
+
+
 def build(jobs: int | None = None, verbose: bool = True) -> pathlib.Path:
     BUILD.mkdir(parents=True, exist_ok=True)
     LIB.parent.mkdir(parents=True, exist_ok=True)
@@ -94,9 +107,9 @@ def build(jobs: int | None = None, verbose: bool = True) -> pathlib.Path:
     if proc.returncode != 0:
         raise RuntimeError(f"link failed: {' '.join(cmd)}\n{proc.stdout}\n{proc.stderr}")
     os.replace(tmp, LIB)
-    _build_ops()
+    built_ops = build_ops()
     if verbose:
-        print(f"[hxmi] built {LIB} and {OPS.name}", flush=True)
+        print(f"[hxmi] built {LIB}" + (f" and {OPS.name}" if built_ops else ""), flush=True)
     return LIB
 
 

@@ -14,6 +14,7 @@ import ctypes
 import importlib.machinery
 import importlib.util
 import pathlib
+import warnings
 from typing import Optional
 
 import torch
@@ -100,21 +101,37 @@ def load_library() -> ctypes.CDLL:
     return _lib
 
 
+class _PythonForms:
+    """Stands for an extension module that takes no call."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
 class _NativeOps:
     """Stands for the extension module until its first use loads it.  Each of
     its functions returns the op's result for plain operands and None for
-    anything else, which the Python form below it then takes."""
+    anything else, which the Python form below it then takes.  Without the
+    module the Python forms run every call (a longer host time, the same
+    kernels)."""
 
     def __getattr__(self, name):
         global _ops
+        if not LIB_PATH.exists():
+            return getattr(_PythonForms(), name)  # (the Python form names the operands, then the library)
         load_library()
-        if not OPS_PATH.exists():
-            raise HxmiNotBuiltError(f"{OPS_PATH} is missing; build it with hexagon-mlir_amd/build.py")
-        loader = importlib.machinery.ExtensionFileLoader("hxmi_torch", str(OPS_PATH))
-        mod = importlib.util.module_from_spec(importlib.util.spec_from_file_location("hxmi_torch", OPS_PATH,
-                                                                                     loader=loader))
-        loader.exec_module(mod)
-        mod.set_workspace(_workspace)
+        try:
+            if not OPS_PATH.exists():
+                raise ImportError(f"{OPS_PATH} is missing; build it with hexagon-mlir_amd/build.py")
+            loader = importlib.machinery.ExtensionFileLoader("hxmi_torch", str(OPS_PATH))
+            mod = importlib.util.module_from_spec(importlib.util.spec_from_file_location("hxmi_torch", OPS_PATH,
+                                                                                         loader=loader))
+            loader.exec_module(mod)
+            mod.set_workspace(_workspace)
+        except ImportError as e:
+            warnings.warn(f"the native entry of the ops is not loaded, calls take longer on the host: {e}",
+                          RuntimeWarning, stacklevel=3)
+            mod = _PythonForms()
         _ops = mod
         return getattr(mod, name)
 

@@ -318,3 +318,40 @@ def test_row_strides_below_a_row(pkg):
     with pytest.raises(pkg.HxmiError, match="unit stride"):
         hx._rowmajor(x.t(), "x")
     assert hx._batched(base.view(2, 3, 10)[:1].expand(5, 3, 10), "x") == (10, 0)  # one slice for a whole batch
+
+
+def test_ops_without_their_native_entry(pkg, monkeypatch, tmp_path):
+    """No extension module: the Python forms take the calls, with one warning.
+    No library either: a call names its operands first, as it did."""
+    hx, x = pkg.hxmi, torch.zeros(8, 8, dtype=torch.float16)
+    empty = tmp_path / "hxmi_torch.so"
+    empty.write_bytes(b"")  # (there, but no module)
+    for path in (tmp_path / "missing.so", empty):
+        monkeypatch.setattr(hx, "OPS_PATH", path)
+        monkeypatch.setattr(hx, "_ops", hx._NativeOps())
+        with pytest.warns(RuntimeWarning, match="native entry") as seen:
+            for _ in range(2):
+                with pytest.raises(pkg.HxmiError, match="on cpu"):
+                    pkg.gemm(x, x)
+            with pytest.raises(pkg.HxmiError, match="on cpu"):
+                pkg.softmax(x)
+        assert len(seen) == 1
+    monkeypatch.setattr(hx, "LIB_PATH", tmp_path / "libhxmi.so")
+    monkeypatch.setattr(hx, "_ops", hx._NativeOps())
+    with pytest.raises(pkg.HxmiError, match="on cpu"):
+        pkg.gemm(x, x)
+
+
+def test_library_builds_without_the_native_entry(pkg, monkeypatch, capsys, tmp_path):
+    import importlib.util
+
+    spec = importlib.util.spec_from_file_location("hxmi_build_test", ROOT / "hexagon-mlir_amd" / "build.py")
+    build = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(build)
+    stale = tmp_path / "hxmi_torch.so"
+    stale.write_bytes(b"")
+    monkeypatch.setattr(build, "OPS", stale)
+    monkeypatch.setattr(build, "CSRC", tmp_path)  # (no source for g++)
+    assert build.build_ops() is False
+    assert "hxmi_torch.so is not built" in capsys.readouterr().err
+    assert not stale.exists()  # one built beside another libhxmi.so is not left behind
