@@ -1,9 +1,9 @@
 // GEMM dispatch: alignment checks, tile choice, and the element-wise kernel
 // used for what no MFMA instantiation takes (fewer than 8 columns in an
 // operand row, activations on an NN operand).  Ragged N and K (not multiples
-// of 8) run on the MFMA path: ragged columns are stored element by element,
-// K not a multiple of 8 runs the instantiations that mask the last K-step,
-// and rows off the 16-byte grid (leading dimensions not a multiple of 8,
+// of 8) run on the MFMA path: the last N % 8 columns go out in at most three
+// stores, K not a multiple of 8 runs the instantiations that mask the last
+// K-step, and rows off the 16-byte grid (leading dimensions not a multiple of 8,
 // misaligned pointers) those that load their tiles through registers.
 #include <algorithm>
 #include <iterator>
@@ -209,39 +209,59 @@ hipError_t launch_fast(const GemmProblem& p, int tile, const KArgs& k, hipStream
 // Tile and K slices of a GEMM: the pair with the least estimated time.  Per
 // 64-deep K-step a tile alone on its CU takes `lat` us (few CUs busy: the
 // loads' latency and its own MFMAs) and, with every CU busy, `thr` us of its
-// CU (memory contention and the power limit slow it), `epi` us for
-// its epilogue; per_cu workgroups share a CU.  Splitting K over s workgroups
-// puts short outputs on more CUs and costs 1.0 + 0.6 s us of fix-up round
-// trips plus the partial tiles' traffic.  Constants fitted to every tile and
-// 1-16 slices on 8 shapes at 20-4096 rows (graph replays, weights rotating);
-// us, the tile rule before it (area over a fixed efficiency, K < 4096 never
-// split) against the pair it takes now:
-//   20 x 80 x 3800 13.6 -> 7.9; 64 x 768 x 3072 12.2 -> 8.6; 64 x 2048 x 5632 18.3 -> 13.2;
-//   256 x 896 x 4864 14.7 -> 11.1; 700 x 2560 x 2048 16.9 -> 13.7; 1028 x 2048 x 5632 54.3 -> 37.2;
-//   2000 x 2048 x 5632 74.8 -> 62.9; 512 x 2048 x 5632 (two slices, as before) 27.3 -> 26.3.
-// int8 weights (fitted the same way): 256 x 151936 x 896 98 -> 86; 150 x 151936 x 896 101 -> 74;
-//   64 x 151936 x 896 48.5 -> 39.7; 256 x 11264 x 2048 26.4 -> 20.6; 17 x 2048 x 2048 14.6 -> 9.5.
+// CU (memory contention and the power limit slow it; with few busy, `part` of
+// that), `epi` us for its epilogue; per_cu workgroups share a CU.  Splitting K
+// over s workgroups puts short outputs on more CUs and costs fix-up round
+// trips plus the partial tiles' traffic (SplitCost).
+//
+// Constants fitted to every tile and 1-8 slices on 1780 shapes, 17-4096 rows,
+// 256-12288 columns (int8 up to 151936) and K 512-8192, both layouts, plain,
+// with the norm and SiLU-mul, each with its weights out of cache and in L2
+// (graph replays on MI355X; two thirds of the shapes random).  Over a shape's
+// best pair the one taken costs 1.0 % out of cache and 0.4 % in L2, int8 0.8 %
+// in both; constants fitted to eight shapes took 2.1 and 0.9 %, int8 2.1 and
+// 2.0, on single shapes up to half again.  us, tile by area and K < 4096 never
+// split / those constants / these:
+//   20 x 80 x 3800 13.8 / 8.4 / 8.4; 64 x 768 x 3072 12.3 / 8.7 / 8.6; 64 x 2048 x 5632 14.6 / 11.5 / 11.3;
+//   256 x 896 x 4864 14.4 / 12.0 / 12.0; 700 x 2560 x 2048 16.6 / 14.6 / 14.4;
+//   700 x 4096 x 4096 48.0 / 54.4 / 39.5; 1028 x 2048 x 5632 49.6 / 38.6 / 37.7;
+//   2000 x 2048 x 5632 64.1 / 62.1 / 52.1; 512 x 2048 x 5632 22.8 / 22.9 / 22.4;
+//   150 x 11264 x 2048 31.3 / 30.6 / 22.7.
+// int8 weights: 256 x 151936 x 896 100.8 / 90.0 / 89.3; 150 x 151936 x 896 101.3 / 78.6 / 77.9;
+//   17 x 1152 x 896 7.3 / 8.3 / 7.3; 100 x 896 x 896 7.6 / 8.5 / 7.6; 400 x 4096 x 4096 32.9 / 33.5 / 28.4.
 namespace {
 
 struct TileCost {
   int id, bm, bn, per_cu;
-  float lat, thr, epi;
+  float lat, thr, epi, part;
 };
 constexpr TileCost kCosts[] = {
-    {TILE_256x256_W8, 256, 256, 1, 1.10f, 1.45f, 3.0f}, {TILE_256x128_W8, 256, 128, 1, 0.68f, 0.92f, 1.8f},
-    {TILE_128x192_W8, 128, 192, 1, 0.55f, 0.72f, 1.6f}, {TILE_128x128_W8, 128, 128, 2, 0.57f, 0.47f, 1.2f},
-    {TILE_64x128, 64, 128, 2, 0.35f, 0.37f, 1.0f},      {TILE_128x64, 128, 64, 2, 0.33f, 0.35f, 1.0f},
-    {TILE_64x64, 64, 64, 2, 0.22f, 0.24f, 0.5f},
+    {TILE_256x256_W8, 256, 256, 1, 0.601f, 1.186f, 5.444f, 0.626f},
+    {TILE_256x128_W8, 256, 128, 1, 0.613f, 0.660f, 3.681f, 0.952f},
+    {TILE_128x192_W8, 128, 192, 1, 0.537f, 0.462f, 3.253f, 0.359f},
+    {TILE_128x128_W8, 128, 128, 2, 0.629f, 0.423f, 1.018f, 0.986f},
+    {TILE_64x128, 64, 128, 2, 0.396f, 0.350f, 1.038f, 0.626f},
+    {TILE_128x64, 128, 64, 2, 0.330f, 0.284f, 1.307f, 0.948f},
+    {TILE_64x64, 64, 64, 2, 0.182f, 0.236f, 0.392f, 1.000f},
 };
 // int8 B: a tile's waves convert every weight they multiply, so the two tiles
 // of one wave row convert each once; two workgroups a CU cover each other's
 // first loads and epilogue
 constexpr TileCost kCostsI8[] = {
-    {TILE_256x256_W8, 256, 256, 1, 2.00f, 2.10f, 3.0f}, {TILE_I8_128x256, 128, 256, 2, 1.10f, 1.00f, 2.5f},
-    {TILE_I8_64x256, 64, 256, 2, 0.53f, 0.72f, 1.5f},   {TILE_128x128, 128, 128, 2, 0.64f, 0.80f, 1.2f},
-    {TILE_64x128, 64, 128, 2, 0.50f, 0.42f, 0.8f},      {TILE_128x64, 128, 64, 2, 0.45f, 0.37f, 0.8f},
-    {TILE_64x64, 64, 64, 2, 0.36f, 0.25f, 0.5f},
+    {TILE_256x256_W8, 256, 256, 1, 1.319f, 1.709f, 3.265f, 0.914f},
+    {TILE_I8_128x256, 128, 256, 2, 1.069f, 0.874f, 1.287f, 0.937f},
+    {TILE_I8_64x256, 64, 256, 2, 0.600f, 0.647f, 1.346f, 0.660f},
+    {TILE_128x128, 128, 128, 2, 0.514f, 0.798f, 1.522f, 1.000f},
+    {TILE_64x128, 64, 128, 2, 0.565f, 0.419f, 0.545f, 0.539f},
+    {TILE_128x64, 128, 64, 2, 0.239f, 0.463f, 1.034f, 0.826f},
+    {TILE_64x64, 64, 64, 2, 0.398f, 0.251f, 0.250f, 0.941f},
 };
+// us of a split: once, per slice, and per element of the partial tiles (their
+// write and read)
+struct SplitCost {
+  float once, slice, element;
+};
+constexpr SplitCost kSplit = {0.204f, 0.769f, 1.39e-6f}, kSplitI8 = {0.285f, 0.632f, 1.40e-6f};
 
 struct Plan {
   int tile, splits;
@@ -255,15 +275,21 @@ float plan_us(const GemmProblem& p, const TileCost& c, int64_t mn, int splits) {
   const int64_t full = c.per_cu == 1 ? tiles / 256 : tiles / 512;
   const int rem = (int)(tiles - full * slots), conc = (rem + 255) / 256;
   const float round = std::max(c.lat, c.per_cu * c.thr);
-  const float last = rem ? std::max(c.lat, conc * c.thr * (0.85f + 0.15f * (float)rem / (256.f * conc))) : 0.f;
+  const float last = rem ? std::max(c.lat, conc * c.thr * (c.part + (1.f - c.part) * (float)rem / (256.f * conc))) : 0.f;
   const float steps = (float)(((uint32_t)((p.K + 63) / 64) + splits - 1) / (uint32_t)splits);
   float t = steps * ((float)full * round + last);
-  if (p.dtype == DT_W8A16) t = std::max(t, (float)(p.N * p.K) * (1.f / 4.2e6f));  // (the weights from HBM)
+  if (p.dtype == DT_W8A16) {  // (the weights from HBM, and what of the rest they do not cover)
+    const float hbm = (float)(p.N * p.K) * (1.f / 4.04e6f);
+    t = std::max(t, hbm) + 0.058f * std::min(t, hbm);
+  }
   // an RMSNorm-folded GEMM sums the squares of its A rows in every tile of a
   // row, so narrow tiles repeat that work more often
-  if (p.rms) t *= c.bn == 64 ? 1.3f : 1.1f;
+  if (p.rms) t *= c.bn == 64 ? 1.090f : 0.915f;
   t += 2.6f + c.epi * ((float)full * c.per_cu + conc);
-  if (splits > 1) t += 1.0f + 0.6f * splits + (float)tiles * (float)(c.bm * c.bn) * (8.f / 6e6f);
+  if (splits > 1) {
+    const SplitCost& f = p.dtype == DT_W8A16 ? kSplitI8 : kSplit;
+    t += f.once + f.slice * splits + (float)tiles * (float)(c.bm * c.bn) * f.element;
+  }
   return t;
 }
 
@@ -285,15 +311,18 @@ Plan gemm_plan(const GemmProblem& p, int splits) {
                                        : std::min<int64_t>({8, p.K / 256, 512 / tiles,
                                                             ((32 << 20) - kWsCounterBytes) / (tiles * c.bm * c.bn * 4)});
     for (int s = first; s == first || s <= most; s += s < 4 ? 1 : 2) {
-      const float us = plan_us(p, c, tiles, s);
-      if (us < (s > 1 ? 0.98f : 1.f) * best.us) best = {c.id, s, us};
+      const float us = plan_us(p, c, tiles, s) * (s > 1 ? 1.02f : 1.f);  // (a split has to gain 2 %)
+      if (us < best.us) best = {c.id, s, us};
     }
   }
-  // 64x64 tiles with a CU each and k-contiguous weights: a fourth LDS stage
-  // (64 x 1152 x 896 6.2 -> 5.9 us, 256 x 2560 x 2048 10.5 -> 9.6; with two
-  // tiles a CU 15.2 -> 15.5 us, and the NN 1024^3 GEMM 6.4 -> 6.5)
+  // 64x64 tiles with a CU each: a fourth LDS stage.  With the weights out of
+  // cache, 12-20 K-steps a slice run 4-6 % shorter with it (NN 3-5 %, under
+  // the norm's sums 0-1 %), 32 13-15 % (NN 7 %); with everything in L2 up to
+  // 20 run 2 % longer, which NN products and the norm are spared (NN 1024^3
+  // 6.4 us, 6.5 with it); two tiles a CU 1-4 % longer either way.
   const int64_t t64 = ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch * best.splits;
-  if (best.tile == TILE_64x64 && !i8 && p.b_nt && t64 <= 256 && p.K >= 768) best.tile = TILE_64x64_S4;
+  if (best.tile == TILE_64x64 && !i8 && t64 <= 256 && p.K >= (p.rms ? 1536 : p.b_nt ? 768 : 1280))
+    best.tile = TILE_64x64_S4;
   return best;
 }
 

@@ -320,6 +320,19 @@ def test_row_strides_below_a_row(pkg):
     assert hx._batched(base.view(2, 3, 10)[:1].expand(5, 3, 10), "x") == (10, 0)  # one slice for a whole batch
 
 
+def test_products_that_leave_cus_idle_split(pkg):
+    """Few tiles and enough K-steps for slices: the plan splits K (a workspace
+    is asked for); one round of tiles, or the norm's whole rows, does not."""
+    lib = pkg.load_library()
+    for m, n, k in ((17, 1152, 896), (32, 768, 768), (100, 896, 896), (256, 2048, 5632)):
+        assert lib.hxmi_w8a16_workspace_bytes(m, n, k) > 0, (m, n, k)
+    for m, n, k in ((700, 4096, 4096), (64, 768, 3072), (1576, 2048, 5632)):
+        for nt in (0, 1):
+            assert lib.hxmi_gemm_workspace_bytes(m, n, k, nt, 0) > 0, (m, n, k, nt)
+    assert lib.hxmi_gemm_workspace_bytes(4096, 4096, 4096, 1, 0) == 0
+    assert lib.hxmi_w8a16_workspace_bytes(256, 151936, 896) == 0
+
+
 def test_ops_without_their_native_entry(pkg, monkeypatch, tmp_path):
     """No extension module: the Python forms take the calls, with one warning.
     No library either: a call names its operands first, as it did."""

@@ -125,6 +125,19 @@ def test_gemm_ragged_k_exact_integer(pkg, dev, layout, K):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", [(128, 128, 64), (129, 136, 72), (1, 8, 8), (255, 264, 640)])
+def test_gemm_nn_128x128_w8_exact(pkg, dev, force_tile, dtype, M, N, K):
+    """The 8-wave 128x128 tile takes another MFMA in NN form than in NT: exact
+    products of small integers at the edges of its tiles and K-steps."""
+    g = torch.Generator().manual_seed(42)
+    a, b = (torch.randint(-1, 2, s, generator=g).to(dtype) for s in ((M, K), (K, N)))
+    if dtype == torch.bfloat16:  # (sums that bf16 holds exactly)
+        a[:, 128:] = 0
+    force_tile(13)
+    assert torch.equal(run_gemm(pkg, dev, a, b, "nn"), (a.float() @ b.float()).to(dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("layout", ["nn", "nt"])
 @pytest.mark.parametrize("batch,M,N,K", [(1, 1, 9, 8), (1, 65, 63, 15), (3, 64, 64, 65), (2, 129, 197, 71),
                                          (70, 197, 197, 64), (66, 131, 197, 197)])
