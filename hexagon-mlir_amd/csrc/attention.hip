@@ -24,23 +24,33 @@ int pick_cfg(const AttnProblem& p) {
   //                         20.4 / 16.0 / 17.7; 4 x 2048 (64 / 128 / 256) 20.3 / 15.9 / 13.4
   //   head dim 64, causal:  32 x 2048 (512 / 1024 / 2048) 25.1 / 28.8 / 38.7; 32 x 1024 (256 / 512 /
   //                         1024) 13.8 / 11.3 / 15.4; 32 x 512 (128 / 256 / 512) 9.5 / 7.3 / 6.9
-  // With few keys a key split over four waves costs more than it spreads;
-  // and a causal workgroup count of two per CU lets heavy and light blocks
-  // pair up, so the causal lines lie at about twice the others.
+  // With few keys a key split over four waves costs more than it spreads,
+  // once its workgroups no longer have a CU each (unmasked 48 x 157, 240 of
+  // them 5.5, 64 queries 5.9; 48 x 177, 288: 6.7 and 5.9); and a causal
+  // workgroup count of two per CU lets heavy and light blocks pair up, so the
+  // causal lines lie at about twice the others.  Up to 224 keys a causal block
+  // has one or two stages whatever its weight, and 128 queries pay from 192
+  // workgroups on (96 x 197 6.5, 64 queries 7.0; head dim 128, 96 x 157 7.6
+  // and 8.2, 192 x 100 7.3 and 8.1; but 96 x 256 10.1 and 9.5), masked calls
+  // and the three-quarter rows of head dims 72-96 aside (96 x 197 masked 9.0
+  // and 8.4, head dim 80 8.3 and 7.3).
   const bool few_keys = p.skv <= 384;
-  const int64_t wg128 = p.bh * ((p.s + 127) / 128), wg64 = p.bh * ((p.s + 63) / 64);
+  const int64_t wg128 = p.bh * ((p.s + 127) / 128), wg64 = p.bh * ((p.s + 63) / 64),
+                wg32 = p.bh * ((p.s + 31) / 32);
   // A mask's entries take registers that eight waves do not have: 128
   // queries run four waves, and pay only from 320 on (8 waves / 4 waves / 64
   // queries: 32 x 1024 full 23.7 / 25.5 / 20.8, 64 x 500 15.3 / 15.7 / 14.1,
   // 64 x 1000 39.1 / 38.7 / 40.3, 128 x 2048 causal 135 / 131 / 142).
   const bool masked64 = p.mask && p.d <= 64;
-  if (wg128 >= (p.causal ? 320 : few_keys ? 192 : masked64 ? 320 : 144))
+  const bool short_causal = p.causal && p.skv <= 224 && !p.mask && (p.d <= 64 || p.d > 96);
+  if (wg128 >= (short_causal ? 192 : p.causal ? 320 : few_keys ? 192 : masked64 ? 320 : 144))
     return p.d <= 64 && !few_keys && !p.mask ? 42 : 41;
   // (64-192 keys at head dims over 64: the merge of four key splits takes as
   // long as the keys; 4 x 157 causal 6.4 us against 7.2, 32 x 155 full 7.4
   // against 7.5, 64 x 201 8.3 against 7.6)
   if (p.d > 64 && p.skv <= 192) return 22;
-  return wg64 >= (few_keys ? 144 : p.causal ? 288 : 192) ? 22 : 14;
+  if (few_keys) return wg64 >= 144 && (p.mask || wg32 > 256) ? 22 : 14;
+  return wg64 >= (p.causal ? 288 : 192) ? 22 : 14;
 }
 
 }  // namespace

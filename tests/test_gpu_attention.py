@@ -35,6 +35,7 @@ def _check(out, q, k, v, scale):
         (2, 77, 300, 128),  # cross-attention, ragged lengths
         (2, 129, 33, 64),
         (1, 256, 512, 64),
+        (48, 157, 157, 64),  # 240 workgroups of 32 queries
     ],
 )
 def test_attention_vs_oracle(pkg, dev, bh, s, skv, d):
@@ -164,6 +165,8 @@ def test_attention_bool_mask(pkg, dev):
     [
         (4, 300, 300, 64, 1),
         (2, 512, 512, 128, 1),  # TinyLlama-sized causal prefill head pair
+        (96, 197, 197, 64, 1),  # 192 workgroups of 128 queries, up to 224 keys
+        (96, 157, 157, 128, 1),
         (3, 100, 300, 128, 2),  # bottom-right: queries are the last 100 positions
         (2, 300, 100, 64, 2),  # S > S_kv: the first 200 queries see no key (NaN rows)
         (2, 45, 197, 64, 1),
