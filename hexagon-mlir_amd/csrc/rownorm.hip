@@ -237,7 +237,8 @@ RArgs make_args(const RowProblem& p) {
 // which then only wait on each other.  us, graph replays on MI355X:
 //   512 x 2048     1 / 2 / 4 / 8 waves 3.1 / 2.9 / 2.7 / 2.8;  4096 x 2048  8.5 / 8.2 / 8.5 / 9.7
 //   512 x 4096     4.4 / 4.0 / 3.7 / 3.7;  2048 x 4096  8.9 / 8.4 / 8.2 / 8.4;  4096 x 4096  12.9 / 12.1 / 14.3 / 14.0
-//   512 x 8192     4 / 8 waves 5.3 / 5.0;  2048 x 8192  12.6 / 14.6;  4096 x 8192  26.6 / 25.0
+//   512 x 8192     4 / 8 waves 5.3 / 5.0;  1536 x 8192  8.9 / 9.8;  2048 x 8192  11.2 / 12.1;  4096 x 8192
+//   20.7 / 21.4;  8192 x 8192  39.8 / 39.7;  16384 x 8192  94.1 / 91.1 (at 1024 rows the same)
 // (4096 x 8192 in two passes of 2-byte loads, as all widths over 4096 and
 // odd ones ran before: 94.7; 512 x 8192 49.2; 4096 x 2049 27.2).  Rows off the
 // 16-byte grid, whose waves share lines, run one wave a row where many rows
